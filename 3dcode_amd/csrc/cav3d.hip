@@ -795,9 +795,15 @@ __device__ __forceinline__ void st_dev(double *p, double v)
 // state, properties, diagonal-inverse terms, and the Jacobian operands of its
 // j and k neighbours) is moved ahead of use into an LDS stage, so a step's
 // critical path is the dq hand-over and the arithmetic.
-// Tiles wait only on tiles upstream in j and k, every tile is resident
-// (cooperative launch) and a workgroup takes its tiles in topological order,
-// so the chain always advances.
+// Tiles wait only on tiles upstream in j and k.  A workgroup takes its tiles
+// from a ticket counter over the topological order, so whatever the number
+// of workgroups the device has started, every tile upstream of a started one
+// has been taken by a running workgroup: the chain always advances, and the
+// launch need not be cooperative.  (Cooperative launches left the stream idle
+// for 10 us before the forward sweep and 22 us between the two, beside their
+// host time: an iteration of 16x8x8 cells took 0.51 ms with them and 0.30 ms
+// with tickets, 64x32x32 0.95 and 0.74, 128x64x64 2.73 and 2.57, state
+// transfers included.)
 constexpr int TJ = 4, TK = 4;
 // LDS stage of one pencil-step (doubles)
 enum {
@@ -935,7 +941,7 @@ static_assert(TJ == 4 && TK == 4, "the poll wavefront maps an edge of four penci
 // stage without branching on the row, so the dependent chain of a step is
 // three row products, the exchange of y and D^-1.
 template <bool FWD>
-__global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *tiles, int ntiles, int *err)
+__global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *tiles, int ntiles, int *err, int *ticket)
 {
     // dq hand-over, one LDS object (so that the compiler can tell its reads
     // from the stage LDS-DMA): [0, HX) the dq of the hyperplane by the parity
@@ -954,7 +960,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
     __shared__ double ylds[FWD ? YR : 1][TJ * TK][NPV];
     __shared__ double win[2][TJ * TK][ST_N][WIN];   // stage windows (see the pencil wavefronts)
     __shared__ const double *src[TJ * TK][ST_N];
-    __shared__ int gave_up;
+    __shared__ int gave_up, taken;
     const int npv = S.npv;
     const int sg = FWD ? 1 : -1;
     const double sgn = FWD ? 1.0 : -1.0;
@@ -964,7 +970,12 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
     constexpr int PER = ST_N / 16;                                  // stage items per lane
     if (threadIdx.x == 0) gave_up = 0;
     if (threadIdx.x < NPV) zrow[threadIdx.x] = 0.0;
-    for (int tq = blockIdx.x; tq < ntiles; tq += gridDim.x) {
+    for (;;) {
+        // the barrier that ends a tile keeps this write behind every read of the last ticket
+        if (threadIdx.x == 0) taken = atomicAdd(ticket, 1);
+        __syncthreads();
+        const int tq = __builtin_amdgcn_readfirstlane(taken);
+        if (tq >= ntiles) break;
         const int *td = tiles + 4 * (FWD ? tq : ntiles - 1 - tq);
         const BlkD B = S.b[td[0]];           // a copy: the loops read the block's extents from registers
         const long NW = S.NW;
@@ -1279,10 +1290,12 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
     }
 }
 
-__global__ __launch_bounds__(256) void k_fill_bits(double *p, long n, unsigned long long bits)
+// both exchange arrays to "not yet written", both tile tickets to zero
+__global__ __launch_bounds__(256) void k_sweep_reset(double *a, double *b, long n, int *ticket)
 {
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) p[t] = __longlong_as_double((long long)bits);
+    if (t < 2) ticket[t] = 0;
+    if (t < n) a[t] = b[t] = __longlong_as_double((long long)DQ_UNSET);
 }
 
 // ------------------------------------------------------------ update + norms
@@ -1509,10 +1522,11 @@ struct cav3d_ctx {
     double *stage = nullptr;
     size_t stage_n = 0;
     int nwg_update = 0;
-    int coop_blocks = 0;      // grid of the cooperative sweep kernels
+    int sweep_blocks = 0;     // grid of the sweep kernels: as many workgroups as fit the device at once
     int *tiles = nullptr;     // tile table of the sweeps (device): block, j0, k0, diagonal
     int ntiles = 0;
     int *sweep_err = nullptr; // set when a sweep wait gave up
+    int *ticket = nullptr;    // next tile of the forward and the backward sweep
     bool profile = false;
     hipEvent_t ev[14] = {};
     double prof_ms[10] = {};  // [8] last cav3d_rhs_vjp, [9] last cav3d_calrhs (device ms)
@@ -1781,8 +1795,7 @@ int launch_sweep_fills(cav3d_ctx *c, hipStream_t st)
 {
     DS &S = c->S;
     const long nq = (long)NPV * S.NW;
-    hipLaunchKernelGGL(k_fill_bits, dim3(nblk(nq, 256)), dim3(256), 0, st, S.xqf, nq, DQ_UNSET);
-    hipLaunchKernelGGL(k_fill_bits, dim3(nblk(nq, 256)), dim3(256), 0, st, S.xqb, nq, DQ_UNSET);
+    hipLaunchKernelGGL(k_sweep_reset, dim3(nblk(nq, 256)), dim3(256), 0, st, S.xqf, S.xqb, nq, c->ticket);
     return 0;
 }
 
@@ -1790,17 +1803,11 @@ int launch_sweeps(cav3d_ctx *c)
 {
     DS &S = c->S;
     hipLaunchKernelGGL(k_lhs_prep, dim3(nblk(S.NC, 128)), dim3(128), 0, c->st, S);
-    const int *tiles = c->tiles;
-    int ntiles = c->ntiles;
-    int *err = c->sweep_err;
-    void *args[4] = {&S, &tiles, &ntiles, &err};
-    dim3 grid(c->coop_blocks), block(SWEEP_THREADS);
+    const dim3 grid(c->sweep_blocks), block(SWEEP_THREADS);
     if (c->profile) hipEventRecord(c->ev[6], c->st);
-    hipError_t e = hipLaunchCooperativeKernel((const void *)k_sweep_tile<true>, grid, block, args, 0, c->st);
-    if (e != hipSuccess) return fail(std::string("forward sweep launch: ") + hipGetErrorString(e), -3);
+    hipLaunchKernelGGL(k_sweep_tile<true>, grid, block, 0, c->st, S, (const int *)c->tiles, c->ntiles, c->sweep_err, c->ticket);
     if (c->profile) hipEventRecord(c->ev[7], c->st);
-    e = hipLaunchCooperativeKernel((const void *)k_sweep_tile<false>, grid, block, args, 0, c->st);
-    if (e != hipSuccess) return fail(std::string("backward sweep launch: ") + hipGetErrorString(e), -3);
+    hipLaunchKernelGGL(k_sweep_tile<false>, grid, block, 0, c->st, S, (const int *)c->tiles, c->ntiles, c->sweep_err, c->ticket + 1);
     if (c->profile) hipEventRecord(c->ev[8], c->st);
     return 0;
 }
@@ -2009,7 +2016,7 @@ int cav3d_create(const cav3d_params *prm, int nblocks, const cav3d_block *blocks
         std::vector<int> tab;
         for (auto &t : tl) tab.insert(tab.end(), t.begin(), t.end());
         c->ntiles = (int)tl.size();
-        if ((rc = dalloc(c, &c->tiles, tab.size())) || (rc = dalloc(c, &c->sweep_err, 1))) {
+        if ((rc = dalloc(c, &c->tiles, tab.size())) || (rc = dalloc(c, &c->sweep_err, 1)) || (rc = dalloc(c, &c->ticket, 2))) {
             cav3d_destroy(c); return rc;
         }
         if (hipMemcpyAsync(c->tiles, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice, c->st) != hipSuccess) {
@@ -2023,7 +2030,7 @@ int cav3d_create(const cav3d_params *prm, int nblocks, const cav3d_block *blocks
         per = std::min(per, per2);
         long cap = (long)ncu * per;
         if (cap < 1) { cav3d_destroy(c); return fail("sweep kernel cannot be made resident", -3); }
-        c->coop_blocks = (int)std::max(1L, std::min((long)c->ntiles, cap));
+        c->sweep_blocks = (int)std::max(1L, std::min((long)c->ntiles, cap));
     }
     c->nwg_update = (int)nblk(S.NC, 256);
     if ((rc = dalloc(c, &S.red, (long)c->nwg_update * (NPV + 2)))) { cav3d_destroy(c); return rc; }
