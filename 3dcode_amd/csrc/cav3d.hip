@@ -855,40 +855,156 @@ __device__ __forceinline__ const double *stage_base(const DS &S, const BlkD &B, 
     return S.jf + (3 * (2 * ax + side) + r - NB_JF) * S.NC + cm;
 }
 
-// row `lane` Jacobian operands of a staged block (pv at b + NB_PV, ...)
-template <class A>
-__device__ __forceinline__ JacNb stage_jnb(const A &st, int b, int lane, int npv)
-{
-    JacNb q;
-    q.pvn = lane < npv ? st[b + NB_PV + lane] : 0.0;
-    q.pv1 = st[b + NB_PV + 1]; q.pv2 = st[b + NB_PV + 2]; q.pv3 = st[b + NB_PV + 3];
-    const int d = b + NB_DC;
-    q.rho = st[d + D_RHO]; q.rp = st[d + D_RP]; q.rt = st[d + D_RT]; q.ry1 = st[d + D_RY1]; q.ry2 = st[d + D_RY2];
-    q.hp = st[d + D_HP]; q.ht = st[d + D_HT]; q.hy1 = st[d + D_HY1]; q.hy2 = st[d + D_HY2];
-    q.n3[0] = st[b + NB_N3]; q.n3[1] = st[b + NB_N3 + 1]; q.n3[2] = st[b + NB_N3 + 2];
-    q.n3n = (lane >= 1 && lane <= 3) ? st[b + NB_N3 + lane - 1] : 0.0;
-    q.jc = JacCell{st[b + NB_JC], st[b + NB_JC + 1]};
-    q.jf = JacFace{st[b + NB_JF], st[b + NB_JF + 1], st[b + NB_JF + 2]};
-    return q;
-}
 static_assert(ST_PV + 9 == ST_DC && ST_DC + ND == ST_N3 && ST_N3 + 3 == ST_JC && ST_JC + 2 == ST_JF,
               "the own-cell part of the stage has the neighbour-block layout");
 
-// lane q of the lane's 16-lane row, by a DPP row broadcast (no LDS traffic)
+// lane q of the lane's 16-lane row, by one 64-bit DPP move (no LDS traffic)
 template <int Q>
 __device__ __forceinline__ double row_lane(double v)
 {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x150 + Q, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x150 + Q, 0xF, 0xF, false);
-    return __hiloint2double(hi, lo);
+    return __longlong_as_double(__builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0x150 + Q, 0xF, 0xF, false));
 }
-// yv[q] = v of lane q of the row, q < 9 (every lane of the wavefront active)
-__device__ __forceinline__ void bcast_rows(double v, double *yv)
+// Row form of a pencil's step.  A pencil's 16 lanes hold the rows of its
+// cell's system; everything else a step reads (the state, properties, face
+// and diagonal-inverse terms: some 90 numbers a cell) is the same for all
+// lanes.  The lanes read them from the stage one item each (lane l its own
+// item, RowMap) and pass them around with DPP row broadcasts.  Reading every
+// item into every lane took 140 LDS reads a step, whose return path (each
+// read brings 64 lanes x 8 bytes at 128 bytes a clock for the four pencil
+// wavefronts of the CU) bound the step: without any coefficient reads
+// the 64x32x32 sweep fell from 268 to 171 us.  Now 24 reads, and
+// the terms that are one expression per column are formed once, a column per
+// lane, not in every lane.
+struct RowMap {
+    int v1, v2, p, g[7], co[3];     // stage items of this lane (v1, v2, p: within a neighbour block)
+    double scale;                   // of v1: the sweep's sign and the factor 0.5 on u, lam, vis, rho
+    double one[7];                  // 1 in the lane of the column
+    bool mom, en, kw, cpl, n0, n4, n5, n7, n8;
+};
+template <bool FWD> __device__ __forceinline__ RowMap row_map(int lane, int npv)
 {
-    static_assert(NPV == 9, "one broadcast per row of the system");
-    yv[0] = row_lane<0>(v); yv[1] = row_lane<1>(v); yv[2] = row_lane<2>(v);
-    yv[3] = row_lane<3>(v); yv[4] = row_lane<4>(v); yv[5] = row_lane<5>(v);
-    yv[6] = row_lane<6>(v); yv[7] = row_lane<7>(v); yv[8] = row_lane<8>(v);
+    RowMap m;
+    // lanes 0..6: the column's factor of r1 (rho_p, n3, rho_T, rho_y1, rho_y2); then u, lam, vis, rho (scaled), beta, rho
+    m.v1 = lane == 0 ? NB_DC + D_RP : lane <= 3 ? NB_N3 + lane - 1 : lane == 4 ? NB_DC + D_RT : lane == 5 ? NB_DC + D_RY1
+         : lane == 6 ? NB_DC + D_RY2 : lane <= 9 ? NB_JF + lane - 7 : lane == 11 ? NB_JC : NB_DC + D_RHO;
+    // lanes 0..6: the column's factor in the energy row (h_p, u, v, w, h_T, h_y1, h_y2)
+    m.v2 = lane == 0 ? NB_DC + D_HP : lane <= 3 ? NB_PV + lane : lane == 4 ? NB_DC + D_HT : lane == 5 ? NB_DC + D_HY1 : NB_DC + D_HY2;
+    // the row's own factor: pv(n), in the energy row the total enthalpy
+    m.p = lane == 4 ? NB_JC + 1 : lane < NPV ? NB_PV + lane : NB_PV;
+    // the row's entries of D^-1 (getx_apply): k1..k4, e1, e2, f1
+    m.n0 = lane == 0; m.n4 = lane == 4; m.n5 = lane == 5; m.n7 = lane == 7; m.n8 = lane == 8;
+    m.cpl = m.n0 || m.n4 || m.n5;
+    const bool row7 = lane >= 7;
+    m.g[0] = ST_GX + (m.n0 ? GX_C4C1 : m.n4 ? GX_C4IB1S1 : m.n7 ? GX_RBT4 : m.n8 ? GX_RBT1 : GX_C4SSIB1);
+    m.g[1] = ST_GX + (m.n0 ? GX_C2 : m.n4 ? GX_C1 : m.n7 ? GX_T2 : m.n8 ? GX_T3 : GX_SS);
+    m.g[2] = ST_GX + (m.n0 ? GX_C3 : m.n4 ? GX_C3IB1 : GX_C1);
+    m.g[3] = ST_GX + (m.n0 ? GX_RB1 : GX_C2IB1);
+    m.g[4] = ST_GX + (m.n0 ? GX_CROSS1 : GX_S1P5);
+    m.g[5] = ST_GX + (m.n0 ? GX_CP5 : GX_SSY1);
+    m.g[6] = ST_GX + (m.cpl ? GX_MM : row7 ? GX_IT : GX_IB1);
+    // lanes 0, 1, 2: the three sums res0 a + b uuu + c res6 that rows 0, 4, 5 share
+    m.co[0] = ST_GX + (lane == 0 ? GX_AAA1 : lane == 1 ? GX_AAA2 : GX_SSHM);
+    m.co[1] = lane == 0 ? ST_DC + D_RY1 : lane == 1 ? ST_DC + D_RT : ST_GX + GX_RRR;
+    m.co[2] = ST_GX + (lane == 0 ? GX_CROSS : lane == 1 ? GX_CROSS2 : GX_SSY2);
+    const double hs = FWD ? 0.5 : -0.5;
+    m.scale = lane == 7 || lane == 10 ? hs : (lane == 8 || lane == 9) ? 0.5 : 1.0;
+    for (int l = 0; l < 7; l++) m.one[l] = lane == l ? 1.0 : 0.0;
+    m.mom = lane >= 1 && lane <= 3;
+    m.en = lane == 4;
+    m.kw = row7 && lane < npv;
+    return m;
+}
+
+// Row coefficients of one neighbour's split Jacobian, c[l] = +-0.5 a(n,l)
+// (jac_row's products and sums in its order; jac_row_coef has the same row by
+// row): r1[l] and the energy row's factor of column l sit in lane l.  The
+// factor 0.5 and the sign are put on u, lam, vis, rho and n3, which they pass
+// through exactly; rho u goes onto the diagonal as fma(rho u, 1 or 0, a),
+// which rounds as the sum.
+template <bool FWD>
+__device__ __forceinline__ void row_coef(const RowMap &m, double v1, double v2, double p, double *c)
+{
+    constexpr double hs = FWD ? 0.5 : -0.5;
+    const double n3n = hs * v1;
+    v1 = m.scale * v1;
+    const double u = row_lane<7>(v1), lam = row_lane<8>(v1), vis = row_lane<9>(v1);
+    // (the broadcasts stay out of the selects: they need every lane active)
+    const double rhos = row_lane<10>(v1), beta = row_lane<11>(v1);
+    const double lb = m.n0 ? beta : v1;
+    const double t = u * v1 + lam * lb + vis * v1, r = m.mom ? v1 * rhos : t;
+    const double ru = row_lane<13>(v1) * (u + lam + vis);
+    const double P = m.n0 ? 1.0 : p, Q = m.en ? ru : 0.0;
+    c[0] = P * row_lane<0>(r) + Q * row_lane<0>(v2);
+    c[1] = P * row_lane<1>(r) + Q * row_lane<1>(v2);
+    c[2] = P * row_lane<2>(r) + Q * row_lane<2>(v2);
+    c[3] = P * row_lane<3>(r) + Q * row_lane<3>(v2);
+    c[4] = P * row_lane<4>(r) + Q * row_lane<4>(v2);
+    c[5] = P * row_lane<5>(r) + Q * row_lane<5>(v2);
+    c[6] = P * row_lane<6>(r) + Q * row_lane<6>(v2);
+    c[0] = c[0] + (m.en ? -lam : (m.mom ? n3n : 0.0));
+    c[0] = c[0] + (m.en ? -vis : 0.0);
+#pragma unroll
+    for (int l = 1; l < 7; l++) if (l != 4) c[l] = fma(ru, m.one[l], c[l]);
+    c[7] = m.kw ? ru : 0.0;
+}
+
+// y += c x, the neighbour's row n in lane n (jac_row_apply)
+__device__ __forceinline__ void row_apply(const double *c, double x, double &y)
+{
+    y = y + c[0] * row_lane<0>(x);
+    y = y + c[1] * row_lane<1>(x);
+    y = y + c[2] * row_lane<2>(x);
+    y = y + c[3] * row_lane<3>(x);
+    y = y + c[4] * row_lane<4>(x);
+    y = y + c[5] * row_lane<5>(x);
+    y = y + c[6] * row_lane<6>(x);
+    y = y + c[7] * x;
+}
+
+// What a step reads of its own cell, read during the step before: the rows'
+// residual, the Jacobian items of its block (v1, v2, p as row_coef), the
+// rows' D^-1 entries
+struct RowCell {
+    double res, v1, v2, p, g[7], a, co[3];
+};
+template <class W> __device__ __forceinline__ RowCell row_cell(const RowMap &m, const W &st, int ln)
+{
+    RowCell c;
+    c.res = st[ST_RES + ln];
+    c.v1 = st[ST_PV + m.v1]; c.v2 = st[ST_PV + m.v2]; c.p = st[ST_PV + m.p];
+#pragma unroll
+    for (int q = 0; q < 7; q++) c.g[q] = st[m.g[q]];
+    c.a = st[ST_GX + GX_A];
+#pragma unroll
+    for (int q = 0; q < 3; q++) c.co[q] = st[m.co[q]];
+    return c;
+}
+
+// Row n of D^-1 y in lane n (y: the row's right-hand side).  Rows 0, 4 and 5
+// are sums of four products, rows 7 and 8 of two, the rest one difference:
+// every row forms ((k1 x1 + k2 x2) + k3 x3) + k4 ((x4 + e1 z1) + e2 z2) with
+// its own entries and operands and takes the partial sum it needs.
+// Subtractions are sums with the entry's sign flipped, so the operations and
+// their order are getx_apply's.
+__device__ __forceinline__ double row_dinv(const RowMap &m, const RowCell &c, double y)
+{
+    auto neg = [](double x, bool f) { return __longlong_as_double(__double_as_longlong(x) ^ (long long)((unsigned long long)f << 63)); };
+    const double y0 = row_lane<0>(y), y5 = row_lane<5>(y), y6 = row_lane<6>(y);
+    const double s1 = y - y0 * c.p;
+    const double r6 = row_lane<6>(s1), rk = row_lane<7>(s1), ro = row_lane<8>(s1);
+    const double uuu = row_lane<1>(y) * row_lane<1>(c.v2) + row_lane<2>(y) * row_lane<2>(c.v2)
+                     + row_lane<3>(y) * row_lane<3>(c.v2) - row_lane<4>(y);
+    const double co = y0 * c.co[0] + c.co[1] * uuu + c.co[2] * y6;
+    const double co1 = row_lane<0>(co), co2 = row_lane<1>(co), co3 = row_lane<2>(co);
+    const bool row7 = m.n7 || m.n8;
+    const double x1 = row7 ? s1 : r6;
+    const double x2 = m.n5 ? s1 : m.n7 ? ro : m.n8 ? rk : co1;
+    const double x3 = m.n4 ? co3 : co2, x4 = m.n0 ? co2 : co3;
+    const double z1 = m.n0 ? y5 : y0, z2 = m.n0 ? y0 : y5;
+    const double s2 = neg(c.g[0], !m.n4) * x1 + neg(c.g[1], m.n0) * x2;
+    const double w = x4 + neg(c.g[4], !m.n0) * z1 + neg(c.g[5], m.n0) * z2;
+    const double s4 = s2 + neg(c.g[2], !m.n0) * x3 + (m.n4 ? -1.0 : c.g[3]) * (m.n5 ? x4 : w);
+    return (m.cpl ? s4 : row7 ? s2 : s1) * c.g[6] * c.a;
 }
 
 // Workgroup barrier for LDS hand-over: this wavefront's LDS accesses are
@@ -963,7 +1079,6 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
     __shared__ int gave_up, taken;
     const int npv = S.npv;
     const int sg = FWD ? 1 : -1;
-    const double sgn = FWD ? 1.0 : -1.0;
     double *const xq = FWD ? S.xqf : S.xqb;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 15, grp = (threadIdx.x >> 4) & 15;
@@ -1184,6 +1299,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
         const int gj = grp % TJ, gk = grp / TJ;
         const bool mine = lane < npv;
         const int ln = lane < NPV ? lane : 0;
+        const RowMap rows = row_map<FWD>(lane, npv);
         const int j = j0 + gj, k = k0 + gk;
         const bool live = (j <= jend && k <= kend);
         const bool edge = down_edge(grp);
@@ -1227,12 +1343,14 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
         const int d0 = FWD ? sa - j - k - 2 : BI - (sa - j - k);
         if (lane < NPV) lds((sa - sg) & 1, grp)[lane] = 0.0;       // the first step's upstream reads zeros
         double ci[8], cj[8], ck[8];                                  // coefficients of the coming step
+        RowCell own;                                                 // its cell
 #pragma unroll
         for (int q = 0; q < 8; q++) ci[q] = 0.0;
         {
             const WinRow s0{&win[(d0 >> 2) & 1][grp][0][slot(d0)]};
-            jac_row_coef(npv, stage_jnb(s0, ST_J, lane, npv), sg, lane, sgn, cj);
-            jac_row_coef(npv, stage_jnb(s0, ST_K, lane, npv), sg, lane, sgn, ck);
+            row_coef<FWD>(rows, s0[ST_J + rows.v1], s0[ST_J + rows.v2], s0[ST_J + rows.p], cj);
+            row_coef<FWD>(rows, s0[ST_K + rows.v1], s0[ST_K + rows.v2], s0[ST_K + rows.p], ck);
+            own = row_cell(rows, s0, ln);
         }
         __syncthreads();
         for (int s = sa;; s += sg) {
@@ -1241,29 +1359,21 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             const bool act = live && i >= 2 && i <= BI;
             // dq of the three upstream neighbours: in the tile from the
             // previous hyperplane, from another tile through the poll wavefront
-            const WinRow st{&win[(d >> 2) & 1][grp][0][slot(d)]};
             const int pb = (s - sg) & 1;
             // (indices into the hand-over object, not pointers chosen among
             // several, so the compiler sees these reads cannot touch the stage)
             const int oi = lds_at(pb, grp);
             const int oj = lj ? lds_at(pb, grp - sg) : (nj ? xch_at(s & 1, 0, grp) : HZ);
             const int ok = lk ? lds_at(pb, grp - sg * TJ) : (nk ? xch_at(s & 1, 1, grp) : HZ);
-            double xi[NPV], xj[NPV], xk[NPV];
-#pragma unroll
-            for (int q = 0; q < NPV; q++) { xi[q] = hand[oi + q]; xj[q] = hand[oj + q]; xk[q] = hand[ok + q]; }
+            const double xi = hand[oi + ln], xj = hand[oj + ln], xk = hand[ok + ln];
             // dcv = res + the three upstream products, in the reference's i, j, k order
-            double y = mine ? st[ST_RES + lane] : 0.0;
-            jac_row_apply(ci, xi, hand[oi + ln], y);
-            jac_row_apply(cj, xj, hand[oj + ln], y);
-            jac_row_apply(ck, xk, hand[ok + ln], y);
+            double y = own.res;
+            row_apply(ci, xi, y);
+            row_apply(cj, xj, y);
+            row_apply(ck, xk, y);
             __builtin_amdgcn_sched_barrier(0);
             // dq = D^-1 dcv
-            double yv[NPV], pc[NPV];
-            bcast_rows(y, yv);
-#pragma unroll
-            for (int q = 0; q < NPV; q++) pc[q] = st[ST_PV + q];
-            const double xn = getx_apply_sel([&](int q) { return st[ST_GX + q]; }, pc, st[ST_DC + D_RY1],
-                                             st[ST_DC + D_RT], yv, lane, y, st[ST_PV + ln]);
+            const double xn = row_dinv(rows, own, y);
             if (lane < NPV) {
                 lds(s & 1, grp)[lane] = act ? xn : 0.0;
                 if constexpr (FWD) ylds[s % YR][grp][lane] = y;
@@ -1274,15 +1384,21 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             __builtin_amdgcn_sched_barrier(0);
             // coefficients of the next step (independent of dq): this cell's
             // row through its face to the next cell, and the j / k neighbours
-            // of the next cell
-            jac_row_coef(npv, stage_jnb(st, ST_PV, lane, npv), sg, lane, sgn, ci);
+            // of the next cell; and the next cell's own terms
             const WinRow s1{&win[((d + 1) >> 2) & 1][grp][0][slot(d + 1)]};
-            jac_row_coef(npv, stage_jnb(s1, ST_J, lane, npv), sg, lane, sgn, cj);
-            jac_row_coef(npv, stage_jnb(s1, ST_K, lane, npv), sg, lane, sgn, ck);
+            const double j1 = s1[ST_J + rows.v1], j2 = s1[ST_J + rows.v2], jp = s1[ST_J + rows.p];
+            const double k1 = s1[ST_K + rows.v1], k2 = s1[ST_K + rows.v2], kp = s1[ST_K + rows.p];
+            row_coef<FWD>(rows, own.v1, own.v2, own.p, ci);
+            row_coef<FWD>(rows, j1, j2, jp, cj);
+            row_coef<FWD>(rows, k1, k2, kp, ck);
+            own = row_cell(rows, s1, ln);
             // formed before the barrier (while the poll wavefront may still be
             // waiting), not after it on the next step's path
 #pragma unroll
             for (int q = 0; q < 8; q++) asm volatile("" : "+v"(ci[q]), "+v"(cj[q]), "+v"(ck[q]));
+#pragma unroll
+            for (int q = 0; q < 7; q++) asm volatile("" : "+v"(own.g[q]));
+            asm volatile("" : "+v"(own.res), "+v"(own.v1), "+v"(own.v2), "+v"(own.p), "+v"(own.a), "+v"(own.co[0]), "+v"(own.co[1]), "+v"(own.co[2]));
             lds_barrier();
             if (s == sb) break;
         }
