@@ -862,7 +862,7 @@ static_assert(ST_PV + 9 == ST_DC && ST_DC + ND == ST_N3 && ST_N3 + 3 == ST_JC &&
 template <int Q>
 __device__ __forceinline__ double row_lane(double v)
 {
-    return __longlong_as_double(__builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0x150 + Q, 0xF, 0xF, false));
+    return __longlong_as_double(__builtin_amdgcn_mov_dpp(__double_as_longlong(v), 0x150 + Q, 0xF, 0xF, false));
 }
 // Row form of a pencil's step.  A pencil's 16 lanes hold the rows of its
 // cell's system; everything else a step reads (the state, properties, face
