@@ -1068,11 +1068,10 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
     auto lds_at = [](int par, int g) { return (par * TJ * TK + g) * NPV; };
     auto xch_at = [](int par, int a, int g) { return HX + ((par * 2 + a) * TJ * TK + g) * NPV; };
     auto lds = [&](int par, int g) { return hand + lds_at(par, g); };
-    auto xch = [&](int par, int a, int g) { return hand + xch_at(par, a, g); };
     double *const zrow = hand + HZ;
     // dcv of the last YR hyperplanes (forward sweep), by s mod YR: the store
     // wavefront writes a pencil's dcv four cells at a time
-    constexpr int YR = 5;
+    constexpr int YR = 8;      // (five are needed; a power of two makes s mod YR a mask)
     __shared__ double ylds[FWD ? YR : 1][TJ * TK][NPV];
     __shared__ double win[2][TJ * TK][ST_N][WIN];   // stage windows (see the pencil wavefronts)
     __shared__ const double *src[TJ * TK][ST_N];
@@ -1103,10 +1102,6 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
         auto down_edge = [](int g) {
             return FWD ? (g % TJ == TJ - 1 || g / TJ == TK - 1) : (g % TJ == 0 || g / TJ == 0);
         };
-        auto active = [&](int g, int ii) {
-            const int jj = j0 + g % TJ, kk = k0 + g / TJ;
-            return jj <= jend && kk <= kend && ii - jj - kk >= 2 && ii - jj - kk <= B.I;
-        };
         if (wave == 4) {
             // store wavefront: hyperplane s is written out during step s+1,
             // while the pencil wavefronts compute.  The dq that other tiles
@@ -1118,42 +1113,62 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             // together and non-temporal (the backward sweep reads them after
             // this launch); backward, the exchange array also takes the other
             // pencils' dq, the update's input.
+            // The store wavefront shares its SIMD with a pencil wavefront: the
+            // step-independent part of its index arithmetic is done once per
+            // tile (a pencil's row advances by one cell a step).
+            const int l = threadIdx.x - 256;
+            long at[3], from[3];
+            int lo[3], hi[3];
+#pragma unroll
+            for (int q = 0; q < 3; q++) {
+                const int v = l + 64 * q;
+                if constexpr (FWD) {
+                    // dcv of row n, cell (i - 3 + c, j0 + p, k0 + gk): at + i + gk * from
+                    const int p = v / (4 * NPV), n = (v >> 2) % NPV, c = v & 3;
+                    at[q] = n * NW + widx(B, c - 3, j0 + p, k0);
+                    from[q] = (long)(B.I + 1) * (B.J + 1);
+                    lo[q] = hi[q] = 0;
+                } else {
+                    // row n of pencil g at hyperplane s: at + 9 s, for lo <= s <= hi
+                    const int g = min(v / NPV, TJ * TK - 1), n = v % NPV, jj = j0 + g % TJ, kk = k0 + g / TJ;
+                    const bool on = v < TJ * TK * NPV && n < npv && jj <= jend && kk <= kend && !down_edge(g);
+                    at[q] = widx(B, -jj - kk, jj, kk) * NPV + n;
+                    lo[q] = on ? 2 + jj + kk : 1;
+                    hi[q] = on ? B.I + jj + kk : 0;
+                    from[q] = g * NPV + n;
+                }
+            }
             auto publish = [&](int s) {
-                const int pb = s & 1;
                 if constexpr (FWD) {
                     // the four pencils whose window closes at hyperplane s
                     // (j + k = s - 5 mod 4) write its four cells, formed at
                     // hyperplanes s - 3 .. s; lane -> (pencil, row, cell), so
                     // that four adjacent lanes write one row's 32 bytes
                     const int r0 = (s - j0 - k0 - 5) & 3;
-                    for (int v = threadIdx.x - 256; v < 4 * NPV * 4; v += 64) {
-                        const int p = v / (4 * NPV), n = (v >> 2) % NPV, c = v & 3;
+#pragma unroll
+                    for (int q = 0; q < 3; q++) {
+                        const int v = l + 64 * q, p = v / (4 * NPV), n = (v >> 2) % NPV, c = v & 3;
                         // the class's pencil with gj = p: gj + gk = r0, or r0 + 4 past the tile's anti-diagonal
-                        const int gj = p, gk = r0 + 4 * (p > r0) - p;
-                        const int jj = j0 + gj, kk = k0 + gk, i = s - jj - kk;
-                        if (n < npv && jj <= jend && kk <= kend && i >= 5 && i <= B.I)
-                            __builtin_nontemporal_store(ylds[(s - 3 + c) % YR][gj + TJ * gk][n], S.dcv + n * NW + widx(B, i - 3 + c, jj, kk));
+                        const int gk = r0 + 4 * (p > r0) - p, i = s - j0 - k0 - p - gk;
+                        if (v < 4 * NPV * 4 && n < npv && j0 + p <= jend && k0 + gk <= kend && i >= 5 && i <= B.I)
+                            __builtin_nontemporal_store(ylds[(s - 3 + c) & (YR - 1)][p + TJ * gk][n], S.dcv + at[q] + (i + (long)gk * from[q]));
                     }
                     // a pencil that ends at hyperplane s in the middle of a window
                     if (s >= B.I + j0 + k0) {
-                        for (int e = threadIdx.x - 256; e < TJ * TK * NPV; e += 64) {
+                        for (int e = l; e < TJ * TK * NPV; e += 64) {
                             const int g = e / NPV, n = e - g * NPV;
                             const int jj = j0 + g % TJ, kk = k0 + g / TJ, i = s - jj - kk;
                             const int m = (i - 2) & 3;
                             if (n < npv && i == B.I && m != 3 && jj <= jend && kk <= kend) {
                                 double *o = S.dcv + n * NW + widx(B, i - m, jj, kk);
-                                for (int c = 0; c <= m; c++) __builtin_nontemporal_store(ylds[(s - m + c) % YR][g][n], o + c);
+                                for (int c = 0; c <= m; c++) __builtin_nontemporal_store(ylds[(s - m + c) & (YR - 1)][g][n], o + c);
                             }
                         }
                     }
                 } else {
-                    for (int e = threadIdx.x - 256; e < TJ * TK * NPV; e += 64) {
-                        const int g = e / NPV, n = e - g * NPV;
-                        if (n < npv && active(g, s) && !down_edge(g)) {
-                            const int jj = j0 + g % TJ, kk = k0 + g / TJ, i = s - jj - kk;
-                            xq[widx(B, i, jj, kk) * NPV + n] = lds(pb, g)[n];
-                        }
-                    }
+#pragma unroll
+                    for (int q = 0; q < 3; q++)
+                        if (s >= lo[q] && s <= hi[q]) xq[at[q] + (long)s * NPV] = hand[(s & 1) * TJ * TK * NPV + (int)from[q]];
                 }
             };
             __syncthreads();
@@ -1238,20 +1253,31 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             // e = q / 9 % 4 along the edge; row n = q % 9)
             const int l64 = threadIdx.x - 320;
             const double *dummy = xq + widx(B, min(max(sa - j0 - k0, 2), B.I), j0, k0) * NPV;
-            auto item = [&](int q, int s, bool &need) -> const double * {
-                const int a = q / (4 * NPV), e = (q / NPV) % 4, n = q % NPV;
+            // per lane and tile: item t's value of step s is at xq[at + 9 s],
+            // read for lo <= s <= hi (the cell is inside the block and its
+            // neighbour too), and goes to the hand-over slot to (+ parity)
+            long at[2];
+            int lo[2], hi[2], to[2];
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const int q = min(l64 + 64 * t, NEDGE - 1), a = q / (4 * NPV), e = (q / NPV) % 4, n = q % NPV;
                 const int g = a == 0 ? e * TJ + (FWD ? 0 : TJ - 1) : (FWD ? 0 : TK - 1) * TJ + e;
                 const int jj = j0 + g % TJ, kk = k0 + g / TJ;
                 const int jn = a == 0 ? jj - sg : jj, kn = a == 0 ? kk : kk - sg;
-                need = q < NEDGE && n < npv && active(g, s) && jn >= 2 && jn <= B.J && kn >= 2 && kn <= B.K;
-                return need ? xq + widx(B, s - jj - kk, jn, kn) * NPV + n : dummy;
-            };
+                const bool on = l64 + 64 * t < NEDGE && n < npv && jj <= jend && kk <= kend && jn >= 2 && jn <= B.J && kn >= 2 && kn <= B.K;
+                at[t] = widx(B, -jj - kk, jn, kn) * NPV + n;
+                lo[t] = on ? 2 + jj + kk : 1;
+                hi[t] = on ? B.I + jj + kk : 0;
+                to[t] = xch_at(0, a, g) + n;
+            }
             bool n0, n1;
             const double *p0, *p1;
             double v0, v1;
             auto issue = [&](int s) {            // loads for step s (unconditional: the count of loads never varies)
-                p0 = item(l64, s, n0);
-                p1 = item(l64 + 64, s, n1);
+                n0 = s >= lo[0] && s <= hi[0];
+                n1 = s >= lo[1] && s <= hi[1];
+                p0 = n0 ? xq + at[0] + (long)s * NPV : dummy;
+                p1 = n1 ? xq + at[1] + (long)s * NPV : dummy;
                 v0 = ld_dev(p0);
                 v1 = ld_dev(p1);
             };
@@ -1271,15 +1297,9 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
                         if (unset(n1, v1)) v1 = ld_dev(p1);
                     } while (__ballot(unset(n0, v0) || unset(n1, v1)));
                 }
-                const int par = s & 1;
-                for (int t = 0; t < 2; t++) {
-                    const int q = l64 + 64 * t;
-                    if (q < NEDGE) {
-                        const int a = q / (4 * NPV), e = (q / NPV) % 4, n = q % NPV;
-                        const int g = a == 0 ? e * TJ + (FWD ? 0 : TJ - 1) : (FWD ? 0 : TK - 1) * TJ + e;
-                        xch(par, a, g)[n] = (t == 0 ? n0 : n1) ? (t == 0 ? v0 : v1) : 0.0;
-                    }
-                }
+                const int par = (s & 1) * (xch_at(1, 0, 0) - xch_at(0, 0, 0));
+                hand[to[0] + par] = n0 ? v0 : 0.0;
+                if (l64 < NEDGE - 64) hand[to[1] + par] = n1 ? v1 : 0.0;
             };
             issue(sa);
             deliver(sa);
@@ -1376,7 +1396,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             const double xn = row_dinv(rows, own, y);
             if (lane < NPV) {
                 lds(s & 1, grp)[lane] = act ? xn : 0.0;
-                if constexpr (FWD) ylds[s % YR][grp][lane] = y;
+                if constexpr (FWD) ylds[s & (YR - 1)][grp][lane] = y;
                 // the pencil wavefronts have no loads in flight, so this store
                 // costs only its issue
                 if (edge && act && mine) st_dev(xq + widx(B, i, j, k) * NPV + lane, xn);
