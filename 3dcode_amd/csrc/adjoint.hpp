@@ -11,25 +11,18 @@
 // and the two scalar derivatives of res_bar . res with respect to p_ref and
 // u_ref.  The reference has no adjoint; this is the VJP of its residual.
 //
-// Method: reverse accumulation over faces and cells, local derivatives in
-// forward mode.  Each face recomputes its reconstruction and flux (nothing is
-// kept from a forward pass) and takes the gradient of
-//   phi_f = g_f . F_f,   g_f = res_bar(right cell) - res_bar(left cell)
-// through dual-number passes (Dn<W>: W inputs seeded per pass) of the same
-// templated physics the residual kernels run, split where the input count is
-// smallest:
-//   flux core       the two face states, rho and h (c^2) of each side, the
-//                   Roe-averaged c^2, [the 18 sensor pressures], u_ref
-//   averaged c^2    the ten quantities it is built from
-//   face EOS        (p, T, y1, y2) of each side
-//   clamps          each clamped value comes from the reconstruction, the
-//                   cell or a constant (recorded in the forward recompute)
-//   reconstruction  each variable's stencil (38 points under MLP, 6 under TVD)
-// The per-face bars of every stencil point go to a buffer and each cell
-// gathers its own in a fixed order: the result is deterministic, with no
-// atomics.  The cell sources are handled per cell the same way, and each
-// cell's property bars return to (p, T, y1, y2) through one 4-lane dual pass
-// of the EOS.  Arithmetic is FP64 throughout.
+// Method: reverse accumulation over faces and cells.  Each face recomputes its
+// reconstruction and flux (nothing is kept from a forward pass) and runs them
+// backwards from g_f = res_bar(right cell) - res_bar(left cell)
+// (adjoint_point.hpp), leaving the bars of its two reconstructed states and
+// of its viscous differences.  A stencil pass (k_adj_stencil) then takes those
+// through the reconstruction and the differences to the stencil points, one
+// wavefront per tile of cells and variable: it runs every face whose stencil
+// reaches its cells, in a fixed order, and adds what falls on them in LDS, so
+// no bars of stencil points are written to memory and the result is
+// deterministic.  The cell sources are differentiated per cell (two-lane dual
+// passes), and each cell's property bars return to (p, T, y1, y2) through its
+// EOS.  Arithmetic is FP64 throughout.
 //
 // d/d(p_ref) is the sum of pv_bar over the pressure component: the residual
 // reads gauge pressure only as p + p_ref or in differences (the pressure
@@ -45,18 +38,20 @@ namespace {
 
 struct AD {
     const double *rb;       // res_bar [npv][NC]
-    double *fb[3];          // bars of a face's stencil points [NSLOT][npv][NF]
-    double *rsb[3];         // a face's reconstruction seeds [4][npv][NF]: left, right, left cell, right cell
+    double *w[3];           // a face's reconstruction bars [2][npv][NF]: left, right
+    int *cell[3];           // which of them belong to the cells' own values (FaceBar::cell) [NF]
     double *snb[3];         // a face's sensor-pressure bars [18][NF] (Roe-M, AUSMPW+)
-    double *db[3];          // cell-property bars of a face's two cells [2][ND][NF]
+    double *fp[3];          // first-order faces: bars of rho, h, c^2 of the two cells [2][3][NF]
+    double *vb[3];          // a face's viscous bars [3 nv + ncv][NF]: differences, averages
+    double *vp[3];          // and of its cells' properties [5][NF]: mu, kappa, rho (each side), h_T left, right
     double *ub[3];          // d(phi_f)/d(u_ref) [NF]
     double *cb;             // cell-source bars on the 7-point stencil [7][npv][NC]
-    double *cdb;            // cell-source property bars [ND][NC]
+    double *cdb;            // cell-source property bars [3][NC]: rho, h, mu
     double *csb;            // cell-source d(phi_c)/d(u_ref, dp_ref, t_ref) [3][NC] (the mass-transfer scales)
     double *pb;             // pv_bar [npv][NG]
-    double *gdb;            // a ghosted cell's gathered property bars [ND][NG], for the EOS pass
     double *mtb[3];         // eddy-viscosity bars of a face's two cells [2][NF] (dmut)
-    unsigned long long mask;   // stencil points a face writes (bit ll-1)
+    const int *tiles;       // tiles of the stencil pass: block, first i, j, k
+    int ntiles;
     int dmut;               // 1: the interior cells' eddy viscosity is the SST function of
                             // the state (differentiated); 0: held fixed
 };
@@ -89,9 +84,9 @@ __device__ __forceinline__ bool face_exists(const BlkD &B, int D, int i, int j, 
     return i >= lo[0] && i <= B.I && j >= lo[1] && j <= B.J && k >= lo[2] && k <= B.K;
 }
 
-// Inviscid part of a face up to its reconstruction: the seeds of the
-// reconstruction (k_face_rvjp takes them to the stencil points), the two
-// cells' property bars and the u_ref derivative.
+// Inviscid part of a face up to its reconstruction: the bars of its left and
+// right states (k_adj_stencil takes them to the stencil points), the cells'
+// property bars (first order) and the u_ref derivative.
 template <int D, bool SENSOR>
 __global__ __launch_bounds__(128) void k_face_vjp(DS S, AD A)
 {
@@ -112,61 +107,39 @@ __global__ __launch_bounds__(128) void k_face_vjp(DS S, AD A)
         g[n] = n < npv ? rbar(S, A, B, ip, jp, kp, n) - rbar(S, A, B, i, j, k, n) : 0.0;
         any = any || g[n] != 0.0;
     }
-    double *rsb = A.rsb[D], *db = A.db[D];
-    if (!any) {
-        for (int m = 0; m < 4 * npv; m++) rsb[m * NF + t] = 0.0;
-        if (SENSOR) for (int q = 0; q < 18; q++) A.snb[D][q * NF + t] = 0.0;
-        for (int m = 0; m < 2 * ND; m++) db[m * NF + t] = 0.0;
-        A.ub[D][t] = 0.0;
-        return;
+    FaceBar o;
+    if (any) {
+        const double *f0 = S.pv + g9;
+        double n3[3];
+        face_vec(S, B, D, i, j, k, n3);
+        const double cellp[6] = {S.dc[D_RHO * S.NG + g9], S.dc[D_H * S.NG + g9], S.dc[D_C2 * S.NG + g9],
+                                 S.dc[D_RHO * S.NG + gq], S.dc[D_H * S.NG + gq], S.dc[D_C2 * S.NG + gq]};
+        face_adj_core<SENSOR>(P, npv, [&](int ll, int n) -> double { return f0[(long)n * S.NG + stencil_off<D>(B, ll)]; },
+                              n3, cellp, g, o);
+    } else {
+        for (int n = 0; n < NPV; n++) o.wl[n] = o.wr[n] = 0.0;
+        for (int q = 0; q < 18; q++) o.sen[q] = 0.0;
+        for (int q = 0; q < 3; q++) o.prop[0][q] = o.prop[1][q] = 0.0;
+        o.uref = 0.0;
+        o.cell = 0;
     }
-    const double *f0 = S.pv + g9;
-    long off[NSLOT];
-    for (int ll = 1; ll <= NSLOT; ll++) off[ll - 1] = stencil_off<D>(B, ll);
-    double n3[3];
-    face_vec(S, B, D, i, j, k, n3);
-    const double cellp[6] = {S.dc[D_RHO * S.NG + g9], S.dc[D_H * S.NG + g9], S.dc[D_C2 * S.NG + g9],
-                             S.dc[D_RHO * S.NG + gq], S.dc[D_H * S.NG + gq], S.dc[D_C2 * S.NG + gq]};
-    double ub, xlb[NPV], xrb[NPV], c9b[NPV], c10b[NPV], senb[18];
-    face_adj_core<SENSOR>(P, npv, f0, S.NG, off, n3, cellp, g, xlb, xrb, c9b, c10b, senb, db + t, NF, ub);
-    for (int n = 0; n < npv; n++) {
-        rsb[(0 * npv + n) * NF + t] = xlb[n];
-        rsb[(1 * npv + n) * NF + t] = xrb[n];
-        rsb[(2 * npv + n) * NF + t] = c9b[n];
-        rsb[(3 * npv + n) * NF + t] = c10b[n];
+    for (int n = 0; n < NPV; n++) if (n < npv) {
+        A.w[D][(long)n * NF + t] = o.wl[n];
+        A.w[D][(long)(npv + n) * NF + t] = o.wr[n];
     }
-    if (SENSOR) for (int q = 0; q < 18; q++) A.snb[D][q * NF + t] = senb[q];
-    A.ub[D][t] = ub;
+    A.cell[D][t] = o.cell;
+    if (SENSOR) for (int q = 0; q < 18; q++) A.snb[D][q * NF + t] = o.sen[q];
+    if (P.nmuscl == 0)
+        for (int q = 0; q < 3; q++) {
+            A.fp[D][q * NF + t] = o.prop[0][q];
+            A.fp[D][(3 + q) * NF + t] = o.prop[1][q];
+        }
+    A.ub[D][t] = o.uref;
 }
 
-// The reconstruction part of a face's inviscid adjoint, one thread per face
-// and variable: the seeds k_face_vjp left, back to the face's stencil points.
-template <int D, bool SENSOR>
-__global__ __launch_bounds__(256) void k_face_rvjp(DS S, AD A)
-{
-    const long NF = S.NF[D];
-    long u = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (u >= (long)S.npv * NF) return;
-    const int n = (int)(u / NF);
-    const long t = u - (long)n * NF;
-    int i, j, k;
-    const BlkD &B = face_of<D>(S, t, i, j, k);
-    const int npv = S.npv;
-    const double *rsb = A.rsb[D];
-    const double *f0 = S.pv + (long)n * S.NG + gidx(B, i, j, k);
-    const double *senb = nullptr;
-    double sn18[18];
-    if (SENSOR && n == 0) {
-        for (int q = 0; q < 18; q++) sn18[q] = A.snb[D][q * NF + t];
-        senb = sn18;
-    }
-    face_adj_recon(S.P, n, [&](int ll) -> double { return f0[stencil_off<D>(B, ll)]; }, rsb[(0 * npv + n) * NF + t],
-                   rsb[(1 * npv + n) * NF + t], rsb[(2 * npv + n) * NF + t], rsb[(3 * npv + n) * NF + t], senb, A.mask,
-                   A.fb[D] + (long)n * NF + t, (long)npv * NF);
-}
-
-// Viscous part of a face, added to the inviscid bars (stencil points 1..18,
-// the two cells' mu, kappa and, under SST, h_T and rho).
+// Viscous part of a face: the bars of its differences and averages (linear in
+// the stencil, k_adj_stencil applies them), of the two cells' mu, kappa and,
+// under SST, rho, h_T and eddy viscosity.
 template <int D>
 __global__ __launch_bounds__(128) void k_vface_vjp(DS S, AD A)
 {
@@ -182,34 +155,24 @@ __global__ __launch_bounds__(128) void k_vface_vjp(DS S, AD A)
     const long gq = g9 + sN;
     int ip = i, jp = j, kp = k;
     if (D == 0) ip++; else if (D == 1) jp++; else kp++;
-    double g[NPV];
-    bool any = false;
-    for (int n = 0; n < NPV; n++) {
-        g[n] = n < npv ? rbar(S, A, B, i, j, k, n) - rbar(S, A, B, ip, jp, kp, n) : 0.0;
-        any = any || g[n] != 0.0;
-    }
+    double gf[NPV];
+    for (int n = 0; n < NPV; n++) gf[n] = n < npv ? rbar(S, A, B, i, j, k, n) - rbar(S, A, B, ip, jp, kp, n) : 0.0;
     const bool turb = P.iturb == 0;
-    const bool dm = A.dmut && turb;
-    if (!any) {
-        if (dm) { A.mtb[D][t] = 0.0; A.mtb[D][NF + t] = 0.0; }
-        return;
-    }
-    const int nv = turb ? 6 : 4;
-    const int vars[6] = {1, 2, 3, 4, 7, 8};
-    auto xs = [&](int ll, int n) -> double { return S.pv[(long)n * S.NG + g9 + stencil_off<D>(B, ll)]; };
+    const int nv = turb ? 6 : 4, ncv = turb ? 5 : 3;
     // inputs: the normal / transverse differences, the face averages, the cell properties
     double g3[6][3], cav[5];
-    for (int q = 0; q < nv; q++) {
-        const int n = vars[q];
-        g3[q][0] = xs(10, n) - xs(9, n);
-        g3[q][1] = 0.0625 * (-xs(1, n) - xs(2, n) + xs(5, n) + xs(6, n) + 2.0 * (-xs(7, n) - xs(8, n) + xs(11, n) + xs(12, n))
-                             - xs(13, n) - xs(14, n) + xs(17, n) + xs(18, n));
-        g3[q][2] = 0.0625 * (-xs(1, n) - xs(2, n) + xs(13, n) + xs(14, n) + 2.0 * (-xs(3, n) - xs(4, n) + xs(15, n) + xs(16, n))
-                             - xs(5, n) - xs(6, n) + xs(17, n) + xs(18, n));
+#pragma unroll
+    for (int q = 0; q < 6; q++) {
+        const int n = q < 4 ? q + 1 : q + 3;
+        if (q >= nv) { g3[q][0] = g3[q][1] = g3[q][2] = 0.0; continue; }
+        auto xs = [&](int ll) -> double { return S.pv[(long)n * S.NG + g9 + stencil_off<D>(B, ll)]; };
+        g3[q][0] = xs(10) - xs(9);
+        g3[q][1] = 0.0625 * (-xs(1) - xs(2) + xs(5) + xs(6) + 2.0 * (-xs(7) - xs(8) + xs(11) + xs(12)) - xs(13) - xs(14) + xs(17) + xs(18));
+        g3[q][2] = 0.0625 * (-xs(1) - xs(2) + xs(13) + xs(14) + 2.0 * (-xs(3) - xs(4) + xs(15) + xs(16)) - xs(5) - xs(6) + xs(17) + xs(18));
+        if (q < 3) cav[q] = 0.5 * (xs(9) + xs(10));
+        if (q > 3) cav[q - 1] = 0.5 * (xs(9) + xs(10));
     }
-    const int ncv = turb ? 5 : 3;
-    const int cvar[5] = {1, 2, 3, 7, 8};
-    for (int q = 0; q < ncv; q++) cav[q] = 0.5 * (xs(9, cvar[q]) + xs(10, cvar[q]));
+    if (!turb) cav[3] = cav[4] = 0.0;
     double dl[ND], dr[ND];
     for (int m = 0; m < ND; m++) { dl[m] = S.dc[m * S.NG + g9]; dr[m] = S.dc[m * S.NG + gq]; }
     const double ml = S.mut ? S.mut[g9] : 0.0, mr = S.mut ? S.mut[gq] : 0.0;
@@ -238,46 +201,186 @@ __global__ __launch_bounds__(128) void k_vface_vjp(DS S, AD A)
     face_vec(S, B, T, p1[0], p1[1], p1[2], t4[3]);
     const long wl = widx(B, i, j, k), wr = widx(B, ip, jp, kp);
     const double gl[2] = {S.vol[wl], S.ydn ? S.ydn[wl] : 1.0}, gr[2] = {S.vol[wr], S.ydn ? S.ydn[wr] : 1.0};
-    // z = {g3[nv][3], cav[ncv], muL, kapL, muR, kapR, [hTL, hTR, rhoL, rhoR, [mutL, mutR]]}
-    constexpr int NZ = 18 + 5 + 8 + 2;
-    const int og = 3 * nv, oc = og + ncv;
-    const int nz = oc + (turb ? (dm ? 10 : 8) : 4);
-    double zx[NZ], zb[NZ];
-    for (int q = 0; q < nv; q++) for (int c = 0; c < 3; c++) zx[3 * q + c] = g3[q][c];
-    for (int q = 0; q < ncv; q++) zx[og + q] = cav[q];
-    zx[oc] = dl[D_MU]; zx[oc + 1] = dl[D_KAP]; zx[oc + 2] = dr[D_MU]; zx[oc + 3] = dr[D_KAP];
-    if (turb) { zx[oc + 4] = dl[D_HT]; zx[oc + 5] = dr[D_HT]; zx[oc + 6] = dl[D_RHO]; zx[oc + 7] = dr[D_RHO]; }
-    if (dm) { zx[oc + 8] = ml; zx[oc + 9] = mr; }
-    visc_adj(P, npv, nv, ncv, nz, zx, n3, e4, t4, gl, gr, dl, dr, ml, mr, dm ? oc + 8 : -1, g, zb);
-    if (dm) { A.mtb[D][t] = zb[oc + 8]; A.mtb[D][NF + t] = zb[oc + 9]; }
-    // the differences and averages are linear in the stencil
-    double *fb = A.fb[D];
-    constexpr double C1[18] = {-1, -1, 0, 0, 1, 1, -2, -2, 0, 0, 2, 2, -1, -1, 0, 0, 1, 1};
-    constexpr double C2[18] = {-1, -1, -2, -2, -1, -1, 0, 0, 0, 0, 0, 0, 1, 1, 2, 2, 1, 1};
-    for (int q = 0; q < nv; q++) {
-        const int n = vars[q];
-        for (int ll = 1; ll <= 18; ll++) {
-            double v = 0.0625 * (C1[ll - 1] * zb[3 * q + 1] + C2[ll - 1] * zb[3 * q + 2]);
-            if (ll == 9) v -= zb[3 * q];
-            if (ll == 10) v += zb[3 * q];
-            if (v != 0.0) fb[((long)(ll - 1) * npv + n) * NF + t] += v;
+    ViscBar o;
+    visc_back(P, n3, e4, t4, gl, gr, g3, cav, dl, dr, ml, mr, gf, o);
+    double *vb = A.vb[D], *vp = A.vp[D];
+#pragma unroll
+    for (int q = 0; q < 6; q++) if (q < nv) for (int c = 0; c < 3; c++) vb[(long)(3 * q + c) * NF + t] = o.g3[q][c];
+#pragma unroll
+    for (int q = 0; q < 5; q++) if (q < ncv) vb[(long)(3 * nv + q) * NF + t] = o.cav[q];
+    vp[t] = o.mu;
+    vp[NF + t] = o.kap;
+    if (turb) {
+        vp[2 * NF + t] = o.rho;
+        vp[3 * NF + t] = o.ht[0];
+        vp[4 * NF + t] = o.ht[1];
+        if (A.dmut) { A.mtb[D][t] = o.mut[0]; A.mtb[D][NF + t] = o.mut[1]; }
+    }
+}
+
+// The stencil pass: one wavefront owns a tile of AI x AJ x AK ghosted cells of
+// one variable and adds to them, in LDS, what every face whose stencil
+// reaches the tile leaves on its points: the reconstruction run backwards
+// from the face's two bars (muscl_back) and the viscous differences'
+// transposes.  Faces near a tile's edge are run by every tile they reach
+// (twice on average at 16 x 8 x 8), which costs arithmetic but no memory: with
+// the bars of all 38 points written per face and variable and gathered by a
+// second kernel, a product moved 9 GB through them at 128 x 64 x 64.  Within
+// one LDS add the lanes (distinct faces, one stencil point) hit distinct
+// cells, and a wavefront's LDS operations run in its program order, so the
+// sums have a fixed order.
+constexpr int AI = 16, AJ = 8, AK = 8;
+template <int D, int NM>
+__device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, const BlkD &B, const int *c0, const int *c1, int n,
+                                                int vq, int cq, int nv, const double *sen, double *acc)
+{
+    constexpr int E = (D + 1) % 3, T = (D + 2) % 3;
+    const int npv = S.npv, ext[3] = {B.I, B.J, B.K}, lane = threadIdx.x;
+    const long NF = S.NF[D];
+    int lo[3], cnt[3];
+    lo[D] = max(c0[D] - 3, 1);
+    lo[E] = max(c0[E] - 1, 2);
+    lo[T] = max(c0[T] - 1, 2);
+    cnt[D] = min(c1[D] + 2, ext[D]) - lo[D] + 1;
+    cnt[E] = min(c1[E] + 1, ext[E]) - lo[E] + 1;
+    cnt[T] = min(c1[T] + 1, ext[T]) - lo[T] + 1;
+    if (cnt[0] <= 0 || cnt[1] <= 0 || cnt[2] <= 0) return;
+    const int total = cnt[0] * cnt[1] * cnt[2];
+    constexpr int st[3] = {1, AI, AI * AJ};
+    for (int base = 0; base < total; base += 64) {
+        const int r = base + lane;
+        const bool on = r < total;
+        const int q = on ? r : 0;
+        const int f[3] = {lo[0] + q % cnt[0], lo[1] + (q / cnt[0]) % cnt[1], lo[2] + q / (cnt[0] * cnt[1])};
+        const long t = fidx(B, D, f[0], f[1], f[2]);
+        double wl = A.w[D][(long)n * NF + t], wr = A.w[D][(long)(npv + n) * NF + t];
+        const int cell = A.cell[D][t];
+        // the face's left cell in tile coordinates; which offsets along each axis land in the tile
+        const int l[3] = {f[0] - c0[0], f[1] - c0[1], f[2] - c0[2]};
+        const int w3[3] = {c1[0] - c0[0], c1[1] - c0[1], c1[2] - c0[2]};
+        bool inN[6], inE[3], inT[3];
+#pragma unroll
+        for (int d = 0; d < 6; d++) inN[d] = on && (unsigned)(l[D] + d - 2) <= (unsigned)w3[D];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            inE[d] = (unsigned)(l[E] + d - 1) <= (unsigned)w3[E];
+            inT[d] = (unsigned)(l[T] + d - 1) <= (unsigned)w3[T];
+        }
+        const int at = l[0] * st[0] + l[1] * st[1] + l[2] * st[2];
+        auto add = [&](int ll, double v) {
+            int dn, de, dt;
+            stencil_ijk(ll, dn, de, dt);
+            if (inN[dn + 2] && inE[de + 1] && inT[dt + 1])
+                __hip_atomic_fetch_add(&acc[at + dn * st[D] + de * st[E] + dt * st[T]], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+        const bool cl = NM == 0 || ((cell >> n) & 1), cr = NM == 0 || ((cell >> (16 + n)) & 1);
+        double b9 = cl ? wl : 0.0, b10 = cr ? wr : 0.0;
+        wl = cl ? 0.0 : wl;
+        wr = cr ? 0.0 : wr;
+        ReconBar o;
+        o.x9 = o.x10 = o.x23 = o.x32 = o.x37 = o.x38 = 0.0;
+        o.x3 = o.x4 = o.x7 = o.x8 = o.x11 = o.x12 = o.x15 = o.x16 = o.el = o.er = 0.0;
+        o.il = o.ir = 0;
+        if constexpr (NM > 0) {
+            const bool rec = on && (wl != 0.0 || wr != 0.0);
+            if (__ballot(rec)) {
+                const double *f0 = S.pv + (long)n * S.NG + gidx(B, f[0], f[1], f[2]);
+                double x[NSLOT];
+#pragma unroll
+                for (int ll = 1; ll <= NSLOT; ll++)
+                    if (NM == 2 || ll == 9 || ll == 10 || ll == 23 || ll == 32 || ll >= 37) x[ll - 1] = f0[stencil_off<D>(B, ll)];
+                if (rec) o = muscl_back<NM == 2>(S.P.nlim, [&](int ll) -> double { return x[ll - 1]; }, wl, wr);
+            }
+        }
+        b9 += o.x9;
+        b10 += o.x10;
+        if (vq >= 0 || sen) {
+            // the 18 points of the viscous differences (and of the pressure sensor)
+            double v0 = 0.0, v1 = 0.0, v2 = 0.0, vc = 0.0;
+            if (vq >= 0) {
+                v0 = A.vb[D][(long)(3 * vq) * NF + t];
+                v1 = 0.0625 * A.vb[D][(long)(3 * vq + 1) * NF + t];
+                v2 = 0.0625 * A.vb[D][(long)(3 * vq + 2) * NF + t];
+                if (cq >= 0) vc = 0.5 * A.vb[D][(long)(3 * nv + cq) * NF + t];
+            }
+            auto sn = [&](int ll) -> double { return sen ? sen[(long)(ll - 1) * NF + t] : 0.0; };
+            add(1, -v1 - v2 + sn(1));
+            add(2, -v1 - v2 + sn(2));
+            add(3, o.x3 - 2.0 * v2 + sn(3));
+            add(4, o.x4 - 2.0 * v2 + sn(4));
+            add(5, v1 - v2 + sn(5));
+            add(6, v1 - v2 + sn(6));
+            add(7, o.x7 - 2.0 * v1 + sn(7));
+            add(8, o.x8 - 2.0 * v1 + sn(8));
+            add(9, b9 + vc - v0 + sn(9));
+            add(10, b10 + vc + v0 + sn(10));
+            add(11, o.x11 + 2.0 * v1 + sn(11));
+            add(12, o.x12 + 2.0 * v1 + sn(12));
+            add(13, -v1 + v2 + sn(13));
+            add(14, -v1 + v2 + sn(14));
+            add(15, o.x15 + 2.0 * v2 + sn(15));
+            add(16, o.x16 + 2.0 * v2 + sn(16));
+            add(17, v1 + v2 + sn(17));
+            add(18, v1 + v2 + sn(18));
+        } else {
+            add(9, b9);
+            add(10, b10);
+            if constexpr (NM == 2) {
+                add(3, o.x3); add(4, o.x4); add(7, o.x7); add(8, o.x8);
+                add(11, o.x11); add(12, o.x12); add(15, o.x15); add(16, o.x16);
+            }
+        }
+        if constexpr (NM > 0) {
+            add(23, o.x23);
+            add(32, o.x32);
+            add(37, o.x37);
+            add(38, o.x38);
+        }
+        if constexpr (NM == 2) {
+            // the extrema the bounds selected: lanes of one stencil point at a time
+            auto extremum = [&](int il, double v) {
+                unsigned long long todo = __ballot(on && il != 0);
+                while (todo) {
+                    const int ll = __builtin_amdgcn_readlane(il, __builtin_ctzll(todo));
+                    const bool mine = on && il == ll;
+                    todo &= ~__ballot(mine);
+                    int dn, de, dt;
+                    stencil_ijk(ll, dn, de, dt);
+                    if (mine && (unsigned)(l[D] + dn) <= (unsigned)w3[D] && (unsigned)(l[E] + de) <= (unsigned)w3[E] &&
+                        (unsigned)(l[T] + dt) <= (unsigned)w3[T])
+                        __hip_atomic_fetch_add(&acc[at + dn * st[D] + de * st[E] + dt * st[T]], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
+            };
+            extremum(o.il, o.el);
+            extremum(o.ir, o.er);
         }
     }
-    for (int q = 0; q < ncv; q++) {
-        const int n = cvar[q];
-        fb[((long)8 * npv + n) * NF + t] += 0.5 * zb[og + q];
-        fb[((long)9 * npv + n) * NF + t] += 0.5 * zb[og + q];
-    }
-    double *db = A.db[D];
-    db[D_MU * NF + t] += zb[oc];
-    db[D_KAP * NF + t] += zb[oc + 1];
-    db[(ND + D_MU) * NF + t] += zb[oc + 2];
-    db[(ND + D_KAP) * NF + t] += zb[oc + 3];
-    if (turb) {
-        db[D_HT * NF + t] += zb[oc + 4];
-        db[(ND + D_HT) * NF + t] += zb[oc + 5];
-        db[D_RHO * NF + t] += zb[oc + 6];
-        db[(ND + D_RHO) * NF + t] += zb[oc + 7];
+}
+
+template <int NM>
+__global__ __launch_bounds__(64) void k_adj_stencil(DS S, AD A)
+{
+    __shared__ double acc[AI * AJ * AK];
+    const int n = blockIdx.x / A.ntiles, lane = threadIdx.x;
+    const int *td = A.tiles + 4 * (blockIdx.x - n * A.ntiles);
+    const BlkD &B = S.b[td[0]];
+    const int c0[3] = {td[1], td[2], td[3]};
+    const int c1[3] = {min(c0[0] + AI - 1, B.I + 3), min(c0[1] + AJ - 1, B.J + 3), min(c0[2] + AK - 1, B.K + 3)};
+    for (int q = lane; q < AI * AJ * AK; q += 64) acc[q] = 0.0;
+    const bool visc = S.P.iturb >= -2;
+    // the variable's place among the viscous differences (u, v, w, T, k, omega) and averages (u, v, w, k, omega)
+    const int vq = !visc ? -1 : (n >= 1 && n <= 4) ? n - 1 : n >= 7 ? n - 3 : -1;
+    const int cq = !visc ? -1 : (n >= 1 && n <= 3) ? n - 1 : n >= 7 ? n - 4 : -1;
+    const int nv = S.P.iturb == 0 ? 6 : 4;
+    const bool sensor = n == 0 && (S.P.nscheme == 2 || S.P.nscheme == 3);
+    adj_stencil_dir<0, NM>(S, A, B, c0, c1, n, vq, cq, nv, sensor ? A.snb[0] : nullptr, acc);
+    adj_stencil_dir<1, NM>(S, A, B, c0, c1, n, vq, cq, nv, sensor ? A.snb[1] : nullptr, acc);
+    adj_stencil_dir<2, NM>(S, A, B, c0, c1, n, vq, cq, nv, sensor ? A.snb[2] : nullptr, acc);
+    __syncthreads();
+    double *pb = A.pb + (long)n * S.NG;
+    for (int q = lane; q < AI * AJ * AK; q += 64) {
+        const int i = c0[0] + q % AI, j = c0[1] + (q / AI) % AJ, k = c0[2] + q / (AI * AJ);
+        if (i <= c1[0] && j <= c1[1] && k <= c1[2]) pb[gidx(B, i, j, k)] = acc[q];
     }
 }
 
@@ -448,18 +551,17 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                         v += wq[q][0] * zb[og + 3 * gv] + wq[q][1] * zb[og + 3 * gv + 1] + wq[q][2] * zb[og + 3 * gv + 2];
             A.cb[((long)q * npv + n) * S.NC + t] = v;
         }
-    for (int m = 0; m < ND; m++) A.cdb[(long)m * S.NC + t] = 0.0;
-    A.cdb[(long)D_RHO * S.NC + t] = zb[od];
-    A.cdb[(long)D_H * S.NC + t] = zb[od + 1];
-    A.cdb[(long)D_MU * S.NC + t] = zb[od + 2];
+    A.cdb[t] = zb[od];
+    A.cdb[S.NC + t] = zb[od + 1];
+    A.cdb[2 * S.NC + t] = zb[od + 2];
     for (int q = 0; q < 3; q++) A.csb[(long)q * S.NC + t] = sc ? zb[osc + q] : 0.0;
 }
 
-// pv_bar of every ghosted cell: its bars from the faces whose stencils hold
-// it and from the sources of its neighbours, in a fixed order, and its
-// gathered property bars (k_adj_eos takes those through the EOS: the dual
-// pass needs the registers this memory-bound gather does not).
-__global__ __launch_bounds__(256) void k_adj_gather(DS S, AD A)
+// The rest of pv_bar of every ghosted cell, added to what k_adj_stencil left:
+// the bars of its neighbours' sources, and its property bars (from the faces
+// whose cell it is and from its own sources) taken through its EOS, in a
+// fixed order.
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adj_cells(DS S, AD A)
 {
     long gl = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (gl >= S.NG) return;
@@ -468,69 +570,56 @@ __global__ __launch_bounds__(256) void k_adj_gather(DS S, AD A)
     const int npv = S.npv;
     const long r = gl - B.g0;
     const int i = (int)(r % B.nx) - 1, j = (int)((r / B.nx) % B.ny) - 1, k = (int)(r / ((long)B.nx * B.ny)) - 1;
-    double acc[NPV], dcb[ND];
-    for (int n = 0; n < NPV; n++) acc[n] = 0.0;
-    for (int m = 0; m < ND; m++) dcb[m] = 0.0;
-    const int c3[3] = {i, j, k};
+    const bool visc = P.iturb >= -2, turb = P.iturb == 0, first = P.nmuscl == 0, sensor = P.nscheme == 2 || P.nscheme == 3;
+    double rho = 0.0, h = 0.0, c2 = 0.0, ht = 0.0, mu = 0.0, kap = 0.0;
     for (int D = 0; D < 3; D++) {
-        const int E = (D + 1) % 3, T = (D + 2) % 3;
         const long NF = S.NF[D];
-        for (int ll = 1; ll <= NSLOT; ll++) {
-            if (!((A.mask >> (ll - 1)) & 1ull)) continue;
-            int dn, de, dt;
-            stencil_ijk(ll, dn, de, dt);
-            int f[3];
-            f[D] = c3[D] - dn; f[E] = c3[E] - de; f[T] = c3[T] - dt;
-            if (!face_exists(B, D, f[0], f[1], f[2])) continue;
-            const long fi = fidx(B, D, f[0], f[1], f[2]);
-            for (int n = 0; n < npv; n++) acc[n] += A.fb[D][((long)(ll - 1) * npv + n) * NF + fi];
+        for (int sd = 0; sd < 2; sd++) {       // the face whose left (right) cell this is
+            const int fi = i - (sd && D == 0), fj = j - (sd && D == 1), fk = k - (sd && D == 2);
+            if (!face_exists(B, D, fi, fj, fk)) continue;
+            const long f = fidx(B, D, fi, fj, fk);
+            if (first) {
+                rho += A.fp[D][(long)(3 * sd) * NF + f];
+                h += A.fp[D][(long)(3 * sd + 1) * NF + f];
+                if (sensor) c2 += A.fp[D][(long)(3 * sd + 2) * NF + f];
+            }
+            if (visc) {
+                mu += A.vp[D][f];
+                kap += A.vp[D][NF + f];
+                if (turb) {
+                    rho += A.vp[D][2 * NF + f];
+                    ht += A.vp[D][(3 + sd) * NF + f];
+                }
+            }
         }
-        if (face_exists(B, D, i, j, k)) {
-            const long fi = fidx(B, D, i, j, k);
-            for (int m = 0; m < ND; m++) dcb[m] += A.db[D][(long)m * NF + fi];
+    }
+    double acc[NPV];
+    for (int n = 0; n < NPV; n++) acc[n] = 0.0;
+    {
+        for (int q = 0; q < 7; q++) {
+            int di, dj, dk;
+            src_off(q, di, dj, dk);
+            const int si = i - di, sj = j - dj, sk = k - dk;
+            if (!interior_cell(B, si, sj, sk)) continue;
+            const long ct = cidx(B, si, sj, sk);
+            for (int n = 0; n < NPV; n++) if (n < npv) acc[n] += A.cb[((long)q * npv + n) * S.NC + ct];
         }
-        const int im = i - (D == 0), jm = j - (D == 1), km = k - (D == 2);
-        if (face_exists(B, D, im, jm, km)) {
-            const long fi = fidx(B, D, im, jm, km);
-            for (int m = 0; m < ND; m++) dcb[m] += A.db[D][(long)(ND + m) * NF + fi];
+        if (interior_cell(B, i, j, k)) {
+            const long ct = cidx(B, i, j, k);
+            rho += A.cdb[ct];
+            h += A.cdb[S.NC + ct];
+            mu += A.cdb[2 * S.NC + ct];
         }
     }
-    for (int q = 0; q < 7; q++) {
-        int di, dj, dk;
-        src_off(q, di, dj, dk);
-        const int si = i - di, sj = j - dj, sk = k - dk;
-        if (!interior_cell(B, si, sj, sk)) continue;
-        const long ct = cidx(B, si, sj, sk);
-        for (int n = 0; n < npv; n++) acc[n] += A.cb[((long)q * npv + n) * S.NC + ct];
+    if (rho != 0.0 || h != 0.0 || c2 != 0.0 || ht != 0.0 || mu != 0.0 || kap != 0.0) {
+        double dcb[ND], gx[4];
+        for (int m = 0; m < ND; m++) dcb[m] = 0.0;
+        dcb[D_RHO] = rho; dcb[D_H] = h; dcb[D_C2] = c2; dcb[D_HT] = ht; dcb[D_MU] = mu; dcb[D_KAP] = kap;
+        const double x4[4] = {S.pv[gl] + P.pref, S.pv[4 * S.NG + gl], S.pv[5 * S.NG + gl], S.pv[6 * S.NG + gl]};
+        eos_adj(P.iturb != -3, x4, dcb, gx);
+        acc[0] += gx[0]; acc[4] += gx[1]; acc[5] += gx[2]; acc[6] += gx[3];
     }
-    if (interior_cell(B, i, j, k)) {
-        const long ct = cidx(B, i, j, k);
-        for (int m = 0; m < ND; m++) dcb[m] += A.cdb[(long)m * S.NC + ct];
-    }
-    for (int n = 0; n < npv; n++) A.pb[(long)n * S.NG + gl] = acc[n];
-    for (int m = 0; m < ND; m++) A.gdb[(long)m * S.NG + gl] = dcb[m];
-}
-
-// the gathered property bars of a ghosted cell back to (p, T, y1, y2),
-// added to the pv_bar k_adj_gather left
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adj_eos(DS S, AD A)
-{
-    long gl = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gl >= S.NG) return;
-    const Par &P = S.P;
-    double dcb[ND];
-    bool any = false;
-    for (int m = 0; m < ND; m++) {
-        dcb[m] = A.gdb[(long)m * S.NG + gl];
-        any = any || dcb[m] != 0.0;
-    }
-    if (!any) return;
-    double x4[4] = {S.pv[gl] + P.pref, S.pv[4 * S.NG + gl], S.pv[5 * S.NG + gl], S.pv[6 * S.NG + gl]}, gx[4];
-    eos_adj(P.iturb != -3, x4, dcb, gx);
-    A.pb[gl] += gx[0];
-    A.pb[4 * S.NG + gl] += gx[1];
-    A.pb[5 * S.NG + gl] += gx[2];
-    A.pb[6 * S.NG + gl] += gx[3];
+    for (int n = 0; n < NPV; n++) if (n < npv) A.pb[(long)n * S.NG + gl] += acc[n];
 }
 
 // deterministic sum of n doubles in two stages: workgroup b sums its strided
@@ -568,34 +657,39 @@ __global__ __launch_bounds__(256) void k_dotdiff_fixed(const double *w, const do
     if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
-// stencil points a face's bars cover under the configuration
-unsigned long long adj_mask(const Par &P)
-{
-    unsigned long long m = 0;
-    auto set = [&](int ll) { m |= 1ull << (ll - 1); };
-    set(9); set(10);
-    if (P.nmuscl == 1) { set(23); set(32); set(37); set(38); }
-    if (P.nmuscl == 2) for (int ll = 1; ll <= NSLOT; ll++) set(ll);
-    if (P.nscheme == 2 || P.nscheme == 3 || P.iturb >= -2) for (int ll = 1; ll <= 18; ll++) set(ll);
-    return m;
-}
-
 int adj_alloc(cav3d_ctx *c)
 {
     if (c->adj_ready) return 0;
     DS &S = c->S;
     const int npv = c->npv;
+    const bool visc = S.P.iturb >= -2, turb = S.P.iturb == 0;
     int rc;
     if ((rc = dalloc(c, &c->a_rb, (long)npv * S.NC)) || (rc = dalloc(c, &c->a_cb, 7L * npv * S.NC)) ||
-        (rc = dalloc(c, &c->a_cdb, (long)ND * S.NC)) || (rc = dalloc(c, &c->a_csb, 3L * S.NC)) || (rc = dalloc(c, &c->a_pb, (long)npv * S.NG)) ||
-        (rc = dalloc(c, &c->a_gdb, (long)ND * S.NG)) || (rc = dalloc(c, &c->a_sum, 16 + 16L * SUM_WG)))
+        (rc = dalloc(c, &c->a_cdb, 3L * S.NC)) || (rc = dalloc(c, &c->a_csb, 3L * S.NC)) || (rc = dalloc(c, &c->a_pb, (long)npv * S.NG)) ||
+        (rc = dalloc(c, &c->a_sum, 16 + 16L * SUM_WG)))
         return rc;
     for (int d = 0; d < 3; d++)
-        if ((rc = dalloc(c, &c->a_fb[d], (long)NSLOT * npv * S.NF[d])) || (rc = dalloc(c, &c->a_db[d], 2L * ND * S.NF[d])) ||
-            (rc = dalloc(c, &c->a_rsb[d], 4L * npv * S.NF[d])) ||
+        if ((rc = dalloc(c, &c->a_w[d], 2L * npv * S.NF[d])) || (rc = dalloc(c, &c->a_cell[d], S.NF[d])) ||
+            (rc = dalloc(c, &c->a_fp[d], S.P.nmuscl == 0 ? 6L * S.NF[d] : 1L)) ||
+            (rc = dalloc(c, &c->a_vb[d], visc ? (turb ? 23L : 15L) * S.NF[d] : 1L)) ||
+            (rc = dalloc(c, &c->a_vp[d], visc ? 5L * S.NF[d] : 1L)) ||
             (rc = dalloc(c, &c->a_snb[d], (S.P.nscheme == 2 || S.P.nscheme == 3) ? 18L * S.NF[d] : 1L)) ||
-            (rc = dalloc(c, &c->a_ub[d], S.NF[d])) || (rc = dalloc(c, &c->a_mtb[d], 2L * S.NF[d])))
+            (rc = dalloc(c, &c->a_ub[d], S.NF[d])) || (rc = dalloc(c, &c->a_mtb[d], turb ? 2L * S.NF[d] : 1L)))
             return rc;
+    // tiles of the stencil pass over every block's ghosted cells
+    std::vector<int> tl;
+    for (int b = 0; b < c->nb; b++) {
+        const BlkD &B = c->blk[b];
+        for (int k = -1; k <= B.K + 3; k += AK)
+            for (int j = -1; j <= B.J + 3; j += AJ)
+                for (int i = -1; i <= B.I + 3; i += AI) {
+                    const int t4[4] = {b, i, j, k};
+                    tl.insert(tl.end(), t4, t4 + 4);
+                }
+    }
+    c->a_ntiles = (int)(tl.size() / 4);
+    if ((rc = dalloc(c, &c->a_tiles, tl.size()))) return rc;
+    HIPCHK(hipMemcpyAsync(c->a_tiles, tl.data(), tl.size() * sizeof(int), hipMemcpyHostToDevice, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
     c->adj_ready = true;
     return 0;
@@ -608,28 +702,25 @@ int launch_vjp(cav3d_ctx *c, int dmut = 0)
     A.rb = c->a_rb;
     A.dmut = dmut;
     for (int d = 0; d < 3; d++) {
-        A.fb[d] = c->a_fb[d]; A.db[d] = c->a_db[d]; A.ub[d] = c->a_ub[d]; A.mtb[d] = c->a_mtb[d];
-        A.rsb[d] = c->a_rsb[d]; A.snb[d] = c->a_snb[d];
+        A.w[d] = c->a_w[d]; A.cell[d] = c->a_cell[d]; A.snb[d] = c->a_snb[d]; A.fp[d] = c->a_fp[d];
+        A.vb[d] = c->a_vb[d]; A.vp[d] = c->a_vp[d]; A.ub[d] = c->a_ub[d]; A.mtb[d] = c->a_mtb[d];
     }
-    A.cb = c->a_cb; A.cdb = c->a_cdb; A.csb = c->a_csb; A.pb = c->a_pb; A.gdb = c->a_gdb;
-    A.mask = adj_mask(S.P);
+    A.cb = c->a_cb; A.cdb = c->a_cdb; A.csb = c->a_csb; A.pb = c->a_pb;
+    A.tiles = c->a_tiles; A.ntiles = c->a_ntiles;
     const bool sensor = S.P.nscheme == 2 || S.P.nscheme == 3;
     const int npv = S.npv;
-    // the three directions write their own face bars: i on st, j and k on
-    // the side streams, joined before the cell sources and the gather
+    // the faces' kernels are independent of each other: i on st, j and k on
+    // the side streams, joined before the stencil pass and the cell sources
+    // (which read every direction's eddy-viscosity bars); those two run
+    // beside each other and are joined before the cells' pass
     hipStream_t sd[3] = {c->st, c->side[0], c->side[1]};
     hipEventRecord(c->fork, c->st);
     hipStreamWaitEvent(c->side[0], c->fork, 0);
     hipStreamWaitEvent(c->side[1], c->fork, 0);
 #define CAV3D_VJP_DIR(D)                                                                                             \
     do {                                                                                                             \
-        if (sensor) {                                                                                                \
-            hipLaunchKernelGGL((k_face_vjp<D, true>), dim3(nblk(S.NF[D], 128)), dim3(128), 0, sd[D], S, A);          \
-            hipLaunchKernelGGL((k_face_rvjp<D, true>), dim3(nblk(npv * S.NF[D], 256)), dim3(256), 0, sd[D], S, A);   \
-        } else {                                                                                                     \
-            hipLaunchKernelGGL((k_face_vjp<D, false>), dim3(nblk(S.NF[D], 128)), dim3(128), 0, sd[D], S, A);         \
-            hipLaunchKernelGGL((k_face_rvjp<D, false>), dim3(nblk(npv * S.NF[D], 256)), dim3(256), 0, sd[D], S, A);  \
-        }                                                                                                            \
+        if (sensor) hipLaunchKernelGGL((k_face_vjp<D, true>), dim3(nblk(S.NF[D], 128)), dim3(128), 0, sd[D], S, A);  \
+        else hipLaunchKernelGGL((k_face_vjp<D, false>), dim3(nblk(S.NF[D], 128)), dim3(128), 0, sd[D], S, A);        \
         if (S.P.iturb >= -2) hipLaunchKernelGGL((k_vface_vjp<D>), dim3(nblk(S.NF[D], 128)), dim3(128), 0, sd[D], S, A); \
     } while (0)
     CAV3D_VJP_DIR(1);
@@ -640,11 +731,17 @@ int launch_vjp(cav3d_ctx *c, int dmut = 0)
     hipEventRecord(c->join[1], c->side[1]);
     hipStreamWaitEvent(c->st, c->join[0], 0);
     hipStreamWaitEvent(c->st, c->join[1], 0);
-    // the cell sources read every direction's eddy-viscosity bars
-    if (S.P.ides > 0 || S.P.ncav >= 2) hipLaunchKernelGGL(k_cell_vjp<true>, dim3(nblk(S.NC, 128)), dim3(128), 0, c->st, S, A);
-    else hipLaunchKernelGGL(k_cell_vjp<false>, dim3(nblk(S.NC, 128)), dim3(128), 0, c->st, S, A);
-    hipLaunchKernelGGL(k_adj_gather, dim3(nblk(S.NG, 256)), dim3(256), 0, c->st, S, A);
-    hipLaunchKernelGGL(k_adj_eos, dim3(nblk(S.NG, 128)), dim3(128), 0, c->st, S, A);
+    hipEventRecord(c->fork, c->st);
+    hipStreamWaitEvent(c->side[0], c->fork, 0);
+    if (S.P.ides > 0 || S.P.ncav >= 2) hipLaunchKernelGGL(k_cell_vjp<true>, dim3(nblk(S.NC, 128)), dim3(128), 0, c->side[0], S, A);
+    else hipLaunchKernelGGL(k_cell_vjp<false>, dim3(nblk(S.NC, 128)), dim3(128), 0, c->side[0], S, A);
+    const dim3 tg((unsigned)(npv * c->a_ntiles));
+    if (S.P.nmuscl == 0) hipLaunchKernelGGL(k_adj_stencil<0>, tg, dim3(64), 0, c->st, S, A);
+    else if (S.P.nmuscl == 1) hipLaunchKernelGGL(k_adj_stencil<1>, tg, dim3(64), 0, c->st, S, A);
+    else hipLaunchKernelGGL(k_adj_stencil<2>, tg, dim3(64), 0, c->st, S, A);
+    hipEventRecord(c->join[0], c->side[0]);
+    hipStreamWaitEvent(c->st, c->join[0], 0);
+    hipLaunchKernelGGL(k_adj_cells, dim3(nblk(S.NG, 128)), dim3(128), 0, c->st, S, A);
     return 0;
 }
 
