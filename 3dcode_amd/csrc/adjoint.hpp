@@ -797,19 +797,20 @@ static int rhs_vjp_run(cav3d_ctx *c, const double *res_bar, double *pv_bar, doub
         c->prof_ms[8] = ms;
     }
     if ((rc = check_launch(name))) return rc;
+    if (scal_bar) {
+        const double *src[5] = {c->a_pb, c->a_ub[0], c->a_ub[1], c->a_ub[2], c->a_csb};
+        const long len[5] = {S.NG, S.NF[0], S.NF[1], S.NF[2], S.NC};
+        for (int q = 0; q < 5; q++) sum_into(c, src[q], len[q], q);
+    }
     off = 0;
     for (int b = 0; b < c->nb; b++) {
         const BlkD &B = c->blk[b];
         hipLaunchKernelGGL(k_soa_to_aos, dim3(nblk(B.ng, 256)), dim3(256), 0, c->st, (const double *)c->a_pb, npv, S.NG, B.g0,
                            c->stage, B.ng);
-        HIPCHK(hipMemcpyAsync(pv_bar + off, c->stage, (long)npv * B.ng * sizeof(double), hipMemcpyDeviceToHost, c->st));
-        HIPCHK(hipStreamSynchronize(c->st));
+        if ((rc = copy_out(c, pv_bar + off, c->stage, (long)npv * B.ng * sizeof(double)))) return rc;
         off += (long)npv * B.ng;
     }
     if (scal_bar) {
-        const double *src[5] = {c->a_pb, c->a_ub[0], c->a_ub[1], c->a_ub[2], c->a_csb};
-        const long len[5] = {S.NG, S.NF[0], S.NF[1], S.NF[2], S.NC};
-        for (int q = 0; q < 5; q++) sum_into(c, src[q], len[q], q);
         double h[5];
         HIPCHK(hipMemcpyAsync(h, c->a_sum, sizeof(h), hipMemcpyDeviceToHost, c->st));
         HIPCHK(hipStreamSynchronize(c->st));
@@ -966,8 +967,7 @@ int cav3d_objective(cav3d_ctx *c, double w_vap, double w_fx, double *J, double *
             const BlkD &B = c->blk[b];
             hipLaunchKernelGGL(k_soa_to_aos, dim3(nblk(B.ng, 256)), dim3(256), 0, c->st, (const double *)c->a_pb, npv, S.NG,
                                B.g0, c->stage, B.ng);
-            HIPCHK(hipMemcpyAsync(pv_bar + o, c->stage, (long)npv * B.ng * sizeof(double), hipMemcpyDeviceToHost, c->st));
-            HIPCHK(hipStreamSynchronize(c->st));
+            if ((rc = copy_out(c, pv_bar + o, c->stage, (long)npv * B.ng * sizeof(double)))) return rc;
             o += (long)npv * B.ng;
         }
     }

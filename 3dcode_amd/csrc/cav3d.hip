@@ -24,9 +24,11 @@
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -1657,6 +1659,8 @@ struct cav3d_ctx {
     int dev = 0;              // device current at creation (the context's device)
     double *stage = nullptr;
     size_t stage_n = 0;
+    char *pin = nullptr;      // pinned staging of large results (copy_out), OUT_BUFS chunks
+    hipEvent_t pin_ev[8] = {};
     int nwg_update = 0;
     int sweep_blocks = 0;     // grid of the sweep kernels: as many workgroups as fit the device at once
     int *tiles = nullptr;     // tile table of the sweeps (device): block, j0, k0, diagonal
@@ -1708,6 +1712,69 @@ int ensure_stage(cav3d_ctx *c, size_t n)
     if (c->stage) { HIPCHK(hipStreamSynchronize(c->st)); HIPCHK(hipFree(c->stage)); c->stage = nullptr; }
     HIPCHK(hipMalloc((void **)&c->stage, n * sizeof(double)));
     c->stage_n = n;
+    return 0;
+}
+
+// Large device results to the caller's memory.  The copy of pageable memory
+// inside the runtime is a serial chain of a transfer to its staging buffer
+// and one thread's memcpy from it (20 and 70 us per chunk), the memcpy paying
+// the page faults of a fresh array as well.  Here OUT_THREADS threads each own
+// OUT_BUFS / OUT_THREADS pinned chunks of the context: a thread copies one out
+// while its next is being filled.  128x64x64: the state (47 MB) 2.75 -> 1.59
+// ms, the residual and its Jacobians (75 MB into fresh arrays, with the 0.9 ms
+// of the kernels) 8.6 -> 4.3 ms.
+// Below OUT_MIN the plain copy is the faster one (the threads cost some 50 us).
+constexpr int OUT_BUFS = 8, OUT_THREADS = 4;
+constexpr size_t OUT_CHUNK = 1u << 20, OUT_MIN = 4 * OUT_CHUNK;
+int copy_out(cav3d_ctx *c, void *dst, const void *src, size_t bytes)
+{
+    if (bytes >= OUT_MIN && !c->pin) {
+        bool ok = hipHostMalloc((void **)&c->pin, OUT_BUFS * OUT_CHUNK, hipHostMallocDefault) == hipSuccess;
+        for (int q = 0; ok && q < OUT_BUFS; q++) ok = hipEventCreateWithFlags(&c->pin_ev[q], hipEventDisableTiming) == hipSuccess;
+        if (!ok) {
+            (void)hipGetLastError();
+            if (c->pin) (void)hipHostFree(c->pin);
+            c->pin = nullptr;
+        }
+    }
+    if (bytes < OUT_MIN || !c->pin) {
+        HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->st));
+        HIPCHK(hipStreamSynchronize(c->st));
+        return 0;
+    }
+    const long n = (long)((bytes + OUT_CHUNK - 1) / OUT_CHUNK);
+    std::atomic<int> err{0};
+    auto size = [&](long q) { return std::min(OUT_CHUNK, bytes - (size_t)q * OUT_CHUNK); };
+    auto fill = [&](long q) {        // chunk q into its buffer
+        const int b = (int)(q % OUT_BUFS);
+        hipError_t e = hipMemcpyAsync(c->pin + b * OUT_CHUNK, (const char *)src + q * OUT_CHUNK, size(q), hipMemcpyDeviceToHost, c->st);
+        if (e == hipSuccess) e = hipEventRecord(c->pin_ev[b], c->st);
+        if (e != hipSuccess) err = (int)e;
+    };
+    for (long q = 0; q < std::min<long>(n, OUT_BUFS); q++) fill(q);
+    auto work = [&](int t) {         // chunks t, t + OUT_THREADS, ...
+        hipSetDevice(c->dev);
+        for (long q = t; q < n && !err; q += OUT_THREADS) {
+            const int b = (int)(q % OUT_BUFS);
+            const hipError_t e = hipEventSynchronize(c->pin_ev[b]);
+            if (e != hipSuccess) { err = (int)e; break; }
+            memcpy((char *)dst + q * OUT_CHUNK, c->pin + b * OUT_CHUNK, size(q));
+            if (q + OUT_BUFS < n) fill(q + OUT_BUFS);
+        }
+    };
+    std::thread th[OUT_THREADS - 1];
+    int started = 0;
+    try {
+        for (; started < OUT_THREADS - 1; started++) th[started] = std::thread(work, started + 1);
+    } catch (const std::system_error &) {
+    }
+    work(0);
+    for (int t = started + 1; t < OUT_THREADS; t++) work(t);      // the threads that could not be started
+    for (int t = 0; t < started; t++) th[t].join();
+    if (err) {
+        (void)hipStreamSynchronize(c->st);
+        return fail(std::string("copy to the host: ") + hipGetErrorString((hipError_t)err.load()), -3);
+    }
     return 0;
 }
 
@@ -2151,9 +2218,10 @@ int cav3d_create(const cav3d_params *prm, int nblocks, const cav3d_block *blocks
         std::vector<int> tab;
         for (auto &t : tl) tab.insert(tab.end(), t.begin(), t.end());
         c->ntiles = (int)tl.size();
-        if ((rc = dalloc(c, &c->tiles, tab.size())) || (rc = dalloc(c, &c->sweep_err, 1)) || (rc = dalloc(c, &c->ticket, 2))) {
+        if ((rc = dalloc(c, &c->tiles, tab.size())) || (rc = dalloc(c, &c->sweep_err, 3))) {
             cav3d_destroy(c); return rc;
         }
+        c->ticket = c->sweep_err + 1;
         if (hipMemcpyAsync(c->tiles, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice, c->st) != hipSuccess) {
             cav3d_destroy(c); return fail("tile table upload failed", -3);
         }
@@ -2193,6 +2261,8 @@ void cav3d_destroy(cav3d_ctx *c)
     if (c->st) hipStreamSynchronize(c->st);
     for (void *p : c->allocs) hipFree(p);
     if (c->stage) hipFree(c->stage);
+    if (c->pin) hipHostFree(c->pin);
+    for (hipEvent_t e : c->pin_ev) if (e) hipEventDestroy(e);
     if (c->xbuf) hipFree(c->xbuf);
     if (c->a_obj) hipFree(c->a_obj);
     for (int q = 0; q < 14; q++) if (c->ev[q]) hipEventDestroy(c->ev[q]);
@@ -2280,15 +2350,14 @@ int cav3d_get_state(cav3d_ctx *c, int b, double *pv, double *dv, double *tv, dou
     if ((rc = ensure_stage(c, (long)(18 + 3) * B.ng + 2L * c->npv * B.nc))) return rc;
     if (pv) {
         hipLaunchKernelGGL(k_soa_to_aos, dim3(nblk(B.ng, 256)), dim3(256), 0, c->st, (const double *)S.pv, c->npv, S.NG, B.g0, c->stage, B.ng);
-        HIPCHK(hipMemcpyAsync(pv, c->stage, (long)c->npv * B.ng * sizeof(double), hipMemcpyDeviceToHost, c->st));
-        HIPCHK(hipStreamSynchronize(c->st));
+        if ((rc = copy_out(c, pv, c->stage, (long)c->npv * B.ng * sizeof(double)))) return rc;
     }
     if (dv || tv) {
         // evaluate the EOS over this block's ghosted cells into AoS staging
         double *dvd = c->stage, *tvd = c->stage + 18L * B.ng;
         hipLaunchKernelGGL(k_eos_full, dim3(nblk(B.ng, 128)), dim3(128), 0, c->st, S, B.g0, B.ng, dvd, tvd);
         HIPCHK(hipStreamSynchronize(c->st));
-        if (dv) HIPCHK(hipMemcpy(dv, dvd, 18L * B.ng * sizeof(double), hipMemcpyDeviceToHost));
+        if (dv && (rc = copy_out(c, dv, dvd, 18L * B.ng * sizeof(double)))) return rc;
         if (tv && c->ntv) {
             std::vector<double> t2(2 * B.ng), mt;
             HIPCHK(hipMemcpy(t2.data(), tvd, 2L * B.ng * sizeof(double), hipMemcpyDeviceToHost));
@@ -2305,8 +2374,7 @@ int cav3d_get_state(cav3d_ctx *c, int b, double *pv, double *dv, double *tv, dou
     }
     if (qq && c->prm.nsteady > 0) {
         hipLaunchKernelGGL(k_cell_to_aos, dim3(nblk(B.nc, 256)), dim3(256), 0, c->st, (const double *)S.qq, 2 * c->npv, S.NC, B.c0, c->stage, B.nc);
-        HIPCHK(hipMemcpyAsync(qq, c->stage, 2L * c->npv * B.nc * sizeof(double), hipMemcpyDeviceToHost, c->st));
-        HIPCHK(hipStreamSynchronize(c->st));
+        if ((rc = copy_out(c, qq, c->stage, 2L * c->npv * B.nc * sizeof(double)))) return rc;
     }
     return check_launch("cav3d_get_state");
 }
@@ -2351,8 +2419,7 @@ int cav3d_calrhs(cav3d_ctx *c, double time, int b, double *res, double *icav, do
         if (!o.h) continue;
         if (!o.d) { memset(o.h, 0, sizeof(double) * o.m * B.nc); continue; }
         hipLaunchKernelGGL(k_cell_to_aos, dim3(nblk(B.nc, 256)), dim3(256), 0, c->st, o.d, o.m, S.NC, B.c0, c->stage, B.nc);
-        HIPCHK(hipMemcpyAsync(o.h, c->stage, (long)o.m * B.nc * sizeof(double), hipMemcpyDeviceToHost, c->st));
-        HIPCHK(hipStreamSynchronize(c->st));
+        if ((rc = copy_out(c, o.h, c->stage, (long)o.m * B.nc * sizeof(double)))) return rc;
     }
     HIPCHK(hipStreamSynchronize(c->st));
     return check_launch("cav3d_calrhs");
@@ -2449,9 +2516,7 @@ int cav3d_eos(cav3d_ctx *c, int n, const double *p, const double *t, const doubl
     HIPCHK(hipMemcpyAsync(d + 3L * n, y2, n * 8, hipMemcpyHostToDevice, c->st));
     hipLaunchKernelGGL(k_eos_points, dim3(nblk(n, 128)), dim3(128), 0, c->st, c->P, n, (const double *)d, (const double *)(d + n),
                        (const double *)(d + 2L * n), (const double *)(d + 3L * n), d + 4L * n, d + 22L * n);
-    HIPCHK(hipMemcpyAsync(dv, d + 4L * n, 18L * n * 8, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipMemcpyAsync(tv, d + 22L * n, 2L * n * 8, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
+    if ((rc = copy_out(c, dv, d + 4L * n, 18L * n * 8)) || (rc = copy_out(c, tv, d + 22L * n, 2L * n * 8))) return rc;
     return check_launch("cav3d_eos");
 }
 

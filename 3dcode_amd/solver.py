@@ -109,6 +109,12 @@ def _p(a, t=C.c_double):
     return a.ctypes.data_as(C.POINTER(t))
 
 
+def _joined(arrays):
+    """The arrays as one flat float64 array; a single one is not copied."""
+    flat = [np.ascontiguousarray(a, dtype=np.float64).ravel() for a in arrays]
+    return flat[0] if len(flat) == 1 else np.concatenate(flat)
+
+
 def _check(rc: int):
     if rc != 0:
         msg = lib().cav3d_last_error().decode()
@@ -297,7 +303,7 @@ class Solver:
         per-block pv_bar arrays (pv layout, ghosted) and [d/d p_ref, d/d u_ref]
         of res_bar . res."""
         blocks = self.case.blocks
-        rb = np.ascontiguousarray(np.concatenate([np.asarray(r, dtype=np.float64).ravel() for r in res_bars]))
+        rb = _joined(res_bars)
         nc = [self.npv * (b.imax - 1) * (b.jmax - 1) * (b.kmax - 1) for b in blocks]
         if rb.size != sum(nc):
             raise ValueError(f"res_bar: expected {sum(nc)} values, got {rb.size}")
@@ -314,7 +320,7 @@ class Solver:
         cases.PARAM_KEYS: p_ref, u_ref, dp_ref, t_ref, bc_pv[0..8],
         bc_pressure.  The current ghost layers must be the boundary fill of
         the interior (call setbc first)."""
-        rb = np.ascontiguousarray(np.concatenate([np.asarray(r, dtype=np.float64).ravel() for r in res_bars]))
+        rb = _joined(res_bars)
         out = np.zeros(14)
         _check(lib().cav3d_rhs_vjp_params(self.h, _p(rb), _p(out)))
         return out
