@@ -433,16 +433,8 @@ template <bool MLP, class F> HD ReconBar muscl_back(int nlim, F xs, double wl, d
         dyr = (xs(12) - xs(8)) / nr;
         dzr = (xs(16) - xs(4)) / nr;
         const double ryl = fabs(dyl), rzl = fabs(dzl), ryr = fabs(dyr), rzr = fabs(dzr);
-        double ao = xs(1), bo = ao, ae = xs(2), be = ae, aL = xs(19), bL = aL, aR = xs(28), bR = aR;
-#pragma unroll
-        for (int q = 3; q <= 17; q += 2) { ao = mn(ao, xs(q)); bo = mx(bo, xs(q)); }
-#pragma unroll
-        for (int q = 4; q <= 18; q += 2) { ae = mn(ae, xs(q)); be = mx(be, xs(q)); }
-#pragma unroll
-        for (int q = 20; q <= 27; q++) { aL = mn(aL, xs(q)); bL = mx(bL, xs(q)); }
-#pragma unroll
-        for (int q = 29; q <= 36; q++) { aR = mn(aR, xs(q)); bR = mx(bR, xs(q)); }
-        const double a18 = mn(ao, ae), b18 = mx(bo, be);
+        const MlpExt<double> e = mlp_extrema<double>(xs);
+        const double a18 = e.a18, b18 = e.b18, aL = e.aL, bL = e.bL, aR = e.aR, bR = e.bR, ao = e.ao, bo = e.bo, ae = e.ae, be = e.be;
         double lo, hi;
         int glo, ghi;
         auto lower = [&](double p, int gp, double q, int gq) { lo = mn(p, q); glo = q < p ? gq : gp; };

@@ -26,6 +26,14 @@ void ac_recon(int nlim, int mlp, const double *x, double wl, double wr, double *
     }
 }
 
+// the ten extrema of the MLP stencil
+void ac_extrema(const double *x, double *o)
+{
+    const MlpExt<double> m = mlp_extrema<double>([&](int ll) -> double { return x[ll - 1]; });
+    const double v[10] = {m.ao, m.bo, m.ae, m.be, m.a18, m.b18, m.aL, m.bL, m.aR, m.bR};
+    for (int q = 0; q < 10; q++) o[q] = v[q];
+}
+
 // flux core of scheme 1 (Roe) or 4 (AUSM+-up): z = {pL[9], pR[9], rhoL, hL, rhoR, hR, c2, u_ref}
 void ac_flux(int scheme, int prec, int npv, double pref, double str, const double *n3, const double *z, const double *g,
              double *rev, double *dual)

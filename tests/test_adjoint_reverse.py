@@ -56,6 +56,25 @@ def test_reconstruction(L, nlim, mlp):
         assert hit > 0
 
 
+@pytest.mark.parametrize("bad", [0] + list(range(1, 37)))
+def test_mlp_extrema_keep_the_order_of_a_comparison_chain(L, bad):
+    """The extrema equal the chains (b < a) ? b : a over the points in order,
+    also where point `bad` is a NaN: a chain that starts at it stays there, any
+    other drops it."""
+    rng = np.random.default_rng(bad)
+    x, o = rng.standard_normal(38), np.zeros(10)
+    if bad:
+        x[bad - 1] = np.nan
+    L.ac_extrema(dp(x), dp(o))
+    chains = [range(1, 18, 2), range(2, 19, 2), range(1, 19), range(19, 28), range(28, 37)]
+    for c, ll in enumerate(chains):
+        lo = hi = x[ll[0] - 1]
+        for q in ll:
+            lo = x[q - 1] if x[q - 1] < lo else lo
+            hi = x[q - 1] if x[q - 1] > hi else hi
+        assert np.array_equal([lo, hi], o[2 * c:2 * c + 2], equal_nan=True), (bad, c)
+
+
 @pytest.mark.parametrize("npv", [7, 9])
 @pytest.mark.parametrize("prec", [0, 1, 2])
 @pytest.mark.parametrize("scheme", [1, 4])
