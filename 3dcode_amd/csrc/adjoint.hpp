@@ -20,8 +20,8 @@
 // wavefront per tile of cells and variable: it runs every face whose stencil
 // reaches its cells, in a fixed order, and adds what falls on them in LDS, so
 // no bars of stencil points are written to memory and the result is
-// deterministic.  The cell sources are differentiated per cell (two-lane dual
-// passes), and each cell's property bars return to (p, T, y1, y2) through its
+// deterministic.  The cell sources are differentiated per cell (dual passes over
+// the few numbers each source reads), and each cell's property bars return to (p, T, y1, y2) through its
 // EOS.  Arithmetic is FP64 throughout.
 //
 // d/d(p_ref) is the sum of pv_bar over the pressure component: the residual
@@ -45,7 +45,8 @@ struct AD {
     double *vb[3];          // a face's viscous bars [3 nv + ncv][NF]: differences, averages
     double *vp[3];          // and of its cells' properties [5][NF]: mu, kappa, rho (each side), h_T left, right
     double *ub[3];          // d(phi_f)/d(u_ref) [NF]
-    double *cb;             // cell-source bars on the 7-point stencil [7][npv][NC]
+    double *cb;             // cell-source bars [npv (+ 15)][NC]: of the cell's state, and under SST of its
+                            // gradients of u, v, w, k, omega (half of them, over the volume)
     double *cdb;            // cell-source property bars [3][NC]: rho, h, mu
     double *csb;            // cell-source d(phi_c)/d(u_ref, dp_ref, t_ref) [3][NC] (the mass-transfer scales)
     double *pb;             // pv_bar [npv][NG]
@@ -247,11 +248,15 @@ __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, const 
     if (cnt[0] <= 0 || cnt[1] <= 0 || cnt[2] <= 0) return;
     const int total = cnt[0] * cnt[1] * cnt[2];
     constexpr int st[3] = {1, AI, AI * AJ};
+    // q / cnt of small numbers through the reciprocal: (q + 0.5) / cnt is at
+    // least 0.5 / cnt away from every whole number, far more than it is rounded by
+    const float i0 = 1.0f / (float)cnt[0], i1 = 1.0f / (float)cnt[1];
     for (int base = 0; base < total; base += 64) {
         const int r = base + lane;
         const bool on = r < total;
         const int q = on ? r : 0;
-        const int f[3] = {lo[0] + q % cnt[0], lo[1] + (q / cnt[0]) % cnt[1], lo[2] + q / (cnt[0] * cnt[1])};
+        const int q1 = (int)(((float)q + 0.5f) * i0), q2 = (int)(((float)q1 + 0.5f) * i1);
+        const int f[3] = {lo[0] + q - q1 * cnt[0], lo[1] + q1 - q2 * cnt[1], lo[2] + q2};
         const long t = fidx(B, D, f[0], f[1], f[2]);
         double wl = A.w[D][(long)n * NF + t], wr = A.w[D][(long)(npv + n) * NF + t];
         const int cell = A.cell[D][t];
@@ -294,6 +299,10 @@ __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, const 
         }
         b9 += o.x9;
         b10 += o.x10;
+        // the bar of the extremum a side's MLP bound selected, if that is point ll
+        auto exl = [&](int ll) -> double { return NM == 2 && o.il == ll ? o.el : 0.0; };
+        auto exr = [&](int ll) -> double { return NM == 2 && o.ir == ll ? o.er : 0.0; };
+        auto ex = [&](int ll) -> double { return exl(ll) + exr(ll); };
         if (vq >= 0 || sen) {
             // the 18 points of the viscous differences (and of the pressure sensor)
             double v0 = 0.0, v1 = 0.0, v2 = 0.0, vc = 0.0;
@@ -303,7 +312,7 @@ __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, const 
                 v2 = 0.0625 * A.vb[D][(long)(3 * vq + 2) * NF + t];
                 if (cq >= 0) vc = 0.5 * A.vb[D][(long)(3 * nv + cq) * NF + t];
             }
-            auto sn = [&](int ll) -> double { return sen ? sen[(long)(ll - 1) * NF + t] : 0.0; };
+            auto sn = [&](int ll) -> double { return (sen ? sen[(long)(ll - 1) * NF + t] : 0.0) + ex(ll); };
             add(1, -v1 - v2 + sn(1));
             add(2, -v1 - v2 + sn(2));
             add(3, o.x3 - 2.0 * v2 + sn(3));
@@ -323,36 +332,28 @@ __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, const 
             add(17, v1 + v2 + sn(17));
             add(18, v1 + v2 + sn(18));
         } else {
-            add(9, b9);
-            add(10, b10);
+            add(9, b9 + ex(9));
+            add(10, b10 + ex(10));
             if constexpr (NM == 2) {
-                add(3, o.x3); add(4, o.x4); add(7, o.x7); add(8, o.x8);
-                add(11, o.x11); add(12, o.x12); add(15, o.x15); add(16, o.x16);
+                add(3, o.x3 + ex(3)); add(4, o.x4 + ex(4)); add(7, o.x7 + ex(7)); add(8, o.x8 + ex(8));
+                add(11, o.x11 + ex(11)); add(12, o.x12 + ex(12)); add(15, o.x15 + ex(15)); add(16, o.x16 + ex(16));
+                auto corner = [&](int ll) { if (o.il == ll || o.ir == ll) add(ll, ex(ll)); };
+                corner(1); corner(2); corner(5); corner(6); corner(13); corner(14); corner(17); corner(18);
             }
         }
         if constexpr (NM > 0) {
-            add(23, o.x23);
-            add(32, o.x32);
+            add(23, o.x23 + exl(23));
+            add(32, o.x32 + exr(32));
             add(37, o.x37);
             add(38, o.x38);
         }
         if constexpr (NM == 2) {
-            // the extrema the bounds selected: lanes of one stencil point at a time
-            auto extremum = [&](int il, double v) {
-                unsigned long long todo = __ballot(on && il != 0);
-                while (todo) {
-                    const int ll = __builtin_amdgcn_readlane(il, __builtin_ctzll(todo));
-                    const bool mine = on && il == ll;
-                    todo &= ~__ballot(mine);
-                    int dn, de, dt;
-                    stencil_ijk(ll, dn, de, dt);
-                    if (mine && (unsigned)(l[D] + dn) <= (unsigned)w3[D] && (unsigned)(l[E] + de) <= (unsigned)w3[E] &&
-                        (unsigned)(l[T] + dt) <= (unsigned)w3[T])
-                        __hip_atomic_fetch_add(&acc[at + dn * st[D] + de * st[E] + dt * st[T]], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+#pragma unroll
+            for (int q = 0; q < 9; q++)
+                if (q != 4) {
+                    if (o.il == 19 + q) add(19 + q, o.el);
+                    if (o.ir == 28 + q) add(28 + q, o.er);
                 }
-            };
-            extremum(o.il, o.el);
-            extremum(o.ir, o.er);
         }
     }
 }
@@ -384,14 +385,6 @@ __global__ __launch_bounds__(64) void k_adj_stencil(DS S, AD A)
     }
 }
 
-// the 7-point stencil of the cell sources (x7 of k_combine)
-__device__ __forceinline__ void src_off(int q, int &di, int &dj, int &dk)
-{
-    di = q == 0 ? -1 : (q == 2 ? 1 : 0);
-    dj = q == 3 ? -1 : (q == 4 ? 1 : 0);
-    dk = q == 5 ? -1 : (q == 6 ? 1 : 0);
-}
-
 // Cell sources of one interior cell: the mass transfer, SST, BDF.  MODELS:
 // the instantiation with the Kunz / Singhal / Schnerr-Sauer / Lee sources
 // (a full EOS of the cell) and the DES length scales, as k_combine<true>.
@@ -406,155 +399,52 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     int i, j, k;
     cell_of(B, t - B.c0, i, j, k);
     const long g = gidx(B, i, j, k);
-    double rb[NPV];
-    for (int n = 0; n < NPV; n++) rb[n] = n < npv ? A.rb[(long)n * S.NC + t] : 0.0;
-    const bool sst = P.iturb == 0, cav_ = P.ncav >= 1, bdf = P.nsteady > 0;
-    // z = {pc[npv], rho, h, mu, the Green-Gauss gradients of u, v, w, k, omega (15),
-    //      the scalars the mass-transfer rates read: u_ref (Singhal), dp_ref
-    //      (Merkle, Kunz's evaporation), t_ref (Merkle, Kunz), [the eddy viscosity]}
-    constexpr int NZ = NPV + 3 + 15 + 3 + 1;
-    const int od = npv, og = npv + 3;
-    const int nz0 = (cav_ || bdf || sst) ? (sst ? og + 15 : og) : 0;
-    const bool sc = nz0 && (P.ncav == 1 || P.ncav == 2 || P.ncav == 3);
-    const int osc = nz0;                                   // u_ref, dp_ref, t_ref lanes
-    const bool dm = A.dmut && sst;                         // the eddy viscosity is a state function
-    const int omu = sc ? nz0 + 3 : nz0;                    // its lane
-    const int nz = omu + (dm ? 1 : 0);
-    double zx[NZ], zb[NZ];
-    for (int q = 0; q < NZ; q++) zx[q] = zb[q] = 0.0;
-    const int gvar[5] = {1, 2, 3, 7, 8};
-    double d[ND];
+    const bool sst = P.iturb == 0;
+    double rb[NPV], pc[NPV], d[ND], gr[5][3], f6[6][3], iv = 1.0;
+    for (int n = 0; n < NPV; n++) {
+        rb[n] = n < npv ? A.rb[(long)n * S.NC + t] : 0.0;
+        pc[n] = n < npv ? S.pv[(long)n * S.NG + g] : 0.0;
+    }
     for (int m = 0; m < ND; m++) d[m] = S.dc[m * S.NG + g];
-    double x7[7][NPV];
-    for (int q = 0; q < 7; q++) {
-        int di, dj, dk;
-        src_off(q, di, dj, dk);
-        const long gn = gidx(B, i + di, j + dj, k + dk);
-        for (int n = 0; n < NPV; n++) x7[q][n] = n < npv ? S.pv[(long)n * S.NG + gn] : 0.0;
-    }
-    const double vol = S.vol[widx(B, i, j, k)];
-    double f6[6][3];
-    cell_faces(S, B, i, j, k, f6);
-    const double iv = 1.0 / vol;
-    if (nz) {
-        for (int n = 0; n < npv; n++) zx[n] = x7[1][n];
-        zx[od] = d[D_RHO]; zx[od + 1] = d[D_H]; zx[od + 2] = d[D_MU];
-        if (sst)
-            for (int v = 0; v < 5; v++) gg_grad<double>(x7, gvar[v], f6, iv, zx + og + 3 * v);
-        if (sc) { zx[osc] = P.uref; zx[osc + 1] = P.dp_ref; zx[osc + 2] = P.t_ref; }
-        const double ydn = sst ? S.ydn[widx(B, i, j, k)] : 1.0;
-        const double mut = S.mut ? S.mut[g] : 0.0;
-        if (dm) zx[omu] = mut;
-        double q1[NPV], q2[NPV];
-        for (int n = 0; n < NPV; n++) {
-            q1[n] = (bdf && n < npv) ? S.qq[(long)n * S.NC + t] : 0.0;
-            q2[n] = (bdf && n < npv) ? S.qq[(long)(npv + n) * S.NC + t] : 0.0;
+    const double vol = S.vol[widx(B, i, j, k)], ydn = sst ? S.ydn[widx(B, i, j, k)] : 1.0;
+    const double mut = S.mut ? S.mut[g] : 0.0;
+    if (sst) {
+        cell_faces(S, B, i, j, k, f6);
+        iv = 1.0 / vol;
+        const long sy = B.nx, sz = (long)B.nx * B.ny;
+        for (int v = 0; v < 5; v++) {
+            const int n = v < 3 ? v + 1 : v + 4;
+            const double *x = S.pv + (long)n * S.NG + g;
+            double x7[7][NPV];
+            x7[0][0] = x[-1]; x7[1][0] = x[0]; x7[2][0] = x[1];
+            x7[3][0] = x[-sy]; x7[4][0] = x[sy]; x7[5][0] = x[-sz]; x7[6][0] = x[sz];
+            gg_grad<double>(x7, 0, f6, iv, gr[v]);
         }
-        constexpr int W = 2;
-        using T = Dn<W>;
-        dn_grad<W>(nz, [&](int q) -> double { return zx[q]; }, [&](auto in, int base) -> T {
-            Par Pu = P;
-            auto lane_of = [&](int q) { const int l = q - base; return (sc && l >= 0 && l < W) ? l + 1 : 0; };
-            Pu.uref_seed = lane_of(osc);
-            Pu.dpref_seed = lane_of(osc + 1);
-            Pu.tref_seed = lane_of(osc + 2);
-            T pc[NPV], dt[ND];
-            for (int n = 0; n < NPV; n++) pc[n] = n < npv ? in(n) : T(0.0);
-            for (int m = 0; m < ND; m++) dt[m] = T(d[m]);
-            dt[D_RHO] = in(od); dt[D_H] = in(od + 1); dt[D_MU] = in(od + 2);
-            T phi(0.0);
-            if (cav_) {
-                T rc, rv, ic[4];
-                if constexpr (MODELS) {
-                    if (P.ncav >= 2) {      // on the cell's full EOS, as k_combine<true>
-                        T dd[ND], full[18];
-                        mixture_eos<T>(pc[0] + P.pref, pc[4], pc[5], pc[6], dd, false, full);
-                        cav_model<T>(Pu, pc, full, vol, rc, rv, ic);
-                    } else {
-                        merkle<T>(Pu, pc, dt, vol, rc, rv, ic);
-                    }
-                } else {
-                    merkle<T>(Pu, pc, dt, vol, rc, rv, ic);
-                }
-                phi = phi + rb[5] * (rv - rc);
-            }
-            if (sst) {
-                T gr[5][3];
-                for (int v = 0; v < 5; v++)
-                    for (int c = 0; c < 3; c++) gr[v][c] = in(og + 3 * v + c);
-                T src[2], it[4], oc;
-                sst_source_g<MODELS, T>(P, gr[0], gr[1], gr[2], gr[3], gr[4], pc[7], pc[8], f6, vol, ydn, dt,
-                                     dm ? in(omu) : T(mut), src, it, oc);
-                phi = phi + rb[7] * src[0] + rb[8] * src[1];
-            }
-            if (bdf) {
-                T fx[NPV];
-                fx[0] = dt[D_RHO];
-                fx[1] = dt[D_RHO] * pc[1];
-                fx[2] = dt[D_RHO] * pc[2];
-                fx[3] = dt[D_RHO] * pc[3];
-                fx[4] = dt[D_RHO] * (dt[D_H] + 0.5 * (pc[1] * pc[1] + pc[2] * pc[2] + pc[3] * pc[3])) - (pc[0] + P.pref);
-                for (int n = 5; n < NPV; n++) fx[n] = n < npv ? dt[D_RHO] * pc[n] : T(0.0);
-                for (int n = 0; n < npv; n++) {
-                    T v = (double)P.nsteady * (P.bdf_b * fx[n] - q1[n]) + 0.5 * ((double)P.nsteady - 1.0) * q2[n];
-                    phi = phi - rb[n] * (v * vol / P.dt_phy);
-                }
-            }
-            return phi;
-        }, zb);
-        if (dm) {
-            // the cell's eddy-viscosity bar: its sources' share and its six
-            // viscous faces' (the left cell of its + faces, the right cell of
-            // its - faces), back to rho, mu, k, omega and the velocity
-            // gradients through mu_t = sst_eddy_g (src/eddy_module.f90:135-187)
-            double mb = zb[omu];
-            for (int D = 0; D < 3; D++) {
-                mb += A.mtb[D][fidx(B, D, i, j, k)];
-                mb += A.mtb[D][S.NF[D] + fidx(B, D, i - (D == 0), j - (D == 1), k - (D == 2))];
-            }
-            if (mb != 0.0) {
-                double ex[13], eb[13];
-                ex[0] = d[D_RHO]; ex[1] = d[D_MU]; ex[2] = x7[1][7]; ex[3] = x7[1][8];
-                for (int q = 0; q < 9; q++) ex[4 + q] = zx[og + q];
-                dn_grad<4>(13, [&](int q) -> double { return ex[q]; }, [&](auto in, int) -> Dn<4> {
-                    const Dn<4> gu[3] = {in(4), in(5), in(6)}, gv[3] = {in(7), in(8), in(9)}, gw[3] = {in(10), in(11), in(12)};
-                    return sst_eddy_g<Dn<4>>(in(0), in(1), in(2), in(3), gu, gv, gw, ydn);
-                }, eb);
-                zb[od] += mb * eb[0];
-                zb[od + 2] += mb * eb[1];
-                zb[7] += mb * eb[2];
-                zb[8] += mb * eb[3];
-                for (int q = 0; q < 9; q++) zb[og + q] += mb * eb[4 + q];
-            }
-        }
+    } else {
+        for (int v = 0; v < 5; v++) for (int c = 0; c < 3; c++) gr[v][c] = 0.0;
+        for (int q = 0; q < 6; q++) for (int c = 0; c < 3; c++) f6[q][c] = 0.0;
     }
-    // outputs: centre (q = 1) and neighbour bars, the cell's property bars;
-    // a gradient component g[c] = iv * sum_q w_q[c] x_q with the Green-Gauss
-    // weights w_q = -f6[0]/2, (face sum)/2, +f6[1]/2, -f6[2]/2, +f6[3]/2,
-    // -f6[4]/2, +f6[5]/2 for q = 0..6
-    double wq[7][3];
-    for (int c = 0; c < 3; c++) {
-        wq[0][c] = -0.5 * f6[0][c] * iv;
-        wq[2][c] = 0.5 * f6[1][c] * iv;
-        wq[3][c] = -0.5 * f6[2][c] * iv;
-        wq[4][c] = 0.5 * f6[3][c] * iv;
-        wq[5][c] = -0.5 * f6[4][c] * iv;
-        wq[6][c] = 0.5 * f6[5][c] * iv;
-        wq[1][c] = 0.5 * (f6[1][c] + f6[3][c] + f6[5][c] - f6[0][c] - f6[2][c] - f6[4][c]) * iv;
-    }
-    for (int q = 0; q < 7; q++)
-        for (int n = 0; n < npv; n++) {
-            double v = q == 1 ? zb[n] : 0.0;
-            if (sst)
-                for (int gv = 0; gv < 5; gv++)
-                    if (gvar[gv] == n)
-                        v += wq[q][0] * zb[og + 3 * gv] + wq[q][1] * zb[og + 3 * gv + 1] + wq[q][2] * zb[og + 3 * gv + 2];
-            A.cb[((long)q * npv + n) * S.NC + t] = v;
+    SourceBar o;
+    source_back<MODELS>(P, pc, d, gr, f6, vol, ydn, mut, rb, o);
+    if (A.dmut && sst) {
+        // the cell's eddy-viscosity bar: its sources' share and its six
+        // viscous faces' (the left cell of its + faces, the right cell of
+        // its - faces), the eddy viscosity being a state function
+        double mb = o.mut;
+        for (int D = 0; D < 3; D++) {
+            mb += A.mtb[D][fidx(B, D, i, j, k)];
+            mb += A.mtb[D][S.NF[D] + fidx(B, D, i - (D == 0), j - (D == 1), k - (D == 2))];
         }
-    A.cdb[t] = zb[od];
-    A.cdb[S.NC + t] = zb[od + 1];
-    A.cdb[2 * S.NC + t] = zb[od + 2];
-    for (int q = 0; q < 3; q++) A.csb[(long)q * S.NC + t] = sc ? zb[osc + q] : 0.0;
+        if (mb != 0.0) eddy_back(mb, pc, d, gr, ydn, o);
+    }
+    for (int n = 0; n < NPV; n++) if (n < npv) A.cb[(long)n * S.NC + t] = o.pc[n];
+    if (sst)
+        for (int v = 0; v < 5; v++)
+            for (int c = 0; c < 3; c++) A.cb[(long)(npv + 3 * v + c) * S.NC + t] = 0.5 * iv * o.g[v][c];
+    A.cdb[t] = o.rho;
+    A.cdb[S.NC + t] = o.h;
+    A.cdb[2 * S.NC + t] = o.mu;
+    for (int q = 0; q < 3; q++) A.csb[(long)q * S.NC + t] = o.sc[q];
 }
 
 // The rest of pv_bar of every ghosted cell, added to what k_adj_stencil left:
@@ -595,20 +485,40 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     double acc[NPV];
     for (int n = 0; n < NPV; n++) acc[n] = 0.0;
-    {
-        for (int q = 0; q < 7; q++) {
-            int di, dj, dk;
-            src_off(q, di, dj, dk);
-            const int si = i - di, sj = j - dj, sk = k - dk;
-            if (!interior_cell(B, si, sj, sk)) continue;
-            const long ct = cidx(B, si, sj, sk);
-            for (int n = 0; n < NPV; n++) if (n < npv) acc[n] += A.cb[((long)q * npv + n) * S.NC + ct];
+    const bool inside = interior_cell(B, i, j, k);
+    if (inside) {
+        const long ct = cidx(B, i, j, k);
+        for (int n = 0; n < NPV; n++) if (n < npv) acc[n] = A.cb[(long)n * S.NC + ct];
+        rho += A.cdb[ct];
+        h += A.cdb[S.NC + ct];
+        mu += A.cdb[2 * S.NC + ct];
+    }
+    if (turb) {
+        // the Green-Gauss gradients' transpose: a cell's gradient of x is
+        // the sum over its faces of the outward face vector times the mean
+        // of x on the two sides, over its volume (A.cb holds half the bar
+        // over the volume), so this cell's value meets the cell across each
+        // of its faces there, and its own gradient at all six
+        double own[3] = {0.0, 0.0, 0.0};
+        for (int q = 0; q < 6; q++) {
+            const int D = q >> 1, hi = q & 1, e = hi ? 1 : -1;
+            const int si = i + (D == 0 ? e : 0), sj = j + (D == 1 ? e : 0), sk = k + (D == 2 ? e : 0);
+            const bool nb = interior_cell(B, si, sj, sk);
+            if (!inside && !nb) continue;
+            double f[3];
+            face_vec(S, B, D, hi ? i : si, hi ? j : sj, hi ? k : sk, f);
+            for (int c = 0; c < 3; c++) own[c] += hi ? f[c] : -f[c];
+            if (!nb) continue;
+            const double *gb = A.cb + (long)npv * S.NC + cidx(B, si, sj, sk);
+            for (int v = 0; v < 5; v++) {
+                const double w = f[0] * gb[(3L * v) * S.NC] + f[1] * gb[(3L * v + 1) * S.NC] + f[2] * gb[(3L * v + 2) * S.NC];
+                acc[v < 3 ? v + 1 : v + 4] += hi ? -w : w;
+            }
         }
-        if (interior_cell(B, i, j, k)) {
-            const long ct = cidx(B, i, j, k);
-            rho += A.cdb[ct];
-            h += A.cdb[S.NC + ct];
-            mu += A.cdb[2 * S.NC + ct];
+        if (inside) {
+            const double *gb = A.cb + (long)npv * S.NC + cidx(B, i, j, k);
+            for (int v = 0; v < 5; v++)
+                acc[v < 3 ? v + 1 : v + 4] += own[0] * gb[(3L * v) * S.NC] + own[1] * gb[(3L * v + 1) * S.NC] + own[2] * gb[(3L * v + 2) * S.NC];
         }
     }
     if (rho != 0.0 || h != 0.0 || c2 != 0.0 || ht != 0.0 || mu != 0.0 || kap != 0.0) {
@@ -664,7 +574,7 @@ int adj_alloc(cav3d_ctx *c)
     const int npv = c->npv;
     const bool visc = S.P.iturb >= -2, turb = S.P.iturb == 0;
     int rc;
-    if ((rc = dalloc(c, &c->a_rb, (long)npv * S.NC)) || (rc = dalloc(c, &c->a_cb, 7L * npv * S.NC)) ||
+    if ((rc = dalloc(c, &c->a_rb, (long)npv * S.NC)) || (rc = dalloc(c, &c->a_cb, (long)(npv + (turb ? 15 : 0)) * S.NC)) ||
         (rc = dalloc(c, &c->a_cdb, 3L * S.NC)) || (rc = dalloc(c, &c->a_csb, 3L * S.NC)) || (rc = dalloc(c, &c->a_pb, (long)npv * S.NG)) ||
         (rc = dalloc(c, &c->a_sum, 16 + 16L * SUM_WG)))
         return rc;

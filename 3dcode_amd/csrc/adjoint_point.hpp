@@ -475,17 +475,17 @@ template <bool MLP, class F> HD ReconBar muscl_back(int nlim, F xs, double wl, d
     limiter_back(nlim, m, 1, -(0.5 * dqp * wr), rR, r1R, r2R, aR);
     if constexpr (MLP) {
         double b23 = 0.0, b32 = 0.0;
-        // the first point of group gq that holds value v
-        auto first = [&](int gq, double v) {
-            int at = 0;
-            const int lo = gq == 4 ? 19 : gq == 5 ? 28 : gq == 3 ? 2 : 1, hi = gq == 4 ? 27 : gq == 5 ? 36 : 18;
-            const int st = (gq == 2 || gq == 3) ? 2 : 1;
+        // the first point of group gq that holds value v: one bit a point
+        // (lo: ll 1..18, hi: the nine of the side's plane), then the group's mask
+        auto first = [&](int gq, double v, int plane) {
+            unsigned lo = 0, hi = 0;
 #pragma unroll
-            for (int q = 1; q <= 36; q++) {
-                const bool in = q >= lo && q <= hi && (st == 1 || ((q - lo) & 1) == 0);
-                if (in && at == 0 && xs(q) == v) at = q;
-            }
-            return at;
+            for (int q = 0; q < 18; q++) lo |= xs(q + 1) == v ? 1u << q : 0u;
+#pragma unroll
+            for (int q = 0; q < 9; q++) hi |= xs(plane + q) == v ? 1u << q : 0u;
+            lo &= gq == 1 ? 0x3FFFFu : gq == 2 ? 0x15555u : gq == 3 ? 0x2AAAAu : 0u;
+            hi = gq >= 4 ? hi : 0u;
+            return lo ? __builtin_ctz(lo) + 1 : hi ? __builtin_ctz(hi) + plane : 0;
         };
         if (a0 != 0.0 && A0 < 2.0 && A0 > 1.0) {
             const double ab = a0 * A0;
@@ -497,7 +497,7 @@ template <bool MLP, class F> HD ReconBar muscl_back(int nlim, F xs, double wl, d
             const double nb = -(yb * dyl + zb * dzl);
             b10 += nb; b23 -= nb;
             const double qb = (vl - x9 < 0.0 ? -1.0 : 1.0) * (ab / qml);
-            o.el = qb; o.il = first(gl, vl);
+            o.el = qb; o.il = first(gl, vl, 19);
             b9 -= qb;
         }
         if (aR != 0.0 && A1 < 2.0 && A1 > 1.0) {
@@ -512,7 +512,7 @@ template <bool MLP, class F> HD ReconBar muscl_back(int nlim, F xs, double wl, d
             const double nb = -(yb * dyr + zb * dzr);
             b32 += nb; b9 -= nb;
             const double qb = (vr - x10 < 0.0 ? -1.0 : 1.0) * (ab / qmr);
-            o.er = qb; o.ir = first(gr, vr);
+            o.er = qb; o.ir = first(gr, vr, 28);
             b10 -= qb;
         }
         o.x23 = b23; o.x32 = b32;
@@ -1082,6 +1082,131 @@ HD void visc_back(const Par &P, const double *nx, const double e4[4][3], const d
         o.g3[q][1] = q < nv ? vol * (gb[q][0] * em[0] + gb[q][1] * em[1] + gb[q][2] * em[2]) : 0.0;
         o.g3[q][2] = q < nv ? vol * (gb[q][0] * tm[0] + gb[q][1] * tm[1] + gb[q][2] * tm[2]) : 0.0;
     }
+}
+
+// bars of one cell's sources
+struct SourceBar {
+    double pc[NPV];                   // the cell's own state
+    double g[5][3];                   // the gradients of u, v, w, k, omega
+    double rho, h, mu, mut;           // its properties and eddy viscosity
+    double sc[3];                     // the mass-transfer scales u_ref, dp_ref, t_ref
+};
+
+// rb . (the cell's sources) backwards: mass transfer, SST, BDF.  MODELS as
+// k_combine.  The sources depend on the cell through few numbers - the
+// mass transfer through (p, T, y1, y2, rho) and its three scales, SST through
+// k, omega, three properties and SstGrad's invariants of the fifteen gradient
+// components - so dual passes run over those of each source alone (one
+// sum over all thirty inputs ran every source in each of fifteen two-lane
+// passes), and the invariants and the BDF term are transposed by hand.
+template <bool MODELS>
+HD void source_back(const Par &P, const double *pc, const double *d, const double gr[5][3], const double f6[6][3], double vol,
+                    double ydn, double mut, const double *rb, SourceBar &o)
+{
+    for (int n = 0; n < NPV; n++) o.pc[n] = 0.0;
+    for (int v = 0; v < 5; v++) for (int c = 0; c < 3; c++) o.g[v][c] = 0.0;
+    o.rho = o.h = o.mu = o.mut = o.sc[0] = o.sc[1] = o.sc[2] = 0.0;
+    if (P.ncav >= 1) {
+        // p, T, y1, y2, rho, u_ref, dp_ref, t_ref
+        constexpr int W = 2;
+        using T = Dn<W>;
+        const double x[5] = {pc[0], pc[4], pc[5], pc[6], d[D_RHO]};
+        double zb[8];
+        dn_grad<W>(8, [&](int q) -> double { return q < 5 ? x[q] : 0.0; }, [&](auto in, int base) -> T {
+            Par Pu = P;
+            auto lane_of = [&](int q) { const int l = q - base; return l >= 0 && l < W ? l + 1 : 0; };
+            Pu.uref_seed = lane_of(5);
+            Pu.dpref_seed = lane_of(6);
+            Pu.tref_seed = lane_of(7);
+            T p[NPV], dt[ND], rc, rv, ic[4];
+            for (int n = 0; n < NPV; n++) p[n] = T(pc[n]);
+            p[0] = in(0); p[4] = in(1); p[5] = in(2); p[6] = in(3);
+            bool full_eos = false;
+            if constexpr (MODELS)
+                if (P.ncav >= 2) {      // on the cell's full EOS, as k_combine<true>
+                    T dd[ND], full[18];
+                    mixture_eos<T>(p[0] + P.pref, p[4], p[5], p[6], dd, false, full);
+                    cav_model<T>(Pu, p, full, vol, rc, rv, ic);
+                    full_eos = true;
+                }
+            if (!full_eos) {
+                for (int m = 0; m < ND; m++) dt[m] = T(d[m]);
+                dt[D_RHO] = in(4);
+                merkle<T>(Pu, p, dt, vol, rc, rv, ic);
+            }
+            return rb[5] * (rv - rc);
+        }, zb);
+        o.pc[0] = zb[0]; o.pc[4] = zb[1]; o.pc[5] = zb[2]; o.pc[6] = zb[3];
+        o.rho = zb[4];
+        const bool sc = P.ncav <= 3;
+        for (int q = 0; q < 3; q++) o.sc[q] = sc ? zb[5 + q] : 0.0;
+    }
+    if (P.iturb == 0) {
+        // k, omega, rho, mu, mu_t and the invariants div, S^2, k-omega product (and W^2)
+        constexpr int W = MODELS ? 3 : 4, NI = MODELS ? 9 : 8;
+        using T = Dn<W>;
+        const double *gu = gr[0], *gv = gr[1], *gw = gr[2];
+        const SstGrad<double> gi = sst_grad<MODELS, double>(gu, gv, gw, gr[3], gr[4]);
+        const double x[9] = {pc[7], pc[8], d[D_RHO], d[D_MU], mut, gi.div, gi.s2, gi.pkw, gi.w2};
+        double zb[NI];
+        dn_grad<W>(NI, [&](int q) -> double { return x[q]; }, [&](auto in, int) -> T {
+            T dt[ND], src[2], it[4], oc;
+            for (int m = 0; m < ND; m++) dt[m] = T(d[m]);
+            dt[D_RHO] = in(2); dt[D_MU] = in(3);
+            const SstGrad<T> g{in(5), in(6), in(7), MODELS ? in(8) : T(0.0)};
+            sst_source_i<MODELS, T>(P, g, in(0), in(1), f6, vol, ydn, dt, in(4), src, it, oc);
+            return rb[7] * src[0] + rb[8] * src[1];
+        }, zb);
+        o.pc[7] = zb[0]; o.pc[8] = zb[1];
+        o.rho += zb[2]; o.mu = zb[3]; o.mut = zb[4];
+        const double s2 = 2.0 * zb[6], w2 = MODELS ? 2.0 * zb[NI - 1] : 0.0;
+        for (int c = 0; c < 3; c++) {
+            o.g[c][c] = zb[5] + 2.0 * s2 * gr[c][c];
+            o.g[3][c] = zb[7] * gr[4][c];
+            o.g[4][c] = zb[7] * gr[3][c];
+        }
+        for (int a = 0; a < 2; a++)
+            for (int b = a + 1; b < 3; b++) {
+                const double sm = s2 * (gr[a][b] + gr[b][a]), df = MODELS ? w2 * (gr[a][b] - gr[b][a]) : 0.0;
+                o.g[a][b] = sm + df;
+                o.g[b][a] = sm - df;
+            }
+    }
+    if (P.nsteady > 0) {
+        // - rb[n] nsteady bdf_b fx[n] vol / dt_phy, fx = rho (1, u, v, w, H, ...) - (0, 0, 0, 0, p, ...)
+        const double c = -((double)P.nsteady * P.bdf_b * vol / P.dt_phy), rho = d[D_RHO];
+        const double e = c * rb[4];
+        o.rho += c * rb[0] + e * (d[D_H] + 0.5 * (pc[1] * pc[1] + pc[2] * pc[2] + pc[3] * pc[3]));
+        o.h += e * rho;
+        o.pc[0] -= e;
+        for (int q = 1; q <= 3; q++) {
+            o.rho += c * rb[q] * pc[q];
+            o.pc[q] += rho * (c * rb[q] + e * pc[q]);
+        }
+        for (int n = 5; n < NPV; n++) if (n < P.npv) { o.rho += c * rb[n] * pc[n]; o.pc[n] += rho * (c * rb[n]); }
+    }
+}
+
+// the eddy viscosity's bar mb back to rho, mu, k, omega and the velocity
+// gradients through mu_t = sst_eddy_g, one dual pass over (rho, mu, k, omega, S:S)
+HD void eddy_back(double mb, const double *pc, const double *d, const double gr[5][3], double ydn, SourceBar &o)
+{
+    const double x[5] = {d[D_RHO], d[D_MU], pc[7], pc[8], sst_sij<double>(gr[0], gr[1], gr[2])};
+    double eb[5];
+    dn_grad<5>(5, [&](int q) -> double { return x[q]; },
+               [&](auto in, int) -> Dn<5> { return sst_eddy_i<Dn<5>>(in(0), in(1), in(2), in(3), in(4), ydn); }, eb);
+    o.rho += mb * eb[0];
+    o.mu += mb * eb[1];
+    o.pc[7] += mb * eb[2];
+    o.pc[8] += mb * eb[3];
+    const double s = mb * eb[4];
+    for (int a = 0; a < 3; a++) o.g[a][a] += 2.0 * s * gr[a][a];
+    for (int a = 0; a < 2; a++)
+        for (int b = a + 1; b < 3; b++) {
+            const double sm = s * (gr[a][b] + gr[b][a]);
+            o.g[a][b] += sm;
+            o.g[b][a] += sm;
+        }
 }
 
 }  // namespace cav

@@ -1714,22 +1714,22 @@ HD R des_length(int ides, R k, R om, const double f6[6][3], double vol, double y
     return fd * (1.0 + fe) * tl_rans + (1.0 - fd) * tl_les;
 }
 
-// The SST source from the cell's Green-Gauss gradients of u, v, w, k, omega
-// and its own k, omega (the adjoint differentiates this form: the neighbours
-// enter only through the gradients, which are linear in them).
+// What the SST source reads of the velocity, k and omega gradients: the
+// divergence, 2 S:S, the k-omega cross product and (DES) the vorticity's square
+template <class R> struct SstGrad { R div, s2, pkw, w2; };
+
+// The SST source from these and the cell's own k, omega (the adjoint
+// differentiates this form: the gradients enter only through the four).
 template <bool DES = false, class R = double>
-HD void sst_source_g(const Par &P, const R *gu, const R *gv, const R *gw, const R *gk, const R *go, R k, R om,
-                     const double f6[6][3], double vol, double ydns, const R *d, R mut, R *src, R *itt, R &ocut)
+HD void sst_source_i(const Par &P, const SstGrad<R> &gi, R k, R om, const double f6[6][3], double vol, double ydns,
+                     const R *d, R mut, R *src, R *itt, R &ocut)
 {
     const double c23 = 2.0 / 3.0, c59 = 5.0 / 9.0;
-    R div = gu[0] + gv[1] + gw[2];
-    R s2 = 2.0 * (gu[0] * gu[0] + gv[1] * gv[1] + gw[2] * gw[2]) + (gu[1] + gv[0]) * (gu[1] + gv[0])
-         + (gu[2] + gw[0]) * (gu[2] + gw[0]) + (gv[2] + gw[1]) * (gv[2] + gw[1]);
+    const R div = gi.div, s2 = gi.s2, pkw = gi.pkw;
     R rho = d[D_RHO];
     R prod = mut * (s2 - c23 * (div * div)) - c23 * rho * k * div;
     prod = mn(prod, 0.9 * rho * k * om);
     ocut = sqrt(s2 - c23 * (div * div));
-    R pkw = gk[0] * go[0] + gk[1] * go[1] + gk[2] * go[2];
     R cdkw = mx(1.712 * rho / om * pkw, R(1.0e-10));
     R t1 = sqrt(k) / (0.09 * om * ydns);
     R t2 = 500.0 * d[D_MU] / rho / (om * (ydns * ydns));
@@ -1742,8 +1742,7 @@ HD void sst_source_g(const Par &P, const R *gu, const R *gv, const R *gw, const 
     R ki = 1.0 / k, oi = 1.0 / om, ei = 1.0 / mut;
     R tl;
     if constexpr (DES) {
-        R w2 = (gu[1] - gv[0]) * (gu[1] - gv[0]) + (gu[2] - gw[0]) * (gu[2] - gw[0]) + (gv[2] - gw[1]) * (gv[2] - gw[1]);
-        tl = des_length<R>(P.ides, k, om, f6, vol, ydns, d[D_MU], mut, bf, s2, w2);
+        tl = des_length<R>(P.ides, k, om, f6, vol, ydns, d[D_MU], mut, bf, s2, gi.w2);
     } else {
         tl = sqrt(k) / 9.0 / om * 100.0;
     }
@@ -1763,6 +1762,29 @@ HD void sst_source_g(const Par &P, const R *gu, const R *gv, const R *gw, const 
     itt[0] = itt[0] * s1; itt[1] = itt[1] * s1; itt[2] = itt[2] * s2s; itt[3] = itt[3] * s2s;
 }
 
+template <bool DES = false, class R = double>
+HD SstGrad<R> sst_grad(const R *gu, const R *gv, const R *gw, const R *gk, const R *go)
+{
+    SstGrad<R> g;
+    g.div = gu[0] + gv[1] + gw[2];
+    g.s2 = 2.0 * (gu[0] * gu[0] + gv[1] * gv[1] + gw[2] * gw[2]) + (gu[1] + gv[0]) * (gu[1] + gv[0])
+         + (gu[2] + gw[0]) * (gu[2] + gw[0]) + (gv[2] + gw[1]) * (gv[2] + gw[1]);
+    g.pkw = gk[0] * go[0] + gk[1] * go[1] + gk[2] * go[2];
+    if constexpr (DES)
+        g.w2 = (gu[1] - gv[0]) * (gu[1] - gv[0]) + (gu[2] - gw[0]) * (gu[2] - gw[0]) + (gv[2] - gw[1]) * (gv[2] - gw[1]);
+    else
+        g.w2 = R(0.0);
+    return g;
+}
+
+// the same from the gradients themselves
+template <bool DES = false, class R = double>
+HD void sst_source_g(const Par &P, const R *gu, const R *gv, const R *gw, const R *gk, const R *go, R k, R om,
+                     const double f6[6][3], double vol, double ydns, const R *d, R mut, R *src, R *itt, R &ocut)
+{
+    sst_source_i<DES, R>(P, sst_grad<DES, R>(gu, gv, gw, gk, go), k, om, f6, vol, ydns, d, mut, src, itt, ocut);
+}
+
 // k-omega SST source: src[2], itt[4], omega_cut.  DES: the length-scale
 // variants are compiled in (the RANS-only instantiation keeps its registers).
 template <bool DES = false, class R = double>
@@ -1780,20 +1802,28 @@ HD void sst_source(const Par &P, const R x7[7][NPV], const double f6[6][3], doub
 }
 
 // SST eddy viscosity mu_t = 0.31 rho k / max(0.31 omega, S F2)
-// the SST eddy viscosity from the cell's rho, mu, k, omega and its velocity
-// gradients gu, gv, gw (src/eddy_module.f90:135-187); R = double or a dual
-// number (the adjoint differentiates it with respect to all eleven inputs)
+// from the cell's rho, mu, k, omega and the S:S of its velocity gradients
+// (src/eddy_module.f90:135-187); R = double or a dual number (the adjoint
+// differentiates it with respect to all five)
 template <class R>
-HD R sst_eddy_g(R rho, R mu, R k, R om, const R *gu, const R *gv, const R *gw, double ydns)
+HD R sst_eddy_i(R rho, R mu, R k, R om, R sij, double ydns)
 {
     R t1 = sqrt(k) / (0.09 * om * ydns);
     R t2 = 500.0 * mu / rho / (om * (ydns * ydns));
     R a2 = mx(2.0 * t1, t2);
     R bf2 = tanh(a2 * a2);
-    R sij = gu[0] * gu[0] + gv[1] * gv[1] + gw[2] * gw[2]
-          + 0.5 * ((gu[1] + gv[0]) * (gu[1] + gv[0]) + (gu[2] + gw[0]) * (gu[2] + gw[0]) + (gv[2] + gw[1]) * (gv[2] + gw[1]));
     R sss = sqrt(2.0 * sij);
     return 0.31 * rho * k / mx(0.31 * om, sss * bf2);
+}
+template <class R> HD R sst_sij(const R *gu, const R *gv, const R *gw)
+{
+    return gu[0] * gu[0] + gv[1] * gv[1] + gw[2] * gw[2]
+         + 0.5 * ((gu[1] + gv[0]) * (gu[1] + gv[0]) + (gu[2] + gw[0]) * (gu[2] + gw[0]) + (gv[2] + gw[1]) * (gv[2] + gw[1]));
+}
+template <class R>
+HD R sst_eddy_g(R rho, R mu, R k, R om, const R *gu, const R *gv, const R *gw, double ydns)
+{
+    return sst_eddy_i<R>(rho, mu, k, om, sst_sij<R>(gu, gv, gw), ydns);
 }
 
 HD double sst_eddy(const double x7[7][NPV], const double f6[6][3], double vol, double ydns, const double *d)
