@@ -50,9 +50,10 @@ struct AD {
     double *cdb;            // cell-source property bars [3][NC]: rho, h, mu
     double *csb;            // cell-source d(phi_c)/d(u_ref, dp_ref, t_ref) [3][NC] (the mass-transfer scales)
     double *pb;             // pv_bar [npv][NG]
+    double *pbd[3];         // the stencil pass's share of it, by direction
     double *mtb[3];         // eddy-viscosity bars of a face's two cells [2][NF] (dmut)
-    const int *tiles;       // tiles of the stencil pass: block, first i, j, k
-    int ntiles;
+    const int *tiles[3];    // tiles of the stencil pass by direction: block, first i, j, k
+    int ntiles[3];
     int dmut;               // 1: the interior cells' eddy viscosity is the SST function of
                             // the state (differentiated); 0: held fixed
 };
@@ -219,22 +220,53 @@ __global__ __launch_bounds__(128) void k_vface_vjp(DS S, AD A)
     }
 }
 
-// The stencil pass: one wavefront owns a tile of AI x AJ x AK ghosted cells of
-// one variable and adds to them, in LDS, what every face whose stencil
-// reaches the tile leaves on its points: the reconstruction run backwards
-// from the face's two bars (muscl_back) and the viscous differences'
-// transposes.  Faces near a tile's edge are run by every tile they reach
-// (twice on average at 16 x 8 x 8), which costs arithmetic but no memory: with
-// the bars of all 38 points written per face and variable and gathered by a
-// second kernel, a product moved 9 GB through them at 128 x 64 x 64.  Within
-// one LDS add the lanes (distinct faces, one stencil point) hit distinct
-// cells, and a wavefront's LDS operations run in its program order, so the
-// sums have a fixed order.
-constexpr int AI = 16, AJ = 8, AK = 8;
-template <int D, int NM>
-__device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, const BlkD &B, const int *c0, const int *c1, int n,
-                                                int vq, int cq, int nv, const double *sen, double *acc)
+// The stencil pass: one wavefront owns a tile of ghosted cells, one variable
+// and one direction, and adds to the tile, in LDS, what every face of that
+// direction whose stencil reaches it leaves on its points: the reconstruction run
+// backwards from the face's two bars (muscl_back) and the viscous differences'
+// transposes.  Faces near a tile's edge are run by every tile they reach,
+// which costs arithmetic but no memory: with the bars of all 38 points written
+// per face and variable and gathered by a second kernel, a product moved 9 GB
+// through them at 128 x 64 x 64.  A stencil reaches further along its normal
+// (-2 .. 3) than across (-1 .. 1), so a direction's tile (16 KB of LDS) is
+// twice as long along it: 1.8 runs a face, 2.2 with one 16 x 8 x 8 tile for
+// the three directions.  SMALL: 16 x 8 x 8, for grids with too few of the
+// larger tiles to fill the chip (adj_alloc).  Within one LDS add the lanes (distinct faces, one
+// stencil point) hit distinct cells, and a wavefront's LDS operations run in
+// its program order, so the sums have a fixed order.
+// What bounds it: the arithmetic of the reconstruction's bound and its
+// transpose (780 vector instructions a round of 64 faces) at two
+// wavefronts a SIMD, which the 38 stencil values in registers allow; three
+// spill (1.95 -> 2.43 ms).  128x64x64 cells, MLP, nine variables: 2.6 ms with
+// one tile for the three directions and a selected extremum looped over, 1.95
+// with the limiter's bars in registers, 1.58 with a tile a direction.
+constexpr int ADJ_TILE[2][3][3] = {{{32, 8, 8}, {16, 16, 8}, {16, 8, 16}}, {{16, 8, 8}, {16, 8, 8}, {16, 8, 8}}};
+constexpr int ADJ_CELLS[2] = {2048, 1024};
+// Element q of the array at base, the same for every lane: the base stays in
+// scalar registers and a lane holds one 32-bit offset for all the stencil's
+// points.  (A field of one block is below 4 GB: 2^29 cells of a context's
+// arrays would take more than the device's memory.)
+template <class T> __device__ __forceinline__ T lane_at(const T *base, unsigned q)
 {
+    return *(const T *)((const char *)base + (size_t)(q * (unsigned)sizeof(T)));
+}
+template <int D, int NM, bool SMALL>
+__device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, int item, double *acc)
+{
+    constexpr int TI = ADJ_TILE[SMALL][D][0], TJ = ADJ_TILE[SMALL][D][1], TK = ADJ_TILE[SMALL][D][2], NT = TI * TJ * TK;
+    static_assert(NT == ADJ_CELLS[SMALL], "a tile fills the LDS array");
+    const int n = item / A.ntiles[D];
+    const int *td = A.tiles[D] + 4 * (item - n * A.ntiles[D]);
+    const BlkD &B = S.b[td[0]];
+    const int c0[3] = {td[1], td[2], td[3]};
+    const int c1[3] = {min(c0[0] + TI - 1, B.I + 3), min(c0[1] + TJ - 1, B.J + 3), min(c0[2] + TK - 1, B.K + 3)};
+    for (int q = threadIdx.x; q < NT; q += 64) acc[q] = 0.0;
+    const bool visc = S.P.iturb >= -2;
+    // the variable's place among the viscous differences (u, v, w, T, k, omega) and averages (u, v, w, k, omega)
+    const int vq = !visc ? -1 : (n >= 1 && n <= 4) ? n - 1 : n >= 7 ? n - 3 : -1;
+    const int cq = !visc ? -1 : (n >= 1 && n <= 3) ? n - 1 : n >= 7 ? n - 4 : -1;
+    const int nv = S.P.iturb == 0 ? 6 : 4;
+    const double *sen = n == 0 && (S.P.nscheme == 2 || S.P.nscheme == 3) ? A.snb[D] : nullptr;
     constexpr int E = (D + 1) % 3, T = (D + 2) % 3;
     const int npv = S.npv, ext[3] = {B.I, B.J, B.K}, lane = threadIdx.x;
     const long NF = S.NF[D];
@@ -245,9 +277,10 @@ __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, const 
     cnt[D] = min(c1[D] + 2, ext[D]) - lo[D] + 1;
     cnt[E] = min(c1[E] + 1, ext[E]) - lo[E] + 1;
     cnt[T] = min(c1[T] + 1, ext[T]) - lo[T] + 1;
-    if (cnt[0] <= 0 || cnt[1] <= 0 || cnt[2] <= 0) return;
-    const int total = cnt[0] * cnt[1] * cnt[2];
-    constexpr int st[3] = {1, AI, AI * AJ};
+    // (no face reaches a tile that lies beyond the last ghost layer but one)
+    const int total = cnt[0] > 0 && cnt[1] > 0 && cnt[2] > 0 ? cnt[0] * cnt[1] * cnt[2] : 0;
+    constexpr int st[3] = {1, TI, TI * TJ};
+    const int fn[2] = {D == 0 ? B.I : B.I - 1, D == 1 ? B.J : B.J - 1};       // the block's faces along i and j
     // q / cnt of small numbers through the reciprocal: (q + 0.5) / cnt is at
     // least 0.5 / cnt away from every whole number, far more than it is rounded by
     const float i0 = 1.0f / (float)cnt[0], i1 = 1.0f / (float)cnt[1];
@@ -257,9 +290,10 @@ __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, const 
         const int q = on ? r : 0;
         const int q1 = (int)(((float)q + 0.5f) * i0), q2 = (int)(((float)q1 + 0.5f) * i1);
         const int f[3] = {lo[0] + q - q1 * cnt[0], lo[1] + q1 - q2 * cnt[1], lo[2] + q2};
-        const long t = fidx(B, D, f[0], f[1], f[2]);
-        double wl = A.w[D][(long)n * NF + t], wr = A.w[D][(long)(npv + n) * NF + t];
-        const int cell = A.cell[D][t];
+        // the face's place in its block (fidx)
+        const unsigned t = (unsigned)(f[0] - (D == 0 ? 1 : 2) + fn[0] * (f[1] - (D == 1 ? 1 : 2) + fn[1] * (f[2] - (D == 2 ? 1 : 2))));
+        double wl = lane_at(A.w[D] + (long)n * NF + B.f0[D], t), wr = lane_at(A.w[D] + (long)(npv + n) * NF + B.f0[D], t);
+        const int cell = lane_at(A.cell[D] + B.f0[D], t);
         // the face's left cell in tile coordinates; which offsets along each axis land in the tile
         const int l[3] = {f[0] - c0[0], f[1] - c0[1], f[2] - c0[2]};
         const int w3[3] = {c1[0] - c0[0], c1[1] - c0[1], c1[2] - c0[2]};
@@ -286,16 +320,23 @@ __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, const 
         o.x9 = o.x10 = o.x23 = o.x32 = o.x37 = o.x38 = 0.0;
         o.x3 = o.x4 = o.x7 = o.x8 = o.x11 = o.x12 = o.x15 = o.x16 = o.el = o.er = 0.0;
         o.il = o.ir = 0;
+        // the viscous bars and the stencil, read ahead of the arithmetic (and
+        // whether or not the reconstruction's bars are zero): one memory latency a round
+        double v0 = 0.0, v1 = 0.0, v2 = 0.0, vc = 0.0;
+        if (vq >= 0) {
+            v0 = lane_at(A.vb[D] + (long)(3 * vq) * NF + B.f0[D], t);
+            v1 = 0.0625 * lane_at(A.vb[D] + (long)(3 * vq + 1) * NF + B.f0[D], t);
+            v2 = 0.0625 * lane_at(A.vb[D] + (long)(3 * vq + 2) * NF + B.f0[D], t);
+            if (cq >= 0) vc = 0.5 * lane_at(A.vb[D] + (long)(3 * nv + cq) * NF + B.f0[D], t);
+        }
         if constexpr (NM > 0) {
-            const bool rec = on && (wl != 0.0 || wr != 0.0);
-            if (__ballot(rec)) {
-                const double *f0 = S.pv + (long)n * S.NG + gidx(B, f[0], f[1], f[2]);
-                double x[NSLOT];
+            const double *f0 = S.pv + (long)n * S.NG + B.g0;
+            const unsigned gl = (unsigned)(f[0] + 1 + B.nx * (f[1] + 1 + B.ny * (f[2] + 1)));
+            double x[NSLOT];
 #pragma unroll
-                for (int ll = 1; ll <= NSLOT; ll++)
-                    if (NM == 2 || ll == 9 || ll == 10 || ll == 23 || ll == 32 || ll >= 37) x[ll - 1] = f0[stencil_off<D>(B, ll)];
-                if (rec) o = muscl_back<NM == 2>(S.P.nlim, [&](int ll) -> double { return x[ll - 1]; }, wl, wr);
-            }
+            for (int ll = 1; ll <= NSLOT; ll++)
+                if (NM == 2 || ll == 9 || ll == 10 || ll == 23 || ll == 32 || ll >= 37) x[ll - 1] = lane_at(f0 + stencil_off<D>(B, ll), gl);
+            if (on && (wl != 0.0 || wr != 0.0)) o = muscl_back<NM == 2>(S.P.nlim, [&](int ll) -> double { return x[ll - 1]; }, wl, wr);
         }
         b9 += o.x9;
         b10 += o.x10;
@@ -305,14 +346,7 @@ __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, const 
         auto ex = [&](int ll) -> double { return exl(ll) + exr(ll); };
         if (vq >= 0 || sen) {
             // the 18 points of the viscous differences (and of the pressure sensor)
-            double v0 = 0.0, v1 = 0.0, v2 = 0.0, vc = 0.0;
-            if (vq >= 0) {
-                v0 = A.vb[D][(long)(3 * vq) * NF + t];
-                v1 = 0.0625 * A.vb[D][(long)(3 * vq + 1) * NF + t];
-                v2 = 0.0625 * A.vb[D][(long)(3 * vq + 2) * NF + t];
-                if (cq >= 0) vc = 0.5 * A.vb[D][(long)(3 * nv + cq) * NF + t];
-            }
-            auto sn = [&](int ll) -> double { return (sen ? sen[(long)(ll - 1) * NF + t] : 0.0) + ex(ll); };
+            auto sn = [&](int ll) -> double { return (sen ? lane_at(sen + (long)(ll - 1) * NF + B.f0[D], t) : 0.0) + ex(ll); };
             add(1, -v1 - v2 + sn(1));
             add(2, -v1 - v2 + sn(2));
             add(3, o.x3 - 2.0 * v2 + sn(3));
@@ -356,33 +390,22 @@ __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, const 
                 }
         }
     }
-}
-
-template <int NM>
-__global__ __launch_bounds__(64) void k_adj_stencil(DS S, AD A)
-{
-    __shared__ double acc[AI * AJ * AK];
-    const int n = blockIdx.x / A.ntiles, lane = threadIdx.x;
-    const int *td = A.tiles + 4 * (blockIdx.x - n * A.ntiles);
-    const BlkD &B = S.b[td[0]];
-    const int c0[3] = {td[1], td[2], td[3]};
-    const int c1[3] = {min(c0[0] + AI - 1, B.I + 3), min(c0[1] + AJ - 1, B.J + 3), min(c0[2] + AK - 1, B.K + 3)};
-    for (int q = lane; q < AI * AJ * AK; q += 64) acc[q] = 0.0;
-    const bool visc = S.P.iturb >= -2;
-    // the variable's place among the viscous differences (u, v, w, T, k, omega) and averages (u, v, w, k, omega)
-    const int vq = !visc ? -1 : (n >= 1 && n <= 4) ? n - 1 : n >= 7 ? n - 3 : -1;
-    const int cq = !visc ? -1 : (n >= 1 && n <= 3) ? n - 1 : n >= 7 ? n - 4 : -1;
-    const int nv = S.P.iturb == 0 ? 6 : 4;
-    const bool sensor = n == 0 && (S.P.nscheme == 2 || S.P.nscheme == 3);
-    adj_stencil_dir<0, NM>(S, A, B, c0, c1, n, vq, cq, nv, sensor ? A.snb[0] : nullptr, acc);
-    adj_stencil_dir<1, NM>(S, A, B, c0, c1, n, vq, cq, nv, sensor ? A.snb[1] : nullptr, acc);
-    adj_stencil_dir<2, NM>(S, A, B, c0, c1, n, vq, cq, nv, sensor ? A.snb[2] : nullptr, acc);
     __syncthreads();
-    double *pb = A.pb + (long)n * S.NG;
-    for (int q = lane; q < AI * AJ * AK; q += 64) {
-        const int i = c0[0] + q % AI, j = c0[1] + (q / AI) % AJ, k = c0[2] + q / (AI * AJ);
+    double *pb = A.pbd[D] + (long)n * S.NG;
+    for (int q = threadIdx.x; q < NT; q += 64) {
+        const int i = c0[0] + q % TI, j = c0[1] + (q / TI) % TJ, k = c0[2] + q / (TI * TJ);
         if (i <= c1[0] && j <= c1[1] && k <= c1[2]) pb[gidx(B, i, j, k)] = acc[q];
     }
+}
+
+template <int NM, bool SMALL>
+__global__ __launch_bounds__(64) void k_adj_stencil(DS S, AD A)
+{
+    __shared__ double acc[ADJ_CELLS[SMALL]];
+    const int n0 = S.npv * A.ntiles[0], n1 = n0 + S.npv * A.ntiles[1], w = blockIdx.x;
+    if (w < n0) adj_stencil_dir<0, NM, SMALL>(S, A, w, acc);
+    else if (w < n1) adj_stencil_dir<1, NM, SMALL>(S, A, w - n0, acc);
+    else adj_stencil_dir<2, NM, SMALL>(S, A, w - n1, acc);
 }
 
 // Cell sources of one interior cell: the mass transfer, SST, BDF.  MODELS:
@@ -451,7 +474,9 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // the bars of its neighbours' sources, and its property bars (from the faces
 // whose cell it is and from its own sources) taken through its EOS, in a
 // fixed order.
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adj_cells(DS S, AD A)
+// Registers: the EOS terms take all 512 of one wavefront a SIMD; held to 256 it
+// kept 1.1 KB a lane in scratch memory (128x64x64: 634 us, now 345).
+__global__ __launch_bounds__(128) void k_adj_cells(DS S, AD A)
 {
     long gl = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (gl >= S.NG) return;
@@ -529,7 +554,10 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         eos_adj(P.iturb != -3, x4, dcb, gx);
         acc[0] += gx[0]; acc[4] += gx[1]; acc[5] += gx[2]; acc[6] += gx[3];
     }
-    for (int n = 0; n < NPV; n++) if (n < npv) A.pb[(long)n * S.NG + gl] += acc[n];
+    for (int n = 0; n < NPV; n++) if (n < npv) {
+        const long q = (long)n * S.NG + gl;
+        A.pb[q] = ((A.pbd[0][q] + A.pbd[1][q]) + A.pbd[2][q]) + acc[n];
+    }
 }
 
 // deterministic sum of n doubles in two stages: workgroup b sums its strided
@@ -567,6 +595,13 @@ __global__ __launch_bounds__(256) void k_dotdiff_fixed(const double *w, const do
     if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
+// The stencil pass takes the small tiles below this many large ones (times the
+// variables): two rounds of the wavefronts that fit the chip (two a SIMD).
+// 64x32x32 cells, 7 variables, TVD: 1575 large tiles take 161 us, the small
+// ones 114; 53x41x27, 9 variables, MLP: 1296, 399 and 358; 128x64x64, 9
+// variables, MLP: 10935, 1577 and 1719.
+constexpr long ADJ_FEW = 4096;
+
 int adj_alloc(cav3d_ctx *c)
 {
     if (c->adj_ready) return 0;
@@ -575,7 +610,7 @@ int adj_alloc(cav3d_ctx *c)
     const bool visc = S.P.iturb >= -2, turb = S.P.iturb == 0;
     int rc;
     if ((rc = dalloc(c, &c->a_rb, (long)npv * S.NC)) || (rc = dalloc(c, &c->a_cb, (long)(npv + (turb ? 15 : 0)) * S.NC)) ||
-        (rc = dalloc(c, &c->a_cdb, 3L * S.NC)) || (rc = dalloc(c, &c->a_csb, 3L * S.NC)) || (rc = dalloc(c, &c->a_pb, (long)npv * S.NG)) ||
+        (rc = dalloc(c, &c->a_cdb, 3L * S.NC)) || (rc = dalloc(c, &c->a_csb, 3L * S.NC)) || (rc = dalloc(c, &c->a_pb, (long)npv * S.NG)) || (rc = dalloc(c, &c->a_pbd, 3L * npv * S.NG)) ||
         (rc = dalloc(c, &c->a_sum, 16 + 16L * SUM_WG)))
         return rc;
     for (int d = 0; d < 3; d++)
@@ -588,18 +623,28 @@ int adj_alloc(cav3d_ctx *c)
             return rc;
     // tiles of the stencil pass over every block's ghosted cells
     std::vector<int> tl;
-    for (int b = 0; b < c->nb; b++) {
-        const BlkD &B = c->blk[b];
-        for (int k = -1; k <= B.K + 3; k += AK)
-            for (int j = -1; j <= B.J + 3; j += AJ)
-                for (int i = -1; i <= B.I + 3; i += AI) {
-                    const int t4[4] = {b, i, j, k};
-                    tl.insert(tl.end(), t4, t4 + 4);
-                }
+    int first[3];
+    for (c->a_small = 0;; c->a_small++) {
+        tl.clear();
+        for (int d = 0; d < 3; d++) {
+            const int *t = ADJ_TILE[c->a_small][d];
+            first[d] = (int)tl.size();
+            for (int b = 0; b < c->nb; b++) {
+                const BlkD &B = c->blk[b];
+                for (int k = -1; k <= B.K + 3; k += t[2])
+                    for (int j = -1; j <= B.J + 3; j += t[1])
+                        for (int i = -1; i <= B.I + 3; i += t[0]) {
+                            const int t4[4] = {b, i, j, k};
+                            tl.insert(tl.end(), t4, t4 + 4);
+                        }
+            }
+            c->a_ntiles[d] = (int)(tl.size() - first[d]) / 4;
+        }
+        if (c->a_small || npv * (long)tl.size() / 4 >= ADJ_FEW) break;
     }
-    c->a_ntiles = (int)(tl.size() / 4);
-    if ((rc = dalloc(c, &c->a_tiles, tl.size()))) return rc;
-    HIPCHK(hipMemcpyAsync(c->a_tiles, tl.data(), tl.size() * sizeof(int), hipMemcpyHostToDevice, c->st));
+    if ((rc = dalloc(c, &c->a_tiles[0], tl.size()))) return rc;
+    for (int d = 1; d < 3; d++) c->a_tiles[d] = c->a_tiles[0] + first[d];
+    HIPCHK(hipMemcpyAsync(c->a_tiles[0], tl.data(), tl.size() * sizeof(int), hipMemcpyHostToDevice, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
     c->adj_ready = true;
     return 0;
@@ -616,7 +661,7 @@ int launch_vjp(cav3d_ctx *c, int dmut = 0)
         A.vb[d] = c->a_vb[d]; A.vp[d] = c->a_vp[d]; A.ub[d] = c->a_ub[d]; A.mtb[d] = c->a_mtb[d];
     }
     A.cb = c->a_cb; A.cdb = c->a_cdb; A.csb = c->a_csb; A.pb = c->a_pb;
-    A.tiles = c->a_tiles; A.ntiles = c->a_ntiles;
+    for (int d = 0; d < 3; d++) { A.tiles[d] = c->a_tiles[d]; A.ntiles[d] = c->a_ntiles[d]; A.pbd[d] = c->a_pbd + (long)d * S.npv * S.NG; }
     const bool sensor = S.P.nscheme == 2 || S.P.nscheme == 3;
     const int npv = S.npv;
     // the faces' kernels are independent of each other: i on st, j and k on
@@ -645,10 +690,15 @@ int launch_vjp(cav3d_ctx *c, int dmut = 0)
     hipStreamWaitEvent(c->side[0], c->fork, 0);
     if (S.P.ides > 0 || S.P.ncav >= 2) hipLaunchKernelGGL(k_cell_vjp<true>, dim3(nblk(S.NC, 128)), dim3(128), 0, c->side[0], S, A);
     else hipLaunchKernelGGL(k_cell_vjp<false>, dim3(nblk(S.NC, 128)), dim3(128), 0, c->side[0], S, A);
-    const dim3 tg((unsigned)(npv * c->a_ntiles));
-    if (S.P.nmuscl == 0) hipLaunchKernelGGL(k_adj_stencil<0>, tg, dim3(64), 0, c->st, S, A);
-    else if (S.P.nmuscl == 1) hipLaunchKernelGGL(k_adj_stencil<1>, tg, dim3(64), 0, c->st, S, A);
-    else hipLaunchKernelGGL(k_adj_stencil<2>, tg, dim3(64), 0, c->st, S, A);
+    const dim3 tg((unsigned)(npv * (c->a_ntiles[0] + c->a_ntiles[1] + c->a_ntiles[2])));
+    auto stencil = [&](auto small) {
+        constexpr bool SMALL = decltype(small)::value;
+        if (S.P.nmuscl == 0) hipLaunchKernelGGL((k_adj_stencil<0, SMALL>), tg, dim3(64), 0, c->st, S, A);
+        else if (S.P.nmuscl == 1) hipLaunchKernelGGL((k_adj_stencil<1, SMALL>), tg, dim3(64), 0, c->st, S, A);
+        else hipLaunchKernelGGL((k_adj_stencil<2, SMALL>), tg, dim3(64), 0, c->st, S, A);
+    };
+    if (c->a_small) stencil(std::true_type());
+    else stencil(std::false_type());
     hipEventRecord(c->join[0], c->side[0]);
     hipStreamWaitEvent(c->st, c->join[0], 0);
     hipLaunchKernelGGL(k_adj_cells, dim3(nblk(S.NG, 128)), dim3(128), 0, c->st, S, A);

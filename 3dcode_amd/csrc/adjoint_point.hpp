@@ -348,33 +348,39 @@ __host__ __device__ __attribute__((always_inline)) inline void eos_adj(bool prop
 }
 
 // ------------------------------------------------------------ reconstruction
-// phib = the bar of limiter(nlim, m, s): adds to the bars of its r, r1, r2 and alp
-HD void limiter_back(int nlim, const LimState<double> &m, int s, double phib, double &rb, double &r1b, double &r2b, double &ab)
+// The bars of limiter(nlim, m, s)'s r, r1, r2 and alp from its own bar phib.
+// The slopes are selected as values (branches that add to one bar or another
+// become a store through a selected pointer: four bars in scratch memory
+// and a round trip to it in every reconstruction).
+struct LimBar { double r, r1, r2, a; };
+HD LimBar limiter_back(int nlim, const LimState<double> &m, int s, double phib)
 {
     const double r = m.r[s], a = m.alp[s];
+    LimBar o{0.0, 0.0, 0.0, 0.0};
     // max(0, min(a, a r, c)), c's slopes (cr, c1, c2) with respect to r, r1, r2
     auto low3 = [&](double c, double cr, double c1, double c2) {
         const double ar = a * r, t = ar < a ? ar : a, v = c < t ? c : t;
-        if (!(v > 0.0)) return;
-        if (c < t) { rb += phib * cr; r1b += phib * c1; r2b += phib * c2; }
-        else if (ar < a) { rb += phib * a; ab += phib * r; }
-        else ab += phib;
+        const bool on = v > 0.0, isc = on && c < t, isr = on && !(c < t) && ar < a, isa = on && !(c < t) && !(ar < a);
+        o.r = isc ? phib * cr : isr ? phib * a : 0.0;
+        o.r1 = isc ? phib * c1 : 0.0;
+        o.r2 = isc ? phib * c2 : 0.0;
+        o.a = isr ? phib * r : isa ? phib : 0.0;
     };
     // max(0, min(c r, 1), min(r, c)), c's slopes cr and ca with respect to r and a
     auto high2 = [&](double c, double cr, double ca) {
         const double q = c * r, i1 = 1.0 < q ? 1.0 : q, t = i1 > 0.0 ? i1 : 0.0, u = c < r ? c : r;
-        if (u > t) {
-            if (c < r) { rb += phib * cr; ab += phib * ca; }
-            else rb += phib;
-        } else if (i1 > 0.0 && !(1.0 < q)) { rb += phib * (c + cr * r); ab += phib * ca * r; }
+        const bool up = u > t, isc = up && c < r, isr = up && !(c < r), isq = !up && i1 > 0.0 && !(1.0 < q);
+        o.r = isc ? phib * cr : isr ? phib : isq ? phib * (c + cr * r) : 0.0;
+        o.a = isc ? phib * ca : isq ? phib * ca * r : 0.0;
     };
     const double ic5 = (-(2.0 * m.r1[s]) + 11.0 + 24.0 * r - 3.0 * m.r2[s]) / 30.0;
     switch (nlim) {
-    case 1: if (r < 1.0 && r > 0.0) rb += phib; break;
+    case 1: o.r = r < 1.0 && r > 0.0 ? phib : 0.0; break;
     case 2: {
         const double ar = a * r, i1 = ar < 1.0 ? ar : 1.0, t = i1 > 0.0 ? i1 : 0.0, u = r < a ? r : a;
-        if (u > t) { if (r < a) rb += phib; else ab += phib; }
-        else if (i1 > 0.0 && ar < 1.0) { rb += phib * a; ab += phib * r; }
+        const bool up = u > t, isq = !up && i1 > 0.0 && ar < 1.0;
+        o.r = up && r < a ? phib : isq ? phib * a : 0.0;
+        o.a = up && !(r < a) ? phib : isq ? phib * r : 0.0;
         break;
     }
     case 3: {
@@ -391,10 +397,11 @@ HD void limiter_back(int nlim, const LimState<double> &m, int s, double phib, do
     case 6: high2(a < 1.5 ? a : 1.5, 0.0, a < 1.5 ? 1.0 : 0.0); break;
     case 7: low3((1.0 + 2.0 * r) / 3.0, 2.0 / 3.0, 0.0, 0.0); break;
     case 8: low3(ic5, 24.0 / 30.0, -2.0 / 30.0, -3.0 / 30.0); break;
-    case 9: rb += phib * (2.0 / 3.0); break;
-    case 10: rb += phib * (24.0 / 30.0); r1b -= phib * (2.0 / 30.0); r2b -= phib * (3.0 / 30.0); break;
+    case 9: o.r = phib * (2.0 / 3.0); break;
+    case 10: o.r = phib * (24.0 / 30.0); o.r1 = -(phib * (2.0 / 30.0)); o.r2 = -(phib * (3.0 / 30.0)); break;
     default: break;
     }
+    return o;
 }
 
 // Bars of one variable's reconstruction: of the fourteen stencil points
@@ -470,9 +477,9 @@ template <bool MLP, class F> HD ReconBar muscl_back(int nlim, F xs, double wl, d
     // backwards
     const double phi0 = limiter(nlim, m, 0), phi1 = limiter(nlim, m, 1);
     double b9 = wl, b10 = wr, dqb = 0.0, dqmb = 0.5 * phi0 * wl, dqpb = -(0.5 * phi1 * wr), imb, ipb;
-    double r0 = 0, r10 = 0, r20 = 0, a0 = 0, rR = 0, r1R = 0, r2R = 0, aR = 0, ipx = 0;
-    limiter_back(nlim, m, 0, 0.5 * dqm * wl, r0, r10, r20, a0);
-    limiter_back(nlim, m, 1, -(0.5 * dqp * wr), rR, r1R, r2R, aR);
+    const LimBar lb = limiter_back(nlim, m, 0, 0.5 * dqm * wl), rb = limiter_back(nlim, m, 1, -(0.5 * dqp * wr));
+    double r0 = lb.r, rR = rb.r, ipx = 0;
+    const double r10 = lb.r1, r20 = lb.r2, a0 = lb.a, r1R = rb.r1, r2R = rb.r2, aR = rb.a;
     if constexpr (MLP) {
         double b23 = 0.0, b32 = 0.0;
         // the first point of group gq that holds value v: one bit a point

@@ -1683,8 +1683,8 @@ struct cav3d_ctx {
     // adjoint work arrays (allocated by the first cav3d_rhs_vjp)
     bool adj_ready = false;
     double *a_rb = nullptr, *a_w[3] = {}, *a_snb[3] = {}, *a_fp[3] = {}, *a_vb[3] = {}, *a_vp[3] = {}, *a_ub[3] = {}, *a_mtb[3] = {},
-           *a_cb = nullptr, *a_cdb = nullptr, *a_csb = nullptr, *a_pb = nullptr, *a_sum = nullptr, *a_save = nullptr, *a_obj = nullptr;
-    int *a_cell[3] = {}, *a_tiles = nullptr, a_ntiles = 0;
+           *a_cb = nullptr, *a_cdb = nullptr, *a_csb = nullptr, *a_pb = nullptr, *a_pbd = nullptr, *a_sum = nullptr, *a_save = nullptr, *a_obj = nullptr;
+    int *a_cell[3] = {}, *a_tiles[3] = {}, a_ntiles[3] = {}, a_small = 0;
     long a_obj_n = 0;
 };
 
