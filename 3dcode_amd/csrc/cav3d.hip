@@ -70,13 +70,9 @@ struct DS {           // device state, passed by value
     long NG, NC, NW, NF[3], NCX, NEX, NTX, NBC[3], NHALO;
     double *pv, *dc, *mut, *vol, *ydn, *cx, *ex, *tx;
     double *res, *dt, *icav, *itt, *ocut, *rcav, *qq;
-    double *dcv;
+    double *img;      // the sweeps' cell records [NW][RC_N]
     double *xqf, *xqb; // dq of the sweeps [NW][NPV], a cell's values adjacent: forward
                        // the cross-tile values only, backward every cell's
-    double *gx;       // diagonal-inverse terms [NGX][NC]
-    double *zero;     // zeros, one more than the longest pencil: the sweeps' source for absent items
-    double *jc;       // Jacobian cell terms [2][NC]: beta, h
-    double *jf;       // Jacobian face terms [18][NC]: faces -i,+i,-j,+j,-k,+k x (u, lam, vis)
     long NPLANE;      // sum over blocks of (J-1)(K-1)
     double *ff[3];    // face fluxes [2*npv][NF]
     double *red;      // norm partials
@@ -729,36 +725,81 @@ __global__ __launch_bounds__(256) void k_combine(DS S)
 }
 
 // ------------------------------------------------------------ LU-SGS sweeps
-// One hyperplane i+j+k = s of block b.  Thread -> (j,k); i = s - j - k.
+// What a sweep step reads of a cell lies side by side in memory, in a record
+// of 92 doubles (736 bytes, 46 pieces of 16), ranges and order of the dcv
+// array of the reference (1:I+1 and so on; the outer layer stays zero and is
+// what a pencil's absent neighbours read):
+//   RC_FP, RC_FM  the +i,+j,+k (-i,-j,-k) faces x (n3[3], u, lam, vis): the
+//                 forward (backward) sweep's split Jacobians
+//   RC_Q          the Jacobian's cell terms, in both sweeps
+//   RC_GX         the diagonal-inverse terms
+//   RC_RES        the residual; the forward sweep puts its dcv there
+// Field by field, the sweeps gathered 128 numbers a cell (the shared ones
+// once for each of the three pencils that read them) in 32-byte pieces of
+// 128-byte lines: 1.46 GB a forward sweep at 128x64x64, sixteen 64-lane
+// transfers of 32 lines each a step, whose issue was the length of a step.
+// Now it is 86 numbers a cell in whole lines and eleven transfers.
+enum { RC_FP = 0, RC_FM = 18, RC_Q = 36, RC_GX = 54, RC_RES = RC_GX + NGX, RC_N = RC_RES + NPV };
+enum { Q_RP = 0, Q_RT, Q_RY1, Q_RY2, Q_RHO, Q_BETA, Q_HP, Q_HT, Q_HY1, Q_HY2, Q_U, Q_V, Q_W, Q_Y1, Q_Y2, Q_K, Q_O, Q_H };
+static_assert(RC_GX - RC_Q == Q_H + 1 && RC_N == 92, "record layout");
+
 // Per-cell terms of the LU-SGS operator that do not depend on the sweep:
 // the diagonal-inverse coefficients and the Jacobian's cell and face terms
-// (src/lhs_module.f90:346-457, src/jacobian_module.f90:182-403).
+// (src/lhs_module.f90:346-457, src/jacobian_module.f90:182-403), written as
+// the cells' records.  Bound by HBM (736 bytes a cell written, some 450
+// read), so a wavefront turns its 64 records around in LDS, 24 numbers a cell
+// at a time, and twelve adjacent lanes write 192 bytes of one record.
 __global__ __launch_bounds__(128) void k_lhs_prep(DS S)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= S.NC) return;
-    const BlkD &B = S.b[find_blk(S, t, 0)];
+    constexpr int CH = 24;
+    __shared__ double turn[2][64][CH + 1];
+    __shared__ double *to[2][64];
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const bool on = t < S.NC;
+    const long tc = on ? t : S.NC - 1;
+    const BlkD &B = S.b[find_blk(S, tc, 0)];
     const Par &P = S.P;
     int i, j, k;
-    cell_of(B, t - B.c0, i, j, k);
+    cell_of(B, tc - B.c0, i, j, k);
+    to[wv][lane] = on ? S.img + widx(B, i, j, k) * RC_N : nullptr;
     CellJ cc;
     load_cell(S, B, i, j, k, cc);
     double f6[6][3];
     cell_faces(S, B, i, j, k, f6);
     double ic[4] = {0, 0, 0, 0}, it[4] = {0, 0, 0, 0};
-    if (P.ncav) for (int m = 0; m < 4; m++) ic[m] = S.icav[m * S.NC + t];
-    if (P.iturb == 0) for (int m = 0; m < 4; m++) it[m] = S.itt[m * S.NC + t];
-    double g[NGX];
-    getx_prep(P, S.npv, cc, f6, S.dt[t], ic, it, g);
-    for (int q = 0; q < NGX; q++) S.gx[q * S.NC + t] = g[q];
-    JacCell jc = jac_cell(P, cc);
-    S.jc[t] = jc.beta;
-    S.jc[S.NC + t] = jc.h;
+    if (P.ncav) for (int m = 0; m < 4; m++) ic[m] = S.icav[m * S.NC + tc];
+    if (P.iturb == 0) for (int m = 0; m < 4; m++) it[m] = S.itt[m * S.NC + tc];
+    double r[RC_N];
     for (int q = 0; q < 6; q++) {
-        JacFace f = jac_face(P, cc, f6[q]);
-        S.jf[(3 * q) * S.NC + t] = f.u;
-        S.jf[(3 * q + 1) * S.NC + t] = f.lam;
-        S.jf[(3 * q + 2) * S.NC + t] = f.vis;
+        const JacFace f = jac_face(P, cc, f6[q]);
+        double *o = r + ((q & 1) ? RC_FP : RC_FM) + 6 * (q >> 1);
+        o[0] = f6[q][0]; o[1] = f6[q][1]; o[2] = f6[q][2];
+        o[3] = f.u; o[4] = f.lam; o[5] = f.vis;
+    }
+    const JacCell jc = jac_cell(P, cc);
+    double *const c = r + RC_Q;
+    c[Q_RP] = cc.d[D_RP]; c[Q_RT] = cc.d[D_RT]; c[Q_RY1] = cc.d[D_RY1]; c[Q_RY2] = cc.d[D_RY2];
+    c[Q_RHO] = cc.d[D_RHO]; c[Q_BETA] = jc.beta;
+    c[Q_HP] = cc.d[D_HP]; c[Q_HT] = cc.d[D_HT]; c[Q_HY1] = cc.d[D_HY1]; c[Q_HY2] = cc.d[D_HY2];
+    c[Q_U] = cc.pv[1]; c[Q_V] = cc.pv[2]; c[Q_W] = cc.pv[3]; c[Q_Y1] = cc.pv[5]; c[Q_Y2] = cc.pv[6];
+    c[Q_K] = S.npv > 7 ? cc.pv[7] : 0.0; c[Q_O] = S.npv > 7 ? cc.pv[8] : 0.0;
+    c[Q_H] = jc.h;
+    getx_prep(P, S.npv, cc, f6, S.dt[tc], ic, it, r + RC_GX);
+    for (int n = 0; n < NPV; n++) r[RC_RES + n] = n < S.npv ? S.res[n * S.NC + tc] : 0.0;
+#pragma unroll
+    for (int c0 = 0; c0 < RC_N; c0 += CH) {
+        const int n = RC_N - c0 < CH ? RC_N - c0 : CH, units = n / 2, per = 64 / units;
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < n; q++) turn[wv][lane][q] = r[c0 + q];
+        __syncthreads();
+        const int u = lane % units, m0 = lane / units;
+        for (int m = m0; m < 64; m += per) {
+            double *o = to[wv][m];
+            if (m0 < per && o)
+                *(double2 *)(o + c0 + 2 * u) = make_double2(turn[wv][m][2 * u], turn[wv][m][2 * u + 1]);
+        }
     }
 }
 
@@ -793,10 +834,10 @@ __device__ __forceinline__ void st_dev(double *p, double v)
 // through a device-coherent exchange array that holds a cell's values side by
 // side (one write of 72 bytes, not nine 8-byte writes to nine lines), waited
 // for with a bounded poll.
-// Everything a cell reads that does not depend on the sweep (its residual,
-// state, properties, diagonal-inverse terms, and the Jacobian operands of its
-// j and k neighbours) is moved ahead of use into an LDS stage, so a step's
-// critical path is the dq hand-over and the arithmetic.
+// Everything a cell reads that does not depend on the sweep (its record and
+// the Jacobian operands of its j and k neighbours) is moved ahead of use into
+// an LDS stage, so a step's critical path is the dq hand-over and the
+// arithmetic.
 // Tiles wait only on tiles upstream in j and k.  A workgroup takes its tiles
 // from a ticket counter over the topological order, so whatever the number
 // of workgroups the device has started, every tile upstream of a started one
@@ -807,58 +848,19 @@ __device__ __forceinline__ void st_dev(double *p, double v)
 // with tickets, 64x32x32 0.95 and 0.74, 128x64x64 2.73 and 2.57, state
 // transfers included.)
 constexpr int TJ = 4, TK = 4;
-// LDS stage of one pencil-step (doubles)
+// LDS stage of one hyperplane (doubles): the tile's sixteen pencils, each its
+// cell's F (the sweep's side), Q, GX and RES; then the upstream neighbours in
+// other tiles of the four j-edge and the four k-edge pencils, each the F of
+// its face towards the tile and its Q.  A ring of SLABS hyperplanes: a step
+// reads its own and the next one's while the ones after are on their way.
 enum {
-    ST_RES = 0, ST_PV = 9, ST_DC = 18, ST_N3 = 31, ST_JC = 34, ST_JF = 36, ST_GX = 39,
-    ST_J = 68, ST_K = 98,                  // neighbour blocks: pv 9, dc 13, n3 3, jc 2, jf 3
-    NB_PV = 0, NB_DC = 9, NB_N3 = 22, NB_JC = 25, NB_JF = 27, ST_N = 128
+    SP_F = 0, SP_Q = 18, SP_GX = 36, SP_RES = SP_GX + NGX, SP_N = SP_RES + NPV,
+    SE_F = 0, SE_Q = 6, SE_N = 24,
+    SLAB_E = TJ * TK * SP_N, SLAB_USED = SLAB_E + (TJ + TK) * SE_N,
+    SLAB_LOADS = (SLAB_USED + 127) / 128, SLAB_N = 128 * SLAB_LOADS
 };
-static_assert(ST_GX + NGX == ST_J, "stage layout");
-
-__device__ __forceinline__ long face_off(const BlkD &B, int ax, const int *p)
-{
-    if (ax == 0) return B.cx0 + (p[0] - 1) + (long)B.I * ((p[1] - 1) + (long)(B.J + 1) * (p[2] - 1));
-    if (ax == 1) return B.ex0 + (p[0] - 1) + (long)(B.I + 1) * ((p[1] - 1) + (long)B.J * (p[2] - 1));
-    return B.tx0 + (p[0] - 1) + (long)(B.I + 1) * ((p[1] - 1) + (long)(B.J + 1) * (p[2] - 1));
-}
-__device__ __forceinline__ const double *face_base(const DS &S, const BlkD &B, int ax, const int *p, int comp)
-{
-    const long o = face_off(B, ax, p);
-    if (ax == 0) return S.cx + comp * S.NCX + o;
-    if (ax == 1) return S.ex + comp * S.NEX + o;
-    return S.tx + comp * S.NTX + o;
-}
-
-// Stage item e of pencil (j,k) of a sweep: every field is stored i fastest,
-// so the item of cell i is base[i]; nullptr where the item is not read.
-template <bool FWD>
-__device__ __forceinline__ const double *stage_base(const DS &S, const BlkD &B, int j, int k, int e)
-{
-    const int sg = FWD ? 1 : -1, side = FWD ? 1 : 0, npv = S.npv;
-    const long c = cidx(B, 0, j, k), g = gidx(B, 0, j, k);
-    if (e < ST_PV) return e < npv ? (FWD ? S.res + e * S.NC + c : S.dcv + e * S.NW + widx(B, 0, j, k)) : nullptr;
-    if (e < ST_DC) return (e - ST_PV) < npv ? S.pv + (e - ST_PV) * S.NG + g : nullptr;
-    if (e < ST_N3) return S.dc + (e - ST_DC) * S.NG + g;
-    if (e < ST_JC) { const int p[3] = {FWD ? 0 : -1, j, k}; return face_base(S, B, 0, p, e - ST_N3); }
-    if (e < ST_JF) return S.jc + (e - ST_JC) * S.NC + c;
-    if (e < ST_GX) return S.jf + (3 * side + e - ST_JF) * S.NC + c;
-    if (e < ST_J) return S.gx + (e - ST_GX) * S.NC + c;
-    const int ax = e < ST_K ? 1 : 2;
-    const int r = e - (ax == 1 ? ST_J : ST_K);
-    int m[3] = {0, j, k};
-    m[ax] -= sg;
-    const int lim = ax == 1 ? B.J : B.K;
-    if (m[ax] < 2 || m[ax] > lim) return nullptr;
-    const long gm = gidx(B, 0, m[1], m[2]), cm = cidx(B, 0, m[1], m[2]);
-    if (r < NB_DC) return r < npv ? S.pv + r * S.NG + gm : nullptr;
-    if (r < NB_N3) return S.dc + (r - NB_DC) * S.NG + gm;
-    if (r < NB_JC) { const int self[3] = {0, j, k}; return face_base(S, B, ax, FWD ? m : self, r - NB_N3); }
-    if (r < NB_JF) return S.jc + (r - NB_JC) * S.NC + cm;
-    return S.jf + (3 * (2 * ax + side) + r - NB_JF) * S.NC + cm;
-}
-
-static_assert(ST_PV + 9 == ST_DC && ST_DC + ND == ST_N3 && ST_N3 + 3 == ST_JC && ST_JC + 2 == ST_JF,
-              "the own-cell part of the stage has the neighbour-block layout");
+constexpr int SLABS = 6;
+static_assert(SP_N == RC_N - 18 && SP_RES - SP_GX == RC_RES - RC_GX && SP_GX - SP_Q == RC_GX - RC_Q, "stage layout");
 
 // lane q of the lane's 16-lane row, by one 64-bit DPP move (no LDS traffic)
 template <int Q>
@@ -878,7 +880,8 @@ __device__ __forceinline__ double row_lane(double v)
 // the terms that are one expression per column are formed once, a column per
 // lane, not in every lane.
 struct RowMap {
-    int v1, v2, p, g[7], co[3];     // stage items of this lane (v1, v2, p: within a neighbour block)
+    int v1, v2, p, g[7], co[3];     // stage items of this lane, within its pencil's part of a slab
+    bool face;                      // v1 is one of F (of the i face; the j and k faces' lie 6 and 12 further)
     double scale;                   // of v1: the sweep's sign and the factor 0.5 on u, lam, vis, rho
     double one[7];                  // 1 in the lane of the column
     bool mom, en, kw, cpl, n0, n4, n5, n7, n8;
@@ -887,27 +890,29 @@ template <bool FWD> __device__ __forceinline__ RowMap row_map(int lane, int npv)
 {
     RowMap m;
     // lanes 0..6: the column's factor of r1 (rho_p, n3, rho_T, rho_y1, rho_y2); then u, lam, vis, rho (scaled), beta, rho
-    m.v1 = lane == 0 ? NB_DC + D_RP : lane <= 3 ? NB_N3 + lane - 1 : lane == 4 ? NB_DC + D_RT : lane == 5 ? NB_DC + D_RY1
-         : lane == 6 ? NB_DC + D_RY2 : lane <= 9 ? NB_JF + lane - 7 : lane == 11 ? NB_JC : NB_DC + D_RHO;
+    m.face = (lane >= 1 && lane <= 3) || (lane >= 7 && lane <= 9);
+    m.v1 = lane >= 1 && lane <= 3 ? SP_F + lane - 1 : lane >= 7 && lane <= 9 ? SP_F + lane - 4
+         : SP_Q + (lane == 0 ? Q_RP : lane == 4 ? Q_RT : lane == 5 ? Q_RY1 : lane == 6 ? Q_RY2 : lane == 11 ? Q_BETA : Q_RHO);
     // lanes 0..6: the column's factor in the energy row (h_p, u, v, w, h_T, h_y1, h_y2)
-    m.v2 = lane == 0 ? NB_DC + D_HP : lane <= 3 ? NB_PV + lane : lane == 4 ? NB_DC + D_HT : lane == 5 ? NB_DC + D_HY1 : NB_DC + D_HY2;
+    m.v2 = SP_Q + (lane == 0 ? Q_HP : lane <= 3 ? Q_U + lane - 1 : lane == 4 ? Q_HT : lane == 5 ? Q_HY1 : Q_HY2);
     // the row's own factor: pv(n), in the energy row the total enthalpy
-    m.p = lane == 4 ? NB_JC + 1 : lane < NPV ? NB_PV + lane : NB_PV;
+    // (lane 0 and the lanes without a row read one that they do not use)
+    m.p = SP_Q + (lane >= 1 && lane <= 3 ? Q_U + lane - 1 : lane == 4 ? Q_H : lane >= 5 && lane <= 8 ? Q_Y1 + lane - 5 : Q_U);
     // the row's entries of D^-1 (getx_apply): k1..k4, e1, e2, f1
     m.n0 = lane == 0; m.n4 = lane == 4; m.n5 = lane == 5; m.n7 = lane == 7; m.n8 = lane == 8;
     m.cpl = m.n0 || m.n4 || m.n5;
     const bool row7 = lane >= 7;
-    m.g[0] = ST_GX + (m.n0 ? GX_C4C1 : m.n4 ? GX_C4IB1S1 : m.n7 ? GX_RBT4 : m.n8 ? GX_RBT1 : GX_C4SSIB1);
-    m.g[1] = ST_GX + (m.n0 ? GX_C2 : m.n4 ? GX_C1 : m.n7 ? GX_T2 : m.n8 ? GX_T3 : GX_SS);
-    m.g[2] = ST_GX + (m.n0 ? GX_C3 : m.n4 ? GX_C3IB1 : GX_C1);
-    m.g[3] = ST_GX + (m.n0 ? GX_RB1 : GX_C2IB1);
-    m.g[4] = ST_GX + (m.n0 ? GX_CROSS1 : GX_S1P5);
-    m.g[5] = ST_GX + (m.n0 ? GX_CP5 : GX_SSY1);
-    m.g[6] = ST_GX + (m.cpl ? GX_MM : row7 ? GX_IT : GX_IB1);
+    m.g[0] = SP_GX + (m.n0 ? GX_C4C1 : m.n4 ? GX_C4IB1S1 : m.n7 ? GX_RBT4 : m.n8 ? GX_RBT1 : GX_C4SSIB1);
+    m.g[1] = SP_GX + (m.n0 ? GX_C2 : m.n4 ? GX_C1 : m.n7 ? GX_T2 : m.n8 ? GX_T3 : GX_SS);
+    m.g[2] = SP_GX + (m.n0 ? GX_C3 : m.n4 ? GX_C3IB1 : GX_C1);
+    m.g[3] = SP_GX + (m.n0 ? GX_RB1 : GX_C2IB1);
+    m.g[4] = SP_GX + (m.n0 ? GX_CROSS1 : GX_S1P5);
+    m.g[5] = SP_GX + (m.n0 ? GX_CP5 : GX_SSY1);
+    m.g[6] = SP_GX + (m.cpl ? GX_MM : row7 ? GX_IT : GX_IB1);
     // lanes 0, 1, 2: the three sums res0 a + b uuu + c res6 that rows 0, 4, 5 share
-    m.co[0] = ST_GX + (lane == 0 ? GX_AAA1 : lane == 1 ? GX_AAA2 : GX_SSHM);
-    m.co[1] = lane == 0 ? ST_DC + D_RY1 : lane == 1 ? ST_DC + D_RT : ST_GX + GX_RRR;
-    m.co[2] = ST_GX + (lane == 0 ? GX_CROSS : lane == 1 ? GX_CROSS2 : GX_SSY2);
+    m.co[0] = SP_GX + (lane == 0 ? GX_AAA1 : lane == 1 ? GX_AAA2 : GX_SSHM);
+    m.co[1] = lane == 0 ? SP_Q + Q_RY1 : lane == 1 ? SP_Q + Q_RT : SP_GX + GX_RRR;
+    m.co[2] = SP_GX + (lane == 0 ? GX_CROSS : lane == 1 ? GX_CROSS2 : GX_SSY2);
     const double hs = FWD ? 0.5 : -0.5;
     m.scale = lane == 7 || lane == 10 ? hs : (lane == 8 || lane == 9) ? 0.5 : 1.0;
     for (int l = 0; l < 7; l++) m.one[l] = lane == l ? 1.0 : 0.0;
@@ -969,14 +974,15 @@ __device__ __forceinline__ void row_apply(const double *c, double x, double &y)
 struct RowCell {
     double res, v1, v2, p, g[7], a, co[3];
 };
-template <class W> __device__ __forceinline__ RowCell row_cell(const RowMap &m, const W &st, int ln)
+// (st: the pencil's part of a slab)
+__device__ __forceinline__ RowCell row_cell(const RowMap &m, const double *st, int ln)
 {
     RowCell c;
-    c.res = st[ST_RES + ln];
-    c.v1 = st[ST_PV + m.v1]; c.v2 = st[ST_PV + m.v2]; c.p = st[ST_PV + m.p];
+    c.res = st[SP_RES + ln];
+    c.v1 = st[m.v1]; c.v2 = st[m.v2]; c.p = st[m.p];
 #pragma unroll
     for (int q = 0; q < 7; q++) c.g[q] = st[m.g[q]];
-    c.a = st[ST_GX + GX_A];
+    c.a = st[SP_GX + GX_A];
 #pragma unroll
     for (int q = 0; q < 3; q++) c.co[q] = st[m.co[q]];
     return c;
@@ -1023,38 +1029,19 @@ __device__ __forceinline__ void lds_barrier()
 // global address space: a pointer read back from LDS would otherwise be
 // generic, and generic loads also count against the LDS wait counter
 #define GLOBAL __attribute__((address_space(1)))
-constexpr int WIN = 4;               // cells of a stage window
-// one cell of a stage window: item e at stride WIN
-struct WinRow {
-    const double *p;
-    __device__ double operator[](int e) const { return p[e * WIN]; }
-};
-constexpr int SWEEP_THREADS = 256 + 64 + 64 + 64;   // 16 pencil groups of 16 lanes, a store, a poll and a loader wavefront
+constexpr int SWEEP_THREADS = 256 + 64 + 64;   // 16 pencil groups of 16 lanes, a poll and a loader wavefront
 constexpr int NEDGE = 2 * 4 * NPV;   // cross-tile dq values a tile reads per step: two edges of four pencils
-// Stage loads, by the loader wavefront, as LDS-DMA (global memory to LDS,
-// 16 bytes a lane, no registers).  A pencil at sweep distance d reads window
-// d >> 2 (its cell) and window (d + 1) >> 2 (the lookahead); while d & 3 is
-// 0, 1 or 2 both are window W = d >> 2 and the other buffer, window W + 1, is
-// free.  The loader issues quarters 0 and 1 of window W + 1 at d & 3 = 0 and
-// quarters 2 and 3 at d & 3 = 1, and waits for each step's transfers before
-// the barrier that ends the next step, so every transfer lands while its
-// buffer is free and window W + 1 is complete when it first becomes the
-// lookahead (d & 3 = 3).  A window's four cells lie in ascending i in LDS in
-// both sweeps, as the transfers copy them.
 static_assert(TJ == 4 && TK == 4, "the poll wavefront maps an edge of four pencils");
 
 // Division of labour inside a tile's workgroup:
 //  - four pencil wavefronts (16 groups of 16 lanes, lane = row) run the
-//    hyperplane steps; they read only LDS (their one global access is the
-//    store of a downstream-edge pencil's dq), so nothing they wait for is
-//    slower than LDS;
+//    hyperplane steps; they read only LDS and store their cells' results
+//    themselves, with no load in flight that a store could wait behind;
 //  - a poll wavefront reads, with device-coherent loads, the dq of the
 //    upstream cells in other tiles during the step before its use and hands
 //    it over through LDS (it is the only wavefront that waits on other tiles);
-//  - a store wavefront writes each hyperplane's dcv (forward) or dq
-//    (backward) one step later; the dq of the pencils on the tile's
-//    downstream edges the pencil wavefronts store as soon as they form it;
-//  - a loader wavefront fills the stage windows ahead of the pencils.
+//  - a loader wavefront fills the stage ahead of the pencils, by LDS-DMA
+//    (global memory to LDS, 16 bytes a lane, no registers).
 // A step's Jacobian coefficients are formed during the step before from its
 // stage without branching on the row, so the dependent chain of a step is
 // three row products, the exchange of y and D^-1.
@@ -1069,21 +1056,14 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
     __shared__ double hand[HZ + NPV];
     auto lds_at = [](int par, int g) { return (par * TJ * TK + g) * NPV; };
     auto xch_at = [](int par, int a, int g) { return HX + ((par * 2 + a) * TJ * TK + g) * NPV; };
-    auto lds = [&](int par, int g) { return hand + lds_at(par, g); };
     double *const zrow = hand + HZ;
-    // dcv of the last YR hyperplanes (forward sweep), by s mod YR: the store
-    // wavefront writes a pencil's dcv four cells at a time
-    constexpr int YR = 8;      // (five are needed; a power of two makes s mod YR a mask)
-    __shared__ double ylds[FWD ? YR : 1][TJ * TK][NPV];
-    __shared__ double win[2][TJ * TK][ST_N][WIN];   // stage windows (see the pencil wavefronts)
-    __shared__ const double *src[TJ * TK][ST_N];
+    __shared__ double stage[SLABS * SLAB_N];
     __shared__ int gave_up, taken;
     const int npv = S.npv;
     const int sg = FWD ? 1 : -1;
     double *const xq = FWD ? S.xqf : S.xqb;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 15, grp = (threadIdx.x >> 4) & 15;
-    constexpr int PER = ST_N / 16;                                  // stage items per lane
     if (threadIdx.x == 0) gave_up = 0;
     if (threadIdx.x < NPV) zrow[threadIdx.x] = 0.0;
     for (;;) {
@@ -1094,7 +1074,6 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
         if (tq >= ntiles) break;
         const int *td = tiles + 4 * (FWD ? tq : ntiles - 1 - tq);
         const BlkD B = S.b[td[0]];           // a copy: the loops read the block's extents from registers
-        const long NW = S.NW;
         const int j0 = td[1], k0 = td[2];
         const int jend = min(j0 + TJ - 1, B.J), kend = min(k0 + TK - 1, B.K);
         // the tile's hyperplane range in sweep order
@@ -1104,144 +1083,67 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
         auto down_edge = [](int g) {
             return FWD ? (g % TJ == TJ - 1 || g / TJ == TK - 1) : (g % TJ == 0 || g / TJ == 0);
         };
-        if (wave == 4) {
-            // store wavefront: hyperplane s is written out during step s+1,
-            // while the pencil wavefronts compute.  The dq that other tiles
-            // wait for (the pencils on the tile's downstream edges) the
-            // pencil wavefronts store themselves into the exchange array, as
-            // soon as it is formed.  Forward, dq is read by nothing else (the
-            // backward sweep starts from dcv), so only dcv is written, a
-            // pencil's four cells of a stage window (or its last few)
-            // together and non-temporal (the backward sweep reads them after
-            // this launch); backward, the exchange array also takes the other
-            // pencils' dq, the update's input.
-            // The store wavefront shares its SIMD with a pencil wavefront: the
-            // step-independent part of its index arithmetic is done once per
-            // tile (a pencil's row advances by one cell a step).
-            const int l = threadIdx.x - 256;
-            long at[3], from[3];
-            int lo[3], hi[3];
+        if (wave == 5) {
+            // Loader wavefront.  Slab n holds hyperplane sa + sg n, slabs from
+            // -1 (all pencils before their first cell).  A step n reads slabs
+            // n and n + 1; during it slab n + SLABS - 1 is issued, into the
+            // place of slab n - 1, which the barrier that ended step n - 1
+            // freed, and before its end slab n + 2 has landed: of the slabs
+            // issued, the last SLABS - 3 may still be on their way.
+            // Lane and transfer (16 bytes) to piece of a record: the 37 pieces
+            // of a pencil, F then Q, GX and RES; the 12 of an edge neighbour.
+            // A pencil outside the block, and a cell before or past a
+            // pencil's ends, is a record of the zero outer layer.
+            const int l = threadIdx.x - 320;
+            const double *base[SLAB_LOADS];      // the piece in the record of i = 1 of its pencil
+            int off[SLAB_LOADS];                 // the cell of hyperplane s is i = 1 + s - off
 #pragma unroll
-            for (int q = 0; q < 3; q++) {
-                const int v = l + 64 * q;
-                if constexpr (FWD) {
-                    // dcv of row n, cell (i - 3 + c, j0 + p, k0 + gk): at + i + gk * from
-                    const int p = v / (4 * NPV), n = (v >> 2) % NPV, c = v & 3;
-                    at[q] = n * NW + widx(B, c - 3, j0 + p, k0);
-                    from[q] = (long)(B.I + 1) * (B.J + 1);
-                    lo[q] = hi[q] = 0;
+            for (int t = 0; t < SLAB_LOADS; t++) {
+                const int u = 64 * t + l, F = FWD ? RC_FP : RC_FM;
+                int jj, kk, jn, kn, q;
+                if (u < TJ * TK * SP_N / 2) {
+                    const int g = u / (SP_N / 2), c = u % (SP_N / 2);
+                    jj = jn = j0 + g % TJ;
+                    kk = kn = k0 + g / TJ;
+                    q = 2 * c < SP_Q ? F + 2 * c : RC_Q + 2 * c - SP_Q;
                 } else {
-                    // row n of pencil g at hyperplane s: at + 9 s, for lo <= s <= hi
-                    const int g = min(v / NPV, TJ * TK - 1), n = v % NPV, jj = j0 + g % TJ, kk = k0 + g / TJ;
-                    const bool on = v < TJ * TK * NPV && n < npv && jj <= jend && kk <= kend && !down_edge(g);
-                    at[q] = widx(B, -jj - kk, jj, kk) * NPV + n;
-                    lo[q] = on ? 2 + jj + kk : 1;
-                    hi[q] = on ? B.I + jj + kk : 0;
-                    from[q] = g * NPV + n;
+                    const int v = u - TJ * TK * SP_N / 2, e = min(v / (SE_N / 2), TJ + TK - 1), c = v % (SE_N / 2);
+                    const bool a = e >= TK;      // a k neighbour
+                    jj = j0 + (a ? e - TK : FWD ? 0 : TJ - 1);
+                    kk = k0 + (!a ? e : FWD ? 0 : TK - 1);
+                    jn = a ? jj : jj - sg;
+                    kn = a ? kk - sg : kk;
+                    q = 2 * c < SE_Q ? F + 6 * (a ? 2 : 1) + 2 * c : RC_Q + 2 * c - SE_Q;
                 }
+                base[t] = S.img + widx(B, 1, min(jn, B.J + 1), min(kn, B.K + 1)) * RC_N + q;
+                off[t] = jj + kk + 1;
             }
-            auto publish = [&](int s) {
-                if constexpr (FWD) {
-                    // the four pencils whose window closes at hyperplane s
-                    // (j + k = s - 5 mod 4) write its four cells, formed at
-                    // hyperplanes s - 3 .. s; lane -> (pencil, row, cell), so
-                    // that four adjacent lanes write one row's 32 bytes
-                    const int r0 = (s - j0 - k0 - 5) & 3;
+            const int BI = B.I;
+            auto issue = [&](int s, int slot) {
 #pragma unroll
-                    for (int q = 0; q < 3; q++) {
-                        const int v = l + 64 * q, p = v / (4 * NPV), n = (v >> 2) % NPV, c = v & 3;
-                        // the class's pencil with gj = p: gj + gk = r0, or r0 + 4 past the tile's anti-diagonal
-                        const int gk = r0 + 4 * (p > r0) - p, i = s - j0 - k0 - p - gk;
-                        if (v < 4 * NPV * 4 && n < npv && j0 + p <= jend && k0 + gk <= kend && i >= 5 && i <= B.I)
-                            __builtin_nontemporal_store(ylds[(s - 3 + c) & (YR - 1)][p + TJ * gk][n], S.dcv + at[q] + (i + (long)gk * from[q]));
-                    }
-                    // a pencil that ends at hyperplane s in the middle of a window
-                    if (s >= B.I + j0 + k0) {
-                        for (int e = l; e < TJ * TK * NPV; e += 64) {
-                            const int g = e / NPV, n = e - g * NPV;
-                            const int jj = j0 + g % TJ, kk = k0 + g / TJ, i = s - jj - kk;
-                            const int m = (i - 2) & 3;
-                            if (n < npv && i == B.I && m != 3 && jj <= jend && kk <= kend) {
-                                double *o = S.dcv + n * NW + widx(B, i - m, jj, kk);
-                                for (int c = 0; c <= m; c++) __builtin_nontemporal_store(ylds[(s - m + c) & (YR - 1)][g][n], o + c);
-                            }
-                        }
-                    }
-                } else {
-#pragma unroll
-                    for (int q = 0; q < 3; q++)
-                        if (s >= lo[q] && s <= hi[q]) xq[at[q] + (long)s * NPV] = hand[(s & 1) * TJ * TK * NPV + (int)from[q]];
+                for (int t = 0; t < SLAB_LOADS; t++) {
+                    const unsigned i = (unsigned)min(max(s - off[t], 0), BI);
+                    __builtin_amdgcn_global_load_lds((const GLOBAL void *)(base[t] + (unsigned long)i * RC_N),
+                                                     (__attribute__((address_space(3))) void *)&stage[slot * SLAB_N + 128 * t],
+                                                     16, 0, 0);
                 }
             };
-            __syncthreads();
-            for (int s = sa;; s += sg) {
-                if (s != sa) publish(s - sg);
-                lds_barrier();
-                if (s == sb) break;
+            // SLABS - 3 slabs of SLAB_LOADS transfers may be outstanding
+            static_assert(SLAB_LOADS == 11 && SLABS == 6, "the wait below");
+            issue(sa - sg, SLABS - 1);
+#pragma unroll
+            for (int n = 0; n < SLABS - 1; n++) {
+                if (n == 3) asm volatile("s_waitcnt vmcnt(33)" ::: "memory");   // (the counter holds 63)
+                issue(sa + sg * n, n);
             }
-            publish(sb);
-            if (gave_up && threadIdx.x == 256) atomicOr(err, 1);
+            asm volatile("s_waitcnt vmcnt(33)" ::: "memory");
             __syncthreads();
-            continue;
-        }
-        if (wave == 6) {
-            // loader wavefront: in a step, the eight pencils with d & 3 = 0
-            // or 1 each get two quarters (32 items x 4 cells, 1 KB each) of
-            // their next window, one 16-byte transfer a lane per quarter:
-            // lane L moves item L / 2, cells 2 (L & 1) and 2 (L & 1) + 1.
-            // The pencils' prologue fills window 0 and the source table is
-            // theirs, so the loader starts after the first barrier.
-            const int l = threadIdx.x - 384, li = l >> 1, lc = 2 * (l & 1);
-            const int BI = B.I;
             __syncthreads();
-            int d0 = FWD ? sa - j0 - k0 - 2 : BI - (sa - j0 - k0);      // distance of pencil 0 (it grows by one a step)
+            int slot = SLABS - 1;
             for (int s = sa;; s += sg) {
-                // the transfers are issued at once (issuing sixteen of them
-                // takes longer than the poll wavefront's two reads; holding
-                // them back behind those reads cost 10 us a sweep)
-                if (s != sb) {
-                    // the eight pencils with d & 3 = e in {0, 1}: four per
-                    // class, pencil p of a class at gj = p on the class's
-                    // anti-diagonals t = c, c + 4 (no branch between them, so
-                    // the pointer reads can be issued ahead of the transfers
-                    // that use them, not each waited for in turn)
-                    const double *pp[2][4][2];
-                    int gg[2][4], ww[2][4];
-#pragma unroll
-                    for (int e = 0; e < 2; e++) {
-                        const int c = (FWD ? d0 - e : e - d0) & 3;
-#pragma unroll
-                        for (int p = 0; p < 4; p++) {
-                            const int t = c + 4 * (p > c), g = p + TJ * (t - p);
-                            const int d = FWD ? d0 - t : d0 + t;
-                            gg[e][p] = g;
-                            ww[e][p] = (d >> 2) + 1;
-#pragma unroll
-                            for (int h = 0; h < 2; h++) pp[e][p][h] = src[g][32 * (2 * e + h) + li];
-                        }
-                    }
-#pragma unroll
-                    for (int e = 0; e < 2; e++) {
-#pragma unroll
-                        for (int p = 0; p < 4; p++) {
-                            const int g = gg[e][p], w1 = ww[e][p];
-                            // first cell of the lane's pair; a pair that lies
-                            // beyond the pencil is clamped to cells 1..I+1 (its
-                            // slots hold no cell of the pencil)
-                            const int c0 = min(max((FWD ? 2 + 4 * w1 : BI - 4 * w1 - 3) + lc, 1), BI);
-#pragma unroll
-                            for (int h = 0; h < 2; h++) {
-                                const int q = 2 * e + h;
-                                __builtin_amdgcn_global_load_lds((const GLOBAL void *)(pp[e][p][h] + c0),
-                                                                 (__attribute__((address_space(3))) void *)&win[w1 & 1][g][32 * q][0],
-                                                                 16, 0, 0);
-                            }
-                        }
-                    }
-                }
-                d0++;
-                // the transfers of the previous step have landed (16 issued since)
-                asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+                issue(s + sg * (SLABS - 1), slot);
+                slot = slot == SLABS - 1 ? 0 : slot + 1;
+                asm volatile("s_waitcnt vmcnt(33)" ::: "memory");
                 lds_barrier();
                 if (s == sb) break;
             }
@@ -1249,11 +1151,11 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             __syncthreads();
             continue;
         }
-        if (wave == 5) {
+        if (wave == 4) {
             // poll wavefront: item q = lane, lane + 64 of the 72 edge values
             // (edge a = q / 36: the j (a = 0) or k (a = 1) neighbours; pencil
             // e = q / 9 % 4 along the edge; row n = q % 9)
-            const int l64 = threadIdx.x - 320;
+            const int l64 = threadIdx.x - 256;
             const double *dummy = xq + widx(B, min(max(sa - j0 - k0, 2), B.I), j0, k0) * NPV;
             // per lane and tile: item t's value of step s is at xq[at + 9 s],
             // read for lo <= s <= hi (the cell is inside the block and its
@@ -1306,6 +1208,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             issue(sa);
             deliver(sa);
             __syncthreads();
+            __syncthreads();
             for (int s = sa;; s += sg) {
                 // the next step's values are read at the start of this step,
                 // while the pencils compute, as late as they can be
@@ -1314,6 +1217,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
                 lds_barrier();
                 if (s == sb) break;
             }
+            if (gave_up && l64 == 0) atomicOr(err, 1);
             __syncthreads();
             continue;
         }
@@ -1329,56 +1233,36 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
         const int jm = j - sg, km = k - sg;
         const bool lj = jm >= j0 && jm <= jend, lk = km >= k0 && km <= kend;
         const bool nj = jm >= 2 && jm <= B.J, nk = km >= 2 && km <= B.K;   // neighbour inside the block
-        // where the stage items come from: item e of cell i is src[grp][e][i]
-        // (the zero array for items a pencil does not read)
-#pragma unroll
-        for (int r = 0; r < PER; r++) {
-            const double *q = live ? stage_base<FWD>(S, B, j, k, lane + 16 * r) : nullptr;
-            src[grp][lane + 16 * r] = q ? q : S.zero;
-        }
-        // Stage windows: window m holds cells at sweep distance 4m..4m+3 of
-        // the pencil (distance d = i - 2 forward, I - i backward), item-major
-        // with the four cells adjacent, in LDS buffer m & 1.  Four adjacent
-        // lanes load one item's four cells (one cache line between them).
-        // The pencils fill window 0 here; the loader wavefront fills the
-        // rest during the steps.
-        const int l4 = lane >> 2, c4 = lane & 3;
-        auto wcell = [&](int m, int c) { return FWD ? 2 + 4 * m + c : BI - 4 * m - 3 + c; };
-        auto slot = [](int dd) { return FWD ? (dd & 3) : 3 - (dd & 3); };     // the cell at distance dd in its window
-        auto fetchq = [&](int m, int qq, double *v) {
-            const int ic = min(max(wcell(m, c4), 2), BI);
-#pragma unroll
-            for (int r = 0; r < 8; r++) v[r] = ((const GLOBAL double *)src[grp][32 * qq + 4 * r + l4])[ic];
-        };
-        auto putq = [&](int m, int qq, const double *v) {
-#pragma unroll
-            for (int r = 0; r < 8; r++) win[m & 1][grp][32 * qq + 4 * r + l4][c4] = v[r];
-        };
-        // prologue: window 0 complete, window -1's buffer zeroed (steps before
-        // the pencil's first cell read it)
-        for (int qq = 0; qq < 4; qq++) {
-            double v[8];
-            fetchq(0, qq, v);
-            putq(0, qq, v);
-        }
-        for (int e = lane; e < ST_N * WIN; e += 16) (&win[1][grp][0][0])[e] = 0.0;
-        const int d0 = FWD ? sa - j - k - 2 : BI - (sa - j - k);
-        if (lane < NPV) lds((sa - sg) & 1, grp)[lane] = 0.0;       // the first step's upstream reads zeros
+        // The stage items of the j and k neighbours: a neighbour pencil of the
+        // tile holds its cell in the slab of this step (it is one hyperplane
+        // ahead), an edge neighbour in its own place of the next one's.
+        const bool ej = gj == (FWD ? 0 : TJ - 1), ek = gk == (FWD ? 0 : TK - 1);
+        const int pj = ej ? SLAB_E + gk * SE_N : (grp - sg) * SP_N, pk = ek ? SLAB_E + (TK + gj) * SE_N : (grp - sg * TJ) * SP_N;
+        const int qj = ej ? SE_Q - SP_Q : 0, qk = ek ? SE_Q - SP_Q : 0;
+        const int j1 = pj + rows.v1 + (rows.face ? (ej ? 0 : 6) : qj), j2 = pj + rows.v2 + qj, jp = pj + rows.p + qj;
+        const int k1 = pk + rows.v1 + (rows.face ? (ek ? 0 : 12) : qk), k2 = pk + rows.v2 + qk, kp = pk + rows.p + qk;
+        double *out = FWD ? S.img + (widx(B, 1, min(j, B.J), min(k, B.K)) * RC_N + RC_RES + lane)
+                          : xq + (widx(B, 1, min(j, B.J), min(k, B.K)) * NPV + lane);
+        double *const xe = xq + (widx(B, 1, min(j, B.J), min(k, B.K)) * NPV + lane);
+        if (lane < NPV) hand[lds_at((sa - sg) & 1, grp) + lane] = 0.0;       // the first step's upstream reads zeros
         double ci[8], cj[8], ck[8];                                  // coefficients of the coming step
         RowCell own;                                                 // its cell
+        int cur = (SLABS - 1) * SLAB_N, nxt = 0;                     // slabs of this step and the next
+        __syncthreads();
 #pragma unroll
         for (int q = 0; q < 8; q++) ci[q] = 0.0;
         {
-            const WinRow s0{&win[(d0 >> 2) & 1][grp][0][slot(d0)]};
-            row_coef<FWD>(rows, s0[ST_J + rows.v1], s0[ST_J + rows.v2], s0[ST_J + rows.p], cj);
-            row_coef<FWD>(rows, s0[ST_K + rows.v1], s0[ST_K + rows.v2], s0[ST_K + rows.p], ck);
-            own = row_cell(rows, s0, ln);
+            const double *const sj = stage + (ej ? nxt : cur), *const sk = stage + (ek ? nxt : cur);
+            row_coef<FWD>(rows, sj[j1], sj[j2], sj[jp], cj);
+            row_coef<FWD>(rows, sk[k1], sk[k2], sk[kp], ck);
+            own = row_cell(rows, stage + nxt + grp * SP_N, ln);
         }
         __syncthreads();
         for (int s = sa;; s += sg) {
             const int i = s - j - k;
-            const int d = FWD ? i - 2 : BI - i;
             const bool act = live && i >= 2 && i <= BI;
+            cur = nxt;
+            nxt = nxt == (SLABS - 1) * SLAB_N ? 0 : nxt + SLAB_N;
             // dq of the three upstream neighbours: in the tile from the
             // previous hyperplane, from another tile through the poll wavefront
             const int pb = (s - sg) & 1;
@@ -1397,23 +1281,27 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             // dq = D^-1 dcv
             const double xn = row_dinv(rows, own, y);
             if (lane < NPV) {
-                lds(s & 1, grp)[lane] = act ? xn : 0.0;
-                if constexpr (FWD) ylds[s & (YR - 1)][grp][lane] = y;
-                // the pencil wavefronts have no loads in flight, so this store
-                // costs only its issue
-                if (edge && act && mine) st_dev(xq + widx(B, i, j, k) * NPV + lane, xn);
+                hand[lds_at(s & 1, grp) + lane] = act ? xn : 0.0;
+                // the dq that other tiles wait for goes out at once.  Forward,
+                // no other dq is read again (the backward sweep starts from
+                // dcv); backward, every cell's is the update's input
+                if (act && mine) {
+                    if (edge) st_dev(xe + (i - 1) * NPV, xn);
+                    if constexpr (FWD) out[(long)(i - 1) * RC_N] = y;
+                    else if (!edge) out[(i - 1) * NPV] = xn;
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
             // coefficients of the next step (independent of dq): this cell's
             // row through its face to the next cell, and the j / k neighbours
             // of the next cell; and the next cell's own terms
-            const WinRow s1{&win[((d + 1) >> 2) & 1][grp][0][slot(d + 1)]};
-            const double j1 = s1[ST_J + rows.v1], j2 = s1[ST_J + rows.v2], jp = s1[ST_J + rows.p];
-            const double k1 = s1[ST_K + rows.v1], k2 = s1[ST_K + rows.v2], kp = s1[ST_K + rows.p];
+            const double *const sj = stage + (ej ? nxt : cur), *const sk = stage + (ek ? nxt : cur);
+            const double vj1 = sj[j1], vj2 = sj[j2], vjp = sj[jp];
+            const double vk1 = sk[k1], vk2 = sk[k2], vkp = sk[kp];
             row_coef<FWD>(rows, own.v1, own.v2, own.p, ci);
-            row_coef<FWD>(rows, j1, j2, jp, cj);
-            row_coef<FWD>(rows, k1, k2, kp, ck);
-            own = row_cell(rows, s1, ln);
+            row_coef<FWD>(rows, vj1, vj2, vjp, cj);
+            row_coef<FWD>(rows, vk1, vk2, vkp, ck);
+            own = row_cell(rows, stage + nxt + grp * SP_N, ln);
             // formed before the barrier (while the poll wavefront may still be
             // waiting), not after it on the next step's path
 #pragma unroll
@@ -1690,19 +1578,13 @@ struct cav3d_ctx {
 
 namespace {
 
-// Every device array carries DPAD zeroed bytes before and after it: the
-// sweeps' stage transfers move cells in pairs and may read one element past
-// either end of an array.
-constexpr size_t DPAD = 256;
 template <class T> int dalloc(cav3d_ctx *c, T **p, size_t n)
 {
     *p = nullptr;
     if (n == 0) n = 1;
-    char *raw = nullptr;
-    HIPCHK(hipMalloc((void **)&raw, n * sizeof(T) + 2 * DPAD));
-    HIPCHK(hipMemsetAsync(raw, 0, n * sizeof(T) + 2 * DPAD, c->st));
-    c->allocs.push_back(raw);
-    *p = (T *)(raw + DPAD);
+    HIPCHK(hipMalloc((void **)p, n * sizeof(T)));
+    c->allocs.push_back(*p);
+    HIPCHK(hipMemsetAsync(*p, 0, n * sizeof(T), c->st));
     return 0;
 }
 
@@ -2183,7 +2065,7 @@ int cav3d_create(const cav3d_params *prm, int nblocks, const cav3d_block *blocks
     if ((rc = dalloc(c, &S.pv, npv * S.NG)) || (rc = dalloc(c, &S.dc, (long)ND * S.NG)) ||
         (rc = dalloc(c, &S.vol, S.NW)) || (rc = dalloc(c, &c->xc, 3 * S.NW)) || (rc = dalloc(c, &S.cx, 3 * S.NCX)) || (rc = dalloc(c, &S.ex, 3 * S.NEX)) ||
         (rc = dalloc(c, &S.tx, 3 * S.NTX)) || (rc = dalloc(c, &S.res, npv * S.NC)) || (rc = dalloc(c, &S.dt, S.NC)) ||
-        (rc = dalloc(c, &S.dcv, npv * S.NW)) ||
+        (rc = dalloc(c, &S.img, (long)RC_N * S.NW)) ||
         (rc = dalloc(c, &S.xqf, (long)NPV * S.NW)) || (rc = dalloc(c, &S.xqb, (long)NPV * S.NW)) ||
         (rc = dalloc(c, &S.scal, 32))) { cav3d_destroy(c); return rc; }
     for (int d = 0; d < 3; d++)
@@ -2198,10 +2080,6 @@ int cav3d_create(const cav3d_params *prm, int nblocks, const cav3d_block *blocks
     if (prm->nsteady > 0) {
         if ((rc = dalloc(c, &S.qq, 2 * npv * S.NC))) { cav3d_destroy(c); return rc; }
     }
-    int maxi = 0;
-    for (int b = 0; b < nblocks; b++) maxi = std::max(maxi, c->blk[b].I);
-    if ((rc = dalloc(c, &S.gx, (long)NGX * S.NC)) || (rc = dalloc(c, &S.jc, 2 * S.NC)) ||
-        (rc = dalloc(c, &S.jf, 18 * S.NC)) || (rc = dalloc(c, &S.zero, maxi + 8))) { cav3d_destroy(c); return rc; }
     {
         // tile table: TJ x TK pencil tiles of every block, ordered by the tile
         // diagonal tj + tk (the forward sweep takes them in this order, the
