@@ -729,8 +729,9 @@ __global__ __launch_bounds__(256) void k_combine(DS S)
 // of 92 doubles (736 bytes, 46 pieces of 16), ranges and order of the dcv
 // array of the reference (1:I+1 and so on; the outer layer stays zero and is
 // what a pencil's absent neighbours read):
-//   RC_FP, RC_FM  the +i,+j,+k (-i,-j,-k) faces x (n3[3], u, lam, vis): the
-//                 forward (backward) sweep's split Jacobians
+//   RC_FP, RC_FM  the +i,+j,+k (-i,-j,-k) faces x (+-n3[3], +-u, lam, vis) / 2:
+//                 the forward (backward) sweep's split Jacobians with their
+//                 sign and factor (exact: a power of two)
 //   RC_Q          the Jacobian's cell terms, in both sweeps
 //   RC_GX         the diagonal-inverse terms
 //   RC_RES        the residual; the forward sweep puts its dcv there
@@ -774,8 +775,9 @@ __global__ __launch_bounds__(128) void k_lhs_prep(DS S)
     for (int q = 0; q < 6; q++) {
         const JacFace f = jac_face(P, cc, f6[q]);
         double *o = r + ((q & 1) ? RC_FP : RC_FM) + 6 * (q >> 1);
-        o[0] = f6[q][0]; o[1] = f6[q][1]; o[2] = f6[q][2];
-        o[3] = f.u; o[4] = f.lam; o[5] = f.vis;
+        const double h = (q & 1) ? 0.5 : -0.5;
+        o[0] = h * f6[q][0]; o[1] = h * f6[q][1]; o[2] = h * f6[q][2];
+        o[3] = h * f.u; o[4] = 0.5 * f.lam; o[5] = 0.5 * f.vis;
     }
     const JacCell jc = jac_cell(P, cc);
     double *const c = r + RC_Q;
@@ -851,15 +853,18 @@ constexpr int TJ = 4, TK = 4;
 // LDS stage of one hyperplane (doubles): the tile's sixteen pencils, each its
 // cell's F (the sweep's side), Q, GX and RES; then the upstream neighbours in
 // other tiles of the four j-edge and the four k-edge pencils, each the F of
-// its face towards the tile and its Q.  A ring of SLABS hyperplanes: a step
-// reads its own and the next one's while the ones after are on their way.
+// its face towards the tile and its Q (those the next hyperplane's cells
+// read, so that every neighbour is in the slab of the step before the one
+// that uses it).  A ring of SLABS hyperplanes: a step reads its own slab and
+// the next one while the ones after are on their way.  The steps are unrolled
+// over the ring, so that the places are constants of the LDS reads.
 enum {
     SP_F = 0, SP_Q = 18, SP_GX = 36, SP_RES = SP_GX + NGX, SP_N = SP_RES + NPV,
     SE_F = 0, SE_Q = 6, SE_N = 24,
     SLAB_E = TJ * TK * SP_N, SLAB_USED = SLAB_E + (TJ + TK) * SE_N,
     SLAB_LOADS = (SLAB_USED + 127) / 128, SLAB_N = 128 * SLAB_LOADS
 };
-constexpr int SLABS = 6;
+constexpr int SLABS = 5;
 static_assert(SP_N == RC_N - 18 && SP_RES - SP_GX == RC_RES - RC_GX && SP_GX - SP_Q == RC_GX - RC_Q, "stage layout");
 
 // lane q of the lane's 16-lane row, by one 64-bit DPP move (no LDS traffic)
@@ -872,32 +877,37 @@ __device__ __forceinline__ double row_lane(double v)
 // cell's system; everything else a step reads (the state, properties, face
 // and diagonal-inverse terms: some 90 numbers a cell) is the same for all
 // lanes.  The lanes read them from the stage one item each (lane l its own
-// item, RowMap) and pass them around with DPP row broadcasts.  Reading every
+// items, RowMap) and pass them around with DPP row broadcasts.  Reading every
 // item into every lane took 140 LDS reads a step, whose return path (each
 // read brings 64 lanes x 8 bytes at 128 bytes a clock for the four pencil
-// wavefronts of the CU) bound the step: without any coefficient reads
-// the 64x32x32 sweep fell from 268 to 171 us.  Now 24 reads, and
-// the terms that are one expression per column are formed once, a column per
-// lane, not in every lane.
+// wavefronts of the CU) bound the step.  Now it is 39, and the terms that are
+// one expression per column are formed once, a column per lane, not in every
+// lane.  What a lane needs another operand for than its neighbours it reads
+// from another place rather than selecting among broadcasts.
 struct RowMap {
-    int v1, v2, p, g[7], co[3];     // stage items of this lane, within its pencil's part of a slab
-    bool face;                      // v1 is one of F (of the i face; the j and k faces' lie 6 and 12 further)
-    double scale;                   // of v1: the sweep's sign and the factor 0.5 on u, lam, vis, rho
+    int v1, a, lb, v2, p, g[7], co[3];     // stage items of this lane, within its pencil's part of a slab
+    bool face, aface;               // v1 (and lb), a: items of F (of the i face; the j and k faces' lie 6 and 12 further)
     double one[7];                  // 1 in the lane of the column
-    bool mom, en, kw, cpl, n0, n4, n5, n7, n8;
+    double en, kw, men, mom;        // 1 in lane 4, 1 in the lanes of k and omega, -1 in lane 4, 1 in lanes 1..3
+    bool m13, cpl, n0, n4, n5, n7, n8;
 };
-template <bool FWD> __device__ __forceinline__ RowMap row_map(int lane, int npv)
+__device__ __forceinline__ RowMap row_map(int lane, int npv)
 {
     RowMap m;
-    // lanes 0..6: the column's factor of r1 (rho_p, n3, rho_T, rho_y1, rho_y2); then u, lam, vis, rho (scaled), beta, rho
-    m.face = (lane >= 1 && lane <= 3) || (lane >= 7 && lane <= 9);
-    m.v1 = lane >= 1 && lane <= 3 ? SP_F + lane - 1 : lane >= 7 && lane <= 9 ? SP_F + lane - 4
-         : SP_Q + (lane == 0 ? Q_RP : lane == 4 ? Q_RT : lane == 5 ? Q_RY1 : lane == 6 ? Q_RY2 : lane == 11 ? Q_BETA : Q_RHO);
+    m.m13 = lane >= 1 && lane <= 3;
+    // lanes 0..6: the column's factor of r1 (rho_p, n3, rho_T, rho_y1, rho_y2); lane 13: rho
+    m.face = m.m13;
+    m.v1 = m.m13 ? SP_F + lane - 1 : SP_Q + (lane == 0 ? Q_RP : lane == 4 ? Q_RT : lane == 5 ? Q_RY1 : lane == 6 ? Q_RY2 : Q_RHO);
+    // u, followed by lam and vis; in lanes 1..3 rho
+    m.aface = !m.m13;
+    m.a = m.m13 ? SP_Q + Q_RHO : SP_F + 3;
+    // the factor of lam: in lane 0 beta, else that of u and vis
+    m.lb = lane == 0 ? SP_Q + Q_BETA : m.v1;
     // lanes 0..6: the column's factor in the energy row (h_p, u, v, w, h_T, h_y1, h_y2)
     m.v2 = SP_Q + (lane == 0 ? Q_HP : lane <= 3 ? Q_U + lane - 1 : lane == 4 ? Q_HT : lane == 5 ? Q_HY1 : Q_HY2);
     // the row's own factor: pv(n), in the energy row the total enthalpy
     // (lane 0 and the lanes without a row read one that they do not use)
-    m.p = SP_Q + (lane >= 1 && lane <= 3 ? Q_U + lane - 1 : lane == 4 ? Q_H : lane >= 5 && lane <= 8 ? Q_Y1 + lane - 5 : Q_U);
+    m.p = SP_Q + (m.m13 ? Q_U + lane - 1 : lane == 4 ? Q_H : lane >= 5 && lane <= 8 ? Q_Y1 + lane - 5 : Q_U);
     // the row's entries of D^-1 (getx_apply): k1..k4, e1, e2, f1
     m.n0 = lane == 0; m.n4 = lane == 4; m.n5 = lane == 5; m.n7 = lane == 7; m.n8 = lane == 8;
     m.cpl = m.n0 || m.n4 || m.n5;
@@ -913,46 +923,46 @@ template <bool FWD> __device__ __forceinline__ RowMap row_map(int lane, int npv)
     m.co[0] = SP_GX + (lane == 0 ? GX_AAA1 : lane == 1 ? GX_AAA2 : GX_SSHM);
     m.co[1] = lane == 0 ? SP_Q + Q_RY1 : lane == 1 ? SP_Q + Q_RT : SP_GX + GX_RRR;
     m.co[2] = SP_GX + (lane == 0 ? GX_CROSS : lane == 1 ? GX_CROSS2 : GX_SSY2);
-    const double hs = FWD ? 0.5 : -0.5;
-    m.scale = lane == 7 || lane == 10 ? hs : (lane == 8 || lane == 9) ? 0.5 : 1.0;
     for (int l = 0; l < 7; l++) m.one[l] = lane == l ? 1.0 : 0.0;
-    m.mom = lane >= 1 && lane <= 3;
-    m.en = lane == 4;
-    m.kw = row7 && lane < npv;
+    m.en = m.one[4]; m.men = -m.one[4];
+    m.mom = m.m13 ? 1.0 : 0.0;
+    m.kw = row7 && lane < npv ? 1.0 : 0.0;
     return m;
 }
+
+// A lane's Jacobian items of a cell and face (RowMap): v1, u (rho in lanes
+// 1..3), lam, vis, the factor of lam, v2, p
+struct RowJac {
+    double v1, a, b, c, lb, v2, p;
+};
 
 // Row coefficients of one neighbour's split Jacobian, c[l] = +-0.5 a(n,l)
 // (jac_row's products and sums in its order; jac_row_coef has the same row by
 // row): r1[l] and the energy row's factor of column l sit in lane l.  The
-// factor 0.5 and the sign are put on u, lam, vis, rho and n3, which they pass
-// through exactly; rho u goes onto the diagonal as fma(rho u, 1 or 0, a),
-// which rounds as the sum.
-template <bool FWD>
-__device__ __forceinline__ void row_coef(const RowMap &m, double v1, double v2, double p, double *c)
+// factor 0.5 and the sign are in u, lam, vis and n3 already, which they pass
+// through exactly.  A term that only some rows have is added as
+// fma(term, 1 or 0, sum), which rounds as the sum.
+__device__ __forceinline__ void row_coef(const RowMap &m, const RowJac &j, double *c)
 {
-    constexpr double hs = FWD ? 0.5 : -0.5;
-    const double n3n = hs * v1;
-    v1 = m.scale * v1;
-    const double u = row_lane<7>(v1), lam = row_lane<8>(v1), vis = row_lane<9>(v1);
-    // (the broadcasts stay out of the selects: they need every lane active)
-    const double rhos = row_lane<10>(v1), beta = row_lane<11>(v1);
-    const double lb = m.n0 ? beta : v1;
-    const double t = u * v1 + lam * lb + vis * v1, r = m.mom ? v1 * rhos : t;
-    const double ru = row_lane<13>(v1) * (u + lam + vis);
-    const double P = m.n0 ? 1.0 : p, Q = m.en ? ru : 0.0;
-    c[0] = P * row_lane<0>(r) + Q * row_lane<0>(v2);
-    c[1] = P * row_lane<1>(r) + Q * row_lane<1>(v2);
-    c[2] = P * row_lane<2>(r) + Q * row_lane<2>(v2);
-    c[3] = P * row_lane<3>(r) + Q * row_lane<3>(v2);
-    c[4] = P * row_lane<4>(r) + Q * row_lane<4>(v2);
-    c[5] = P * row_lane<5>(r) + Q * row_lane<5>(v2);
-    c[6] = P * row_lane<6>(r) + Q * row_lane<6>(v2);
-    c[0] = c[0] + (m.en ? -lam : (m.mom ? n3n : 0.0));
-    c[0] = c[0] + (m.en ? -vis : 0.0);
+    const double t0 = j.a * j.v1, t = t0 + j.b * j.lb + j.c * j.v1, r = m.m13 ? t0 : t;
+    // (lane 13 holds rho, u, lam and vis; the broadcasts stay out of the
+    // selects: they need every lane active)
+    const double ru = row_lane<13>(j.v1 * (j.a + j.b + j.c));
+    const double P = m.n0 ? 1.0 : j.p, Q = ru * m.en;
+    c[0] = P * row_lane<0>(r) + Q * row_lane<0>(j.v2);
+    c[1] = P * row_lane<1>(r) + Q * row_lane<1>(j.v2);
+    c[2] = P * row_lane<2>(r) + Q * row_lane<2>(j.v2);
+    c[3] = P * row_lane<3>(r) + Q * row_lane<3>(j.v2);
+    c[4] = P * row_lane<4>(r) + Q * row_lane<4>(j.v2);
+    c[5] = P * row_lane<5>(r) + Q * row_lane<5>(j.v2);
+    c[6] = P * row_lane<6>(r) + Q * row_lane<6>(j.v2);
+    // the pressure column: n3 in the momentum rows, -lam, then -vis in the energy row
+    c[0] = fma(j.v1, m.mom, c[0]);
+    c[0] = fma(j.b, m.men, c[0]);
+    c[0] = fma(j.c, m.men, c[0]);
 #pragma unroll
     for (int l = 1; l < 7; l++) if (l != 4) c[l] = fma(ru, m.one[l], c[l]);
-    c[7] = m.kw ? ru : 0.0;
+    c[7] = ru * m.kw;
 }
 
 // y += c x, the neighbour's row n in lane n (jac_row_apply)
@@ -969,24 +979,11 @@ __device__ __forceinline__ void row_apply(const double *c, double x, double &y)
 }
 
 // What a step reads of its own cell, read during the step before: the rows'
-// residual, the Jacobian items of its block (v1, v2, p as row_coef), the
-// rows' D^-1 entries
+// residual, the Jacobian items, the rows' D^-1 entries
 struct RowCell {
-    double res, v1, v2, p, g[7], a, co[3];
+    RowJac j;
+    double res, g[7], a, co[3];
 };
-// (st: the pencil's part of a slab)
-__device__ __forceinline__ RowCell row_cell(const RowMap &m, const double *st, int ln)
-{
-    RowCell c;
-    c.res = st[SP_RES + ln];
-    c.v1 = st[m.v1]; c.v2 = st[m.v2]; c.p = st[m.p];
-#pragma unroll
-    for (int q = 0; q < 7; q++) c.g[q] = st[m.g[q]];
-    c.a = st[SP_GX + GX_A];
-#pragma unroll
-    for (int q = 0; q < 3; q++) c.co[q] = st[m.co[q]];
-    return c;
-}
 
 // Row n of D^-1 y in lane n (y: the row's right-hand side).  Rows 0, 4 and 5
 // are sums of four products, rows 7 and 8 of two, the rest one difference:
@@ -998,10 +995,10 @@ __device__ __forceinline__ double row_dinv(const RowMap &m, const RowCell &c, do
 {
     auto neg = [](double x, bool f) { return __longlong_as_double(__double_as_longlong(x) ^ (long long)((unsigned long long)f << 63)); };
     const double y0 = row_lane<0>(y), y5 = row_lane<5>(y), y6 = row_lane<6>(y);
-    const double s1 = y - y0 * c.p;
+    const double s1 = y - y0 * c.j.p;
     const double r6 = row_lane<6>(s1), rk = row_lane<7>(s1), ro = row_lane<8>(s1);
-    const double uuu = row_lane<1>(y) * row_lane<1>(c.v2) + row_lane<2>(y) * row_lane<2>(c.v2)
-                     + row_lane<3>(y) * row_lane<3>(c.v2) - row_lane<4>(y);
+    const double uuu = row_lane<1>(y) * row_lane<1>(c.j.v2) + row_lane<2>(y) * row_lane<2>(c.j.v2)
+                     + row_lane<3>(y) * row_lane<3>(c.j.v2) - row_lane<4>(y);
     const double co = y0 * c.co[0] + c.co[1] * uuu + c.co[2] * y6;
     const double co1 = row_lane<0>(co), co2 = row_lane<1>(co), co3 = row_lane<2>(co);
     const bool row7 = m.n7 || m.n8;
@@ -1049,14 +1046,12 @@ template <bool FWD>
 __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *tiles, int ntiles, int *err, int *ticket)
 {
     // dq hand-over, one LDS object (so that the compiler can tell its reads
-    // from the stage LDS-DMA): [0, HX) the dq of the hyperplane by the parity
-    // of s, [HX, HZ) the dq of the j / k neighbour in another tile by the
-    // parity of s, [HZ, HZ + NPV) zeros for a ghost neighbour
-    constexpr int HX = 2 * TJ * TK * NPV, HZ = HX + 2 * 2 * TJ * TK * NPV;
-    __shared__ double hand[HZ + NPV];
-    auto lds_at = [](int par, int g) { return (par * TJ * TK + g) * NPV; };
-    auto xch_at = [](int par, int a, int g) { return HX + ((par * 2 + a) * TJ * TK + g) * NPV; };
-    double *const zrow = hand + HZ;
+    // from the stage LDS-DMA), by the place of the step in the ring: what
+    // the step after reads, i.e. the step's dq of the sixteen pencils, the
+    // dq of the j / k neighbours of the four and four edge pencils in other
+    // tiles, and zeros for a neighbour outside the block
+    constexpr int HX = TJ * TK * NPV, HZ = HX + (TJ + TK) * NPV, HN = HZ + NPV;
+    __shared__ double hand[SLABS * HN];
     __shared__ double stage[SLABS * SLAB_N];
     __shared__ int gave_up, taken;
     const int npv = S.npv;
@@ -1065,7 +1060,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 15, grp = (threadIdx.x >> 4) & 15;
     if (threadIdx.x == 0) gave_up = 0;
-    if (threadIdx.x < NPV) zrow[threadIdx.x] = 0.0;
+    if (threadIdx.x < SLABS * NPV) hand[threadIdx.x / NPV * HN + HZ + threadIdx.x % NPV] = 0.0;
     for (;;) {
         // the barrier that ends a tile keeps this write behind every read of the last ticket
         if (threadIdx.x == 0) taken = atomicAdd(ticket, 1);
@@ -1094,18 +1089,20 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             // of a pencil, F then Q, GX and RES; the 12 of an edge neighbour.
             // A pencil outside the block, and a cell before or past a
             // pencil's ends, is a record of the zero outer layer.
-            const int l = threadIdx.x - 320;
-            const double *base[SLAB_LOADS];      // the piece in the record of i = 1 of its pencil
-            int off[SLAB_LOADS];                 // the cell of hyperplane s is i = 1 + s - off
+            int l = threadIdx.x - 320;
+            asm volatile("" : "+v"(l));          // (worked out per tile: kept across tiles, its pieces end up in scratch memory)
+            const double *src[SLAB_LOADS];       // the piece of the coming slab
+            int at[SLAB_LOADS];                  // its cell is at - 1 past the pencil's first zero record in sweep order
 #pragma unroll
             for (int t = 0; t < SLAB_LOADS; t++) {
                 const int u = 64 * t + l, F = FWD ? RC_FP : RC_FM;
-                int jj, kk, jn, kn, q;
+                int jj, kk, jn, kn, q, early;
                 if (u < TJ * TK * SP_N / 2) {
                     const int g = u / (SP_N / 2), c = u % (SP_N / 2);
                     jj = jn = j0 + g % TJ;
                     kk = kn = k0 + g / TJ;
                     q = 2 * c < SP_Q ? F + 2 * c : RC_Q + 2 * c - SP_Q;
+                    early = 0;
                 } else {
                     const int v = u - TJ * TK * SP_N / 2, e = min(v / (SE_N / 2), TJ + TK - 1), c = v % (SE_N / 2);
                     const bool a = e >= TK;      // a k neighbour
@@ -1114,36 +1111,39 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
                     jn = a ? jj : jj - sg;
                     kn = a ? kk - sg : kk;
                     q = 2 * c < SE_Q ? F + 6 * (a ? 2 : 1) + 2 * c : RC_Q + 2 * c - SE_Q;
+                    early = 1;
                 }
-                base[t] = S.img + widx(B, 1, min(jn, B.J + 1), min(kn, B.K + 1)) * RC_N + q;
-                off[t] = jj + kk + 1;
+                // cells are numbered 0..I in sweep order, the zero records at
+                // the pencil's ends included; slab -1 holds cell at - 1 of it
+                at[t] = FWD ? sa - sg - jj - kk - 1 + early : B.I + 1 - (sa - sg - jj - kk) + early;
+                const int c0 = min(max(at[t], 0), B.I);
+                src[t] = S.img + widx(B, FWD ? 1 + c0 : B.I + 1 - c0, min(jn, B.J + 1), min(kn, B.K + 1)) * RC_N + q;
             }
-            const int BI = B.I;
-            auto issue = [&](int s, int slot) {
+            const unsigned BI = B.I;
+            auto issue = [&](int slot) {
 #pragma unroll
                 for (int t = 0; t < SLAB_LOADS; t++) {
-                    const unsigned i = (unsigned)min(max(s - off[t], 0), BI);
-                    __builtin_amdgcn_global_load_lds((const GLOBAL void *)(base[t] + (unsigned long)i * RC_N),
+                    __builtin_amdgcn_global_load_lds((const GLOBAL void *)src[t],
                                                      (__attribute__((address_space(3))) void *)&stage[slot * SLAB_N + 128 * t],
                                                      16, 0, 0);
+                    // on to the next cell, from the first zero record to the last
+                    src[t] += (unsigned)at[t] < BI ? sg * RC_N : 0;
+                    at[t]++;
                 }
             };
             // SLABS - 3 slabs of SLAB_LOADS transfers may be outstanding
-            static_assert(SLAB_LOADS == 11 && SLABS == 6, "the wait below");
-            issue(sa - sg, SLABS - 1);
+            static_assert(SLAB_LOADS == 11 && SLABS == 5, "the wait below");
+            issue(SLABS - 1);
 #pragma unroll
-            for (int n = 0; n < SLABS - 1; n++) {
-                if (n == 3) asm volatile("s_waitcnt vmcnt(33)" ::: "memory");   // (the counter holds 63)
-                issue(sa + sg * n, n);
-            }
-            asm volatile("s_waitcnt vmcnt(33)" ::: "memory");
+            for (int n = 0; n < SLABS - 1; n++) issue(n);
+            asm volatile("s_waitcnt vmcnt(22)" ::: "memory");
             __syncthreads();
             __syncthreads();
             int slot = SLABS - 1;
             for (int s = sa;; s += sg) {
-                issue(s + sg * (SLABS - 1), slot);
+                issue(slot);
                 slot = slot == SLABS - 1 ? 0 : slot + 1;
-                asm volatile("s_waitcnt vmcnt(33)" ::: "memory");
+                asm volatile("s_waitcnt vmcnt(22)" ::: "memory");
                 lds_barrier();
                 if (s == sb) break;
             }
@@ -1159,7 +1159,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             const double *dummy = xq + widx(B, min(max(sa - j0 - k0, 2), B.I), j0, k0) * NPV;
             // per lane and tile: item t's value of step s is at xq[at + 9 s],
             // read for lo <= s <= hi (the cell is inside the block and its
-            // neighbour too), and goes to the hand-over slot to (+ parity)
+            // neighbour too), and goes to the hand-over item to
             long at[2];
             int lo[2], hi[2], to[2];
 #pragma unroll
@@ -1172,7 +1172,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
                 at[t] = widx(B, -jj - kk, jn, kn) * NPV + n;
                 lo[t] = on ? 2 + jj + kk : 1;
                 hi[t] = on ? B.I + jj + kk : 0;
-                to[t] = xch_at(0, a, g) + n;
+                to[t] = HX + (a * TK + e) * NPV + n;
             }
             bool n0, n1;
             const double *p0, *p1;
@@ -1185,7 +1185,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
                 v0 = ld_dev(p0);
                 v1 = ld_dev(p1);
             };
-            auto deliver = [&](int s) {          // wait (bounded) for step s's values, then hand them over
+            auto deliver = [&](int s, int slot) {    // wait (bounded) for step s's values, then hand them over
                 auto unset = [](bool nd, double v) { return nd && (unsigned long long)__double_as_longlong(v) == DQ_UNSET; };
                 if (__ballot(unset(n0, v0) || unset(n1, v1))) {
                     long polls = 0;
@@ -1201,19 +1201,20 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
                         if (unset(n1, v1)) v1 = ld_dev(p1);
                     } while (__ballot(unset(n0, v0) || unset(n1, v1)));
                 }
-                const int par = (s & 1) * (xch_at(1, 0, 0) - xch_at(0, 0, 0));
-                hand[to[0] + par] = n0 ? v0 : 0.0;
-                if (l64 < NEDGE - 64) hand[to[1] + par] = n1 ? v1 : 0.0;
+                hand[to[0] + slot * HN] = n0 ? v0 : 0.0;
+                if (l64 < NEDGE - 64) hand[to[1] + slot * HN] = n1 ? v1 : 0.0;
             };
+            int slot = SLABS - 1;                // the place of the step before the one whose values are read
             issue(sa);
-            deliver(sa);
+            deliver(sa, slot);
             __syncthreads();
             __syncthreads();
             for (int s = sa;; s += sg) {
+                slot = slot == SLABS - 1 ? 0 : slot + 1;
                 // the next step's values are read at the start of this step,
                 // while the pencils compute, as late as they can be
                 if (s != sb) issue(s + sg);
-                if (s != sb) deliver(s + sg);
+                if (s != sb) deliver(s + sg, slot);
                 lds_barrier();
                 if (s == sb) break;
             }
@@ -1225,7 +1226,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
         const int gj = grp % TJ, gk = grp / TJ;
         const bool mine = lane < npv;
         const int ln = lane < NPV ? lane : 0;
-        const RowMap rows = row_map<FWD>(lane, npv);
+        const RowMap rows = row_map(lane, npv);
         const int j = j0 + gj, k = k0 + gk;
         const bool live = (j <= jend && k <= kend);
         const bool edge = down_edge(grp);
@@ -1233,84 +1234,104 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
         const int jm = j - sg, km = k - sg;
         const bool lj = jm >= j0 && jm <= jend, lk = km >= k0 && km <= kend;
         const bool nj = jm >= 2 && jm <= B.J, nk = km >= 2 && km <= B.K;   // neighbour inside the block
-        // The stage items of the j and k neighbours: a neighbour pencil of the
-        // tile holds its cell in the slab of this step (it is one hyperplane
-        // ahead), an edge neighbour in its own place of the next one's.
         const bool ej = gj == (FWD ? 0 : TJ - 1), ek = gk == (FWD ? 0 : TK - 1);
-        const int pj = ej ? SLAB_E + gk * SE_N : (grp - sg) * SP_N, pk = ek ? SLAB_E + (TK + gj) * SE_N : (grp - sg * TJ) * SP_N;
-        const int qj = ej ? SE_Q - SP_Q : 0, qk = ek ? SE_Q - SP_Q : 0;
-        const int j1 = pj + rows.v1 + (rows.face ? (ej ? 0 : 6) : qj), j2 = pj + rows.v2 + qj, jp = pj + rows.p + qj;
-        const int k1 = pk + rows.v1 + (rows.face ? (ek ? 0 : 12) : qk), k2 = pk + rows.v2 + qk, kp = pk + rows.p + qk;
-        double *out = FWD ? S.img + (widx(B, 1, min(j, B.J), min(k, B.K)) * RC_N + RC_RES + lane)
-                          : xq + (widx(B, 1, min(j, B.J), min(k, B.K)) * NPV + lane);
-        double *const xe = xq + (widx(B, 1, min(j, B.J), min(k, B.K)) * NPV + lane);
-        if (lane < NPV) hand[lds_at((sa - sg) & 1, grp) + lane] = 0.0;       // the first step's upstream reads zeros
+        // Places of the stage items: this pencil's, and its j and k
+        // neighbours' (a pencil of the tile, or an edge neighbour), each in a
+        // slab; of the upstream dq in the hand-over object
+        struct JacAt { const double *v1, *a, *lb, *v2, *p; };
+        auto jac_at = [&](int pencil, bool e, int f) {
+            const int q = e ? SE_Q - SP_Q : 0;
+            const double *st = stage + pencil;
+            return JacAt{st + rows.v1 + (rows.face ? f : q), st + rows.a + (rows.aface ? f : q), st + rows.lb + (rows.face ? f : q),
+                         st + rows.v2 + q, st + rows.p + q};
+        };
+        auto jac = [&](const JacAt &w, int slab) {
+            return RowJac{w.v1[slab], w.a[slab], w.a[slab + 1], w.a[slab + 2], w.lb[slab], w.v2[slab], w.p[slab]};
+        };
+        const int mp = grp * SP_N;
+        const JacAt ai = jac_at(mp, false, 0), aj = jac_at(ej ? SLAB_E + gk * SE_N : (grp - sg) * SP_N, ej, ej ? 0 : 6),
+                    ak = jac_at(ek ? SLAB_E + (TK + gj) * SE_N : (grp - sg * TJ) * SP_N, ek, ek ? 0 : 12);
+        auto cell = [&](int slab) {
+            const double *st = stage + mp;
+            RowCell c;
+            c.j = jac(ai, slab);
+            c.res = st[slab + SP_RES + ln];
+#pragma unroll
+            for (int q = 0; q < 7; q++) c.g[q] = st[slab + rows.g[q]];
+            c.a = st[slab + SP_GX + GX_A];
+#pragma unroll
+            for (int q = 0; q < 3; q++) c.co[q] = st[slab + rows.co[q]];
+            return c;
+        };
+        // (indices into the hand-over object, not pointers chosen among
+        // several, so the compiler sees these reads cannot touch the stage)
+        const int oi = grp * NPV + ln, oj = (lj ? (grp - sg) * NPV : nj ? HX + gk * NPV : HZ) + ln,
+                  ok = (lk ? (grp - sg * TJ) * NPV : nk ? HX + (TK + gj) * NPV : HZ) + ln;
+        // where this pencil's results go, from the cell of the first hyperplane on
+        const int i0 = sa - j - k;
+        double *xe = xq + (widx(B, i0, min(j, B.J), min(k, B.K)) * NPV + lane);
+        double *yo = S.img + (widx(B, i0, min(j, B.J), min(k, B.K)) * RC_N + RC_RES + lane);
+        if (lane < NPV) hand[(SLABS - 1) * HN + oi] = 0.0;           // the first step's upstream reads zeros
         double ci[8], cj[8], ck[8];                                  // coefficients of the coming step
         RowCell own;                                                 // its cell
-        int cur = (SLABS - 1) * SLAB_N, nxt = 0;                     // slabs of this step and the next
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < 8; q++) ci[q] = 0.0;
-        {
-            const double *const sj = stage + (ej ? nxt : cur), *const sk = stage + (ek ? nxt : cur);
-            row_coef<FWD>(rows, sj[j1], sj[j2], sj[jp], cj);
-            row_coef<FWD>(rows, sk[k1], sk[k2], sk[kp], ck);
-            own = row_cell(rows, stage + nxt + grp * SP_N, ln);
-        }
+        row_coef(rows, jac(aj, (SLABS - 1) * SLAB_N), cj);
+        row_coef(rows, jac(ak, (SLABS - 1) * SLAB_N), ck);
+        own = cell(0);
         __syncthreads();
-        for (int s = sa;; s += sg) {
-            const int i = s - j - k;
+        int i = i0, left = (sb - sa) * sg;                           // this step's cell, the steps after it
+        // step n of the tile, n mod SLABS = C; false after the last one
+        auto step = [&](auto C) {
+            constexpr int c = C, before = (c + SLABS - 1) % SLABS, after = (c + 1) % SLABS;
             const bool act = live && i >= 2 && i <= BI;
-            cur = nxt;
-            nxt = nxt == (SLABS - 1) * SLAB_N ? 0 : nxt + SLAB_N;
             // dq of the three upstream neighbours: in the tile from the
             // previous hyperplane, from another tile through the poll wavefront
-            const int pb = (s - sg) & 1;
-            // (indices into the hand-over object, not pointers chosen among
-            // several, so the compiler sees these reads cannot touch the stage)
-            const int oi = lds_at(pb, grp);
-            const int oj = lj ? lds_at(pb, grp - sg) : (nj ? xch_at(s & 1, 0, grp) : HZ);
-            const int ok = lk ? lds_at(pb, grp - sg * TJ) : (nk ? xch_at(s & 1, 1, grp) : HZ);
-            const double xi = hand[oi + ln], xj = hand[oj + ln], xk = hand[ok + ln];
+            const double xi = hand[oi + before * HN], xj = hand[oj + before * HN], xk = hand[ok + before * HN];
             // dcv = res + the three upstream products, in the reference's i, j, k order
             double y = own.res;
             row_apply(ci, xi, y);
             row_apply(cj, xj, y);
             row_apply(ck, xk, y);
-            __builtin_amdgcn_sched_barrier(0);
             // dq = D^-1 dcv
             const double xn = row_dinv(rows, own, y);
             if (lane < NPV) {
-                hand[lds_at(s & 1, grp) + lane] = act ? xn : 0.0;
+                hand[oi + c * HN] = act ? xn : 0.0;
                 // the dq that other tiles wait for goes out at once.  Forward,
                 // no other dq is read again (the backward sweep starts from
                 // dcv); backward, every cell's is the update's input
                 if (act && mine) {
-                    if (edge) st_dev(xe + (i - 1) * NPV, xn);
-                    if constexpr (FWD) out[(long)(i - 1) * RC_N] = y;
-                    else if (!edge) out[(i - 1) * NPV] = xn;
+                    if (edge) st_dev(xe, xn);
+                    if constexpr (FWD) *yo = y;
+                    else if (!edge) *xe = xn;
                 }
             }
-            __builtin_amdgcn_sched_barrier(0);
+            xe += sg * NPV;
+            if constexpr (FWD) yo += RC_N;
+            i += sg;
             // coefficients of the next step (independent of dq): this cell's
             // row through its face to the next cell, and the j / k neighbours
             // of the next cell; and the next cell's own terms
-            const double *const sj = stage + (ej ? nxt : cur), *const sk = stage + (ek ? nxt : cur);
-            const double vj1 = sj[j1], vj2 = sj[j2], vjp = sj[jp];
-            const double vk1 = sk[k1], vk2 = sk[k2], vkp = sk[kp];
-            row_coef<FWD>(rows, own.v1, own.v2, own.p, ci);
-            row_coef<FWD>(rows, vj1, vj2, vjp, cj);
-            row_coef<FWD>(rows, vk1, vk2, vkp, ck);
-            own = row_cell(rows, stage + nxt + grp * SP_N, ln);
+            const RowJac nbj = jac(aj, c * SLAB_N), nbk = jac(ak, c * SLAB_N);
+            row_coef(rows, own.j, ci);
+            row_coef(rows, nbj, cj);
+            row_coef(rows, nbk, ck);
+            own = cell(after * SLAB_N);
             // formed before the barrier (while the poll wavefront may still be
             // waiting), not after it on the next step's path
 #pragma unroll
             for (int q = 0; q < 8; q++) asm volatile("" : "+v"(ci[q]), "+v"(cj[q]), "+v"(ck[q]));
 #pragma unroll
             for (int q = 0; q < 7; q++) asm volatile("" : "+v"(own.g[q]));
-            asm volatile("" : "+v"(own.res), "+v"(own.v1), "+v"(own.v2), "+v"(own.p), "+v"(own.a), "+v"(own.co[0]), "+v"(own.co[1]), "+v"(own.co[2]));
+            asm volatile("" : "+v"(own.res), "+v"(own.j.v1), "+v"(own.j.a), "+v"(own.j.b), "+v"(own.j.c), "+v"(own.j.lb), "+v"(own.j.v2), "+v"(own.j.p),
+                         "+v"(own.a), "+v"(own.co[0]), "+v"(own.co[1]), "+v"(own.co[2]));
             lds_barrier();
-            if (s == sb) break;
+            return left-- > 0;
+        };
+        static_assert(SLABS == 5, "the steps of the ring");
+        while (step(std::integral_constant<int, 0>{}) && step(std::integral_constant<int, 1>{}) && step(std::integral_constant<int, 2>{}) &&
+               step(std::integral_constant<int, 3>{}) && step(std::integral_constant<int, 4>{})) {
         }
         __syncthreads();
     }
