@@ -149,6 +149,58 @@ __device__ __forceinline__ void cell_of(const BlkD &B, long r, int &i, int &j, i
     k = 2 + (int)(r / ((long)ni * nj));
 }
 
+// Kernels over faces or cells that read many neighbours keep a workgroup
+// inside one block (the blocks' ranges are rounded up to whole workgroups), so
+// the block's extents are scalars: a stencil point or a variable is another
+// scalar base, and all of a lane's reads share its one 32-bit offset.
+// With per-lane 64-bit places and divisions the viscous face kernels took 85
+// us a direction at 128x64x64 cells, now 70, the combine 149, now 143, the
+// inviscid ones (bound by their arithmetic) 1 % more than now.  (32 bits: a
+// block of 2^29 cells would take more than the device's memory.)
+constexpr int BLK_WG = 256;
+// the workgroup's block, and the lane's item t of that block's n[b] ones
+template <class N> __device__ __forceinline__ int wg_block(const DS &S, N n, unsigned &t)
+{
+    unsigned w = blockIdx.x;
+    int b = 0;
+    for (int q = 0; q + 1 < S.nb; q++) {
+        const unsigned m = (unsigned)((n(S.b[q]) + BLK_WG - 1) / BLK_WG);
+        if (b == q && w >= m) { w -= m; b = q + 1; }
+    }
+    t = w * BLK_WG + threadIdx.x;
+    return b;
+}
+// item q (32 bits, the lane's) of a scalar base
+template <class T> __device__ __forceinline__ T &at32(T *base, unsigned q)
+{
+    return *(T *)((char *)base + (size_t)(q * (unsigned)sizeof(T)));
+}
+template <class T> __device__ __forceinline__ const T &at32(const T *base, unsigned q)
+{
+    return *(const T *)((const char *)base + (size_t)(q * (unsigned)sizeof(T)));
+}
+// 32-bit places within block B's arrays: ghosted, dcv ranges, face vectors of axis AX
+__device__ __forceinline__ unsigned gidx32(const BlkD &B, int i, int j, int k)
+{
+    return (unsigned)(i + 1) + (unsigned)B.nx * ((unsigned)(j + 1) + (unsigned)B.ny * (unsigned)(k + 1));
+}
+__device__ __forceinline__ unsigned widx32(const BlkD &B, int i, int j, int k)
+{
+    return (unsigned)(i - 1) + (unsigned)(B.I + 1) * ((unsigned)(j - 1) + (unsigned)(B.J + 1) * (unsigned)(k - 1));
+}
+template <int AX> __device__ __forceinline__ unsigned vidx32(const BlkD &B, int i, int j, int k)
+{
+    const unsigned nx = B.I + (AX != 0), ny = B.J + (AX != 1);
+    return (unsigned)(i - 1) + nx * ((unsigned)(j - 1) + ny * (unsigned)(k - 1));
+}
+// face vector of axis AX at place q, di, dj, dk (uniform) further
+template <int AX> __device__ __forceinline__ void face_vec32(const DS &S, const BlkD &B, unsigned q, int di, int dj, int dk, double *v)
+{
+    const long nx = B.I + (AX != 0), ny = B.J + (AX != 1), n = AX == 0 ? S.NCX : AX == 1 ? S.NEX : S.NTX;
+    const double *a = (AX == 0 ? S.cx + B.cx0 : AX == 1 ? S.ex + B.ex0 : S.tx + B.tx0) + (di + nx * (dj + ny * dk));
+    v[0] = at32(a, q); v[1] = at32(a + n, q); v[2] = at32(a + 2 * n, q);
+}
+
 // ------------------------------------------------------------ EOS kernels
 // dc (and mut = emutref) of interior cells from pv
 __global__ __launch_bounds__(256) void k_eos_cells(DS S, int interior_only, int set_mut)
@@ -496,6 +548,17 @@ __device__ __forceinline__ const BlkD &face_of(const DS &S, long t, int &i, int 
     return B;
 }
 
+// the same with the workgroup inside one block: t is the face's number there
+template <int D>
+__device__ __forceinline__ void face_at32(const BlkD &B, unsigned t, int &i, int &j, int &k)
+{
+    const unsigned ni = D == 0 ? B.I : B.I - 1, nj = D == 1 ? B.J : B.J - 1;
+    const unsigned row = t / ni, pl = row / nj;
+    i = (D == 0 ? 1 : 2) + (int)(t - row * ni);
+    j = (D == 1 ? 1 : 2) + (int)(row - pl * nj);
+    k = (D == 2 ? 1 : 2) + (int)pl;
+}
+
 // offset of stencil point ll (Fortran numbering) from the face's left cell
 template <int D>
 __device__ __forceinline__ long stencil_off(const BlkD &B, int ll)
@@ -518,57 +581,58 @@ __device__ __forceinline__ long stencil_off(const BlkD &B, int ll)
 // pressure keeps the low-Mach pressure differences; the metastable-vapour
 // switch compares against the FP64 saturation pressure).
 template <int D, bool SENSOR, class R>
-__global__ __launch_bounds__(256) void k_face(DS S)
+__global__ __launch_bounds__(BLK_WG) void k_face(DS S)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= S.NF[D]) return;
+    unsigned t;
+    const BlkD &B = S.b[wg_block(S, [](const BlkD &b) { return b.nf[D]; }, t)];
+    if (t >= (unsigned)B.nf[D]) return;
     int i, j, k;
-    const BlkD &B = face_of<D>(S, t, i, j, k);
+    face_at32<D>(B, t, i, j, k);
     const Par &P = S.P;
     const int npv = S.npv;
-    const long g9 = gidx(B, i, j, k);
+    const unsigned g9 = gidx32(B, i, j, k);
     const long sN = D == 0 ? 1 : (D == 1 ? (long)B.nx : (long)B.nx * B.ny);
     R c9[NPV], c10[NPV], xl[NPV], xr[NPV];
     R g3[6][3];
-    const double *f0 = S.pv + g9;
+    const double *f0 = S.pv + B.g0, *d0 = S.dc + B.g0;
     Par Pi = P;
     Pi.iturb = -3;          // no viscous differences here
-    face_recon<R>(Pi, npv, [&](int ll, int n) -> R { return R(f0[(long)n * S.NG + stencil_off<D>(B, ll)]); },
+    face_recon<R>(Pi, npv, [&](int ll, int n) -> R { return R(at32(f0 + ((long)n * S.NG + stencil_off<D>(B, ll)), g9)); },
                   c9, c10, xl, xr, g3);
-    const long gq = g9 + sN;
     double n3d[3];
-    face_vec(S, B, D, i, j, k, n3d);
+    face_vec32<D>(S, B, vidx32<D>(B, i, j, k), 0, 0, 0, n3d);
     const R n3[3] = {R(n3d[0]), R(n3d[1]), R(n3d[2])};
-    R rh9[3] = {R(S.dc[D_RHO * S.NG + g9]), R(S.dc[D_H * S.NG + g9]), R(0)};
-    R rh10[3] = {R(S.dc[D_RHO * S.NG + gq]), R(S.dc[D_H * S.NG + gq]), R(0)};
+    R rh9[3] = {R(at32(d0 + D_RHO * S.NG, g9)), R(at32(d0 + D_H * S.NG, g9)), R(0)};
+    R rh10[3] = {R(at32(d0 + (D_RHO * S.NG + sN), g9)), R(at32(d0 + (D_H * S.NG + sN), g9)), R(0)};
     R fx[NPV];
     if constexpr (SENSOR) {
         // the pressure sensor of Roe-M / AUSMPW+: x(1:18,1) of the face stencil
         R sd[18];
-        for (int ll = 1; ll <= 18; ll++) sd[ll - 1] = R(f0[stencil_off<D>(B, ll)]);
-        rh9[2] = R(S.dc[D_C2 * S.NG + g9]);
-        rh10[2] = R(S.dc[D_C2 * S.NG + gq]);
+        for (int ll = 1; ll <= 18; ll++) sd[ll - 1] = R(at32(f0 + stencil_off<D>(B, ll), g9));
+        rh9[2] = R(at32(d0 + D_C2 * S.NG, g9));
+        rh10[2] = R(at32(d0 + (D_C2 * S.NG + sN), g9));
         inviscid_face<R, true>(P, npv, n3, c9, c10, xl, xr, rh9, rh10, fx, sd);
     } else {
         inviscid_face<R, false>(P, npv, n3, c9, c10, xl, xr, rh9, rh10, fx);
     }
-    double *out = S.ff[D];
+    double *out = S.ff[D] + B.f0[D];
     const long NF = S.NF[D];
-    for (int n = 0; n < NPV; n++) if (n < npv) out[n * NF + t] = double(fx[n]);
+    for (int n = 0; n < NPV; n++) if (n < npv) at32(out + n * NF, t) = double(fx[n]);
 }
 
 // Viscous flux of every face of direction D (src/vsflux_module.f90:182-398),
 // with the metric averaging of src/rhs_module.f90:340-357.  R as k_face.
 template <int D, class R>
-__global__ __launch_bounds__(256) void k_vface(DS S)
+__global__ __launch_bounds__(BLK_WG) void k_vface(DS S)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= S.NF[D]) return;
+    unsigned t;
+    const BlkD &B = S.b[wg_block(S, [](const BlkD &b) { return b.nf[D]; }, t)];
+    if (t >= (unsigned)B.nf[D]) return;
     int i, j, k;
-    const BlkD &B = face_of<D>(S, t, i, j, k);
+    face_at32<D>(B, t, i, j, k);
     const Par &P = S.P;
     const int npv = S.npv;
-    const long g9 = gidx(B, i, j, k);
+    const unsigned g9 = gidx32(B, i, j, k);
     const long sN = D == 0 ? 1 : (D == 1 ? (long)B.nx : (long)B.nx * B.ny);
     R g3[6][3] = {};
     R c9[NPV], c10[NPV];
@@ -576,10 +640,10 @@ __global__ __launch_bounds__(256) void k_vface(DS S)
     for (int n = 0; n < NPV; n++) {
         c9[n] = c10[n] = R(0);
         if (n >= npv) continue;
-        const double *f = S.pv + (long)n * S.NG + g9;
-        auto xs = [&](int ll) -> R { return R(f[stencil_off<D>(B, ll)]); };
-        c9[n] = R(f[0]);
-        c10[n] = R(f[sN]);
+        const double *f = S.pv + (B.g0 + (long)n * S.NG);
+        auto xs = [&](int ll) -> R { return R(at32(f + stencil_off<D>(B, ll), g9)); };
+        c9[n] = R(at32(f, g9));
+        c10[n] = R(at32(f + sN, g9));
         if ((n >= 1 && n <= 4) || n >= 7) {
             const int q = (n <= 4) ? n - 1 : n - 3;     // u, v, w, T, k, omega
             g3[q][0] = xs(10) - xs(9);
@@ -589,51 +653,43 @@ __global__ __launch_bounds__(256) void k_vface(DS S)
                                     - xs(5) - xs(6) + xs(17) + xs(18));
         }
     }
-    int ip = i, jp = j, kp = k;
-    if (D == 0) ip++; else if (D == 1) jp++; else kp++;
-    const long gq = g9 + sN;
-    double n3d[3];
-    face_vec(S, B, D, i, j, k, n3d);
-    double e4d[4][3], t4d[4][3];
-    const int E = (D + 1) % 3, T = (D + 2) % 3;
-    int p0[3] = {i, j, k}, p1[3] = {ip, jp, kp};
-    int a0[3], a1[3];
+    constexpr int E = (D + 1) % 3, T = (D + 2) % 3;
+    constexpr int dp[3] = {D == 0, D == 1, D == 2}, de[3] = {E == 0, E == 1, E == 2}, dt[3] = {T == 0, T == 1, T == 2};
+    double n3d[3], e4d[4][3], t4d[4][3];
+    face_vec32<D>(S, B, vidx32<D>(B, i, j, k), 0, 0, 0, n3d);
+    const unsigned qe = vidx32<E>(B, i, j, k), qt = vidx32<T>(B, i, j, k);
     // e-family: (P,e-1), (P+1,e-1), (P,e), (P+1,e)
-    for (int q = 0; q < 3; q++) { a0[q] = p0[q]; a1[q] = p1[q]; }
-    a0[E]--; a1[E]--;
-    face_vec(S, B, E, a0[0], a0[1], a0[2], e4d[0]);
-    face_vec(S, B, E, a1[0], a1[1], a1[2], e4d[1]);
-    face_vec(S, B, E, p0[0], p0[1], p0[2], e4d[2]);
-    face_vec(S, B, E, p1[0], p1[1], p1[2], e4d[3]);
+    face_vec32<E>(S, B, qe, -de[0], -de[1], -de[2], e4d[0]);
+    face_vec32<E>(S, B, qe, dp[0] - de[0], dp[1] - de[1], dp[2] - de[2], e4d[1]);
+    face_vec32<E>(S, B, qe, 0, 0, 0, e4d[2]);
+    face_vec32<E>(S, B, qe, dp[0], dp[1], dp[2], e4d[3]);
     // t-family: i faces (P,t-1),(P+1,t-1),(P,t),(P+1,t); j and k faces (P,t-1),(P,t),(P+1,t-1),(P+1,t)
-    for (int q = 0; q < 3; q++) { a0[q] = p0[q]; a1[q] = p1[q]; }
-    a0[T]--; a1[T]--;
-    face_vec(S, B, T, a0[0], a0[1], a0[2], t4d[0]);
-    if (D == 0) {
-        face_vec(S, B, T, a1[0], a1[1], a1[2], t4d[1]);
-        face_vec(S, B, T, p0[0], p0[1], p0[2], t4d[2]);
-    } else {
-        face_vec(S, B, T, p0[0], p0[1], p0[2], t4d[1]);
-        face_vec(S, B, T, a1[0], a1[1], a1[2], t4d[2]);
-    }
-    face_vec(S, B, T, p1[0], p1[1], p1[2], t4d[3]);
+    face_vec32<T>(S, B, qt, -dt[0], -dt[1], -dt[2], t4d[0]);
+    face_vec32<T>(S, B, qt, dp[0] - dt[0], dp[1] - dt[1], dp[2] - dt[2], t4d[D == 0 ? 1 : 2]);
+    face_vec32<T>(S, B, qt, 0, 0, 0, t4d[D == 0 ? 2 : 1]);
+    face_vec32<T>(S, B, qt, dp[0], dp[1], dp[2], t4d[3]);
     R n3[3], e4[4][3], t4[4][3];
     for (int q = 0; q < 3; q++) n3[q] = R(n3d[q]);
     for (int a = 0; a < 4; a++)
         for (int q = 0; q < 3; q++) { e4[a][q] = R(e4d[a][q]); t4[a][q] = R(t4d[a][q]); }
     R gl[2], gr[2], dl[ND], dr[ND];
-    long wl = widx(B, i, j, k), wr = widx(B, ip, jp, kp);
-    gl[0] = R(S.vol[wl]); gr[0] = R(S.vol[wr]);
-    gl[1] = S.ydn ? R(S.ydn[wl]) : R(1); gr[1] = S.ydn ? R(S.ydn[wr]) : R(1);
-    for (int m = 0; m < ND; m++) { dl[m] = R(S.dc[m * S.NG + g9]); dr[m] = R(S.dc[m * S.NG + gq]); }
-    R ml = S.mut ? R(S.mut[g9]) : R(0), mr = S.mut ? R(S.mut[gq]) : R(0);
+    const unsigned w = widx32(B, i, j, k);
+    const long sW = D == 0 ? 1 : (D == 1 ? (long)(B.I + 1) : (long)(B.I + 1) * (B.J + 1));
+    const double *vol = S.vol + B.w0;
+    gl[0] = R(at32(vol, w)); gr[0] = R(at32(vol + sW, w));
+    gl[1] = R(1); gr[1] = R(1);
+    if (S.ydn) { gl[1] = R(at32(S.ydn + B.w0, w)); gr[1] = R(at32(S.ydn + (B.w0 + sW), w)); }
+    const double *d0 = S.dc + B.g0;
+    for (int m = 0; m < ND; m++) { dl[m] = R(at32(d0 + m * S.NG, g9)); dr[m] = R(at32(d0 + (m * S.NG + sN), g9)); }
+    R ml = R(0), mr = R(0);
+    if (S.mut) { ml = R(at32(S.mut + B.g0, g9)); mr = R(at32(S.mut + (B.g0 + sN), g9)); }
     R cav[5] = {R(0.5) * (c9[1] + c10[1]), R(0.5) * (c9[2] + c10[2]), R(0.5) * (c9[3] + c10[3]), R(0), R(0)};
     if (npv > 7) { cav[3] = R(0.5) * (c9[7] + c10[7]); cav[4] = R(0.5) * (c9[8] + c10[8]); }
     R fv[NPV];
     visc_flux<R>(P, n3, e4, t4, gl, gr, g3, cav, dl, dr, ml, mr, fv);
-    double *out = S.ff[D];
+    double *out = S.ff[D] + B.f0[D];
     const long NF = S.NF[D];
-    for (int n = 0; n < NPV; n++) if (n < npv) out[(npv + n) * NF + t] = double(fv[n]);
+    for (int n = 0; n < NPV; n++) if (n < npv) at32(out + (npv + n) * NF, t) = double(fv[n]);
 }
 
 __device__ __forceinline__ long fidx(const BlkD &B, int D, int i, int j, int k)
@@ -648,33 +704,37 @@ __device__ __forceinline__ long fidx(const BlkD &B, int D, int i, int j, int k)
 // sources (a full EOS per cell) and the DES length scales; Merkle, no
 // cavitation and RANS SST run the lighter one.
 template <bool MODELS>
-__global__ __launch_bounds__(256) void k_combine(DS S)
+__global__ __launch_bounds__(BLK_WG) void k_combine(DS S)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= S.NC) return;
-    const BlkD &B = S.b[find_blk(S, t, 0)];
+    unsigned t;
+    const BlkD &B = S.b[wg_block(S, [](const BlkD &b) { return b.nc; }, t)];
+    if (t >= (unsigned)B.nc) return;
     const Par &P = S.P;
     const int npv = S.npv;
     const bool visc = (P.iturb >= -2);
-    int i, j, k;
-    cell_of(B, t - B.c0, i, j, k);
+    const unsigned nI = B.I - 1, nJ = B.J - 1, row = t / nI, pl = row / nJ;
+    const int i = 2 + (int)(t - row * nI), j = 2 + (int)(row - pl * nJ), k = 2 + (int)pl;
     double r[NPV];
+#pragma unroll
     for (int D = 0; D < 3; D++) {
-        long f1 = fidx(B, D, i, j, k);
-        long f0 = fidx(B, D, i - (D == 0), j - (D == 1), k - (D == 2));
-        const double *F = S.ff[D];
-        long NF = S.NF[D];
+        // the cell's lower face of direction D, and from it to the upper one
+        const unsigned f = (unsigned)(i - 2) + (nI + (D == 0)) * ((unsigned)(j - 2) + (nJ + (D == 1)) * (unsigned)(k - 2));
+        const long up = D == 0 ? 1 : D == 1 ? (long)nI : (long)nI * nJ;
+        const double *F = S.ff[D] + B.f0[D];
+        const long NF = S.NF[D];
         for (int n = 0; n < NPV; n++) if (n < npv) {
-            double a = -(F[n * NF + f1] - F[n * NF + f0]);
+            double a = -(at32(F + (n * NF + up), f) - at32(F + n * NF, f));
             r[n] = (D == 0) ? a : r[n] + a;
-            if (visc) r[n] = r[n] + (F[(npv + n) * NF + f1] - F[(npv + n) * NF + f0]);
+            if (visc) r[n] = r[n] + (at32(F + ((npv + n) * NF + up), f) - at32(F + (npv + n) * NF, f));
         }
     }
-    long g = gidx(B, i, j, k);
+    const unsigned g = gidx32(B, i, j, k), w = widx32(B, i, j, k);
+    const double *f0 = S.pv + B.g0;
+    const long NC = S.NC, c0 = B.c0;
     double d[ND], pc[NPV];
-    for (int m = 0; m < ND; m++) d[m] = S.dc[m * S.NG + g];
-    for (int n = 0; n < NPV; n++) if (n < npv) pc[n] = S.pv[n * S.NG + g];
-    double vol = S.vol[widx(B, i, j, k)];
+    for (int m = 0; m < ND; m++) d[m] = at32(S.dc + (B.g0 + m * S.NG), g);
+    for (int n = 0; n < NPV; n++) if (n < npv) pc[n] = at32(f0 + n * S.NG, g);
+    double vol = at32(S.vol + B.w0, w);
     if (P.ncav) {
         double rc, rv, ic[4];
         if constexpr (MODELS) {
@@ -689,23 +749,27 @@ __global__ __launch_bounds__(256) void k_combine(DS S)
             merkle(P, pc, d, vol, rc, rv, ic);
         }
         r[5] = r[5] + rv - rc;
-        for (int q = 0; q < 4; q++) S.icav[q * S.NC + t] = ic[q];
-        S.rcav[t] = rc;
-        S.rcav[S.NC + t] = rv;
+        for (int q = 0; q < 4; q++) at32(S.icav + (c0 + q * NC), t) = ic[q];
+        at32(S.rcav + c0, t) = rc;
+        at32(S.rcav + (c0 + NC), t) = rv;
     }
     if (P.iturb == 0) {
         double x7[7][NPV], f6[6][3], src[2], it[4], oc;
-        const int di[7] = {-1, 0, 1, 0, 0, 0, 0}, dj[7] = {0, 0, 0, -1, 1, 0, 0}, dk[7] = {0, 0, 0, 0, 0, -1, 1};
-        for (int q = 0; q < 7; q++) {
-            long gn = gidx(B, i + di[q], j + dj[q], k + dk[q]);
-            for (int n = 0; n < NPV; n++) if (n < npv) x7[q][n] = S.pv[n * S.NG + gn];
-        }
-        cell_faces(S, B, i, j, k, f6);
-        sst_source<MODELS>(P, x7, f6, vol, S.ydn[widx(B, i, j, k)], d, S.mut[g], src, it, oc);
-        S.ocut[t] = oc;
+        const long ny = B.nx, nz = (long)B.nx * B.ny, to[7] = {-1, 0, 1, -ny, ny, -nz, nz};
+        for (int q = 0; q < 7; q++)
+            for (int n = 0; n < NPV; n++) if (n < npv) x7[q][n] = at32(f0 + (n * S.NG + to[q]), g);
+        const unsigned q0 = vidx32<0>(B, i, j, k), q1 = vidx32<1>(B, i, j, k), q2 = vidx32<2>(B, i, j, k);
+        face_vec32<0>(S, B, q0, -1, 0, 0, f6[0]);
+        face_vec32<0>(S, B, q0, 0, 0, 0, f6[1]);
+        face_vec32<1>(S, B, q1, 0, -1, 0, f6[2]);
+        face_vec32<1>(S, B, q1, 0, 0, 0, f6[3]);
+        face_vec32<2>(S, B, q2, 0, 0, -1, f6[4]);
+        face_vec32<2>(S, B, q2, 0, 0, 0, f6[5]);
+        sst_source<MODELS>(P, x7, f6, vol, at32(S.ydn + B.w0, w), d, at32(S.mut + B.g0, g), src, it, oc);
+        at32(S.ocut + c0, t) = oc;
         r[7] = r[7] + src[0];
         r[8] = r[8] + src[1];
-        for (int q = 0; q < 4; q++) S.itt[q * S.NC + t] = it[q];
+        for (int q = 0; q < 4; q++) at32(S.itt + (c0 + q * NC), t) = it[q];
     }
     if (P.nsteady > 0) {
         double fx[NPV];
@@ -716,12 +780,12 @@ __global__ __launch_bounds__(256) void k_combine(DS S)
         fx[4] = d[D_RHO] * (d[D_H] + 0.5 * (pc[1] * pc[1] + pc[2] * pc[2] + pc[3] * pc[3])) - (pc[0] + P.pref);
         for (int n = 5; n < NPV; n++) if (n < npv) fx[n] = d[D_RHO] * pc[n];
         for (int n = 0; n < NPV; n++) if (n < npv) {
-            double q1 = S.qq[(long)n * S.NC + t], q2 = S.qq[(long)(npv + n) * S.NC + t];
+            double q1 = at32(S.qq + (c0 + (long)n * NC), t), q2 = at32(S.qq + (c0 + (long)(npv + n) * NC), t);
             double v = (double)P.nsteady * (P.bdf_b * fx[n] - q1) + 0.5 * ((double)P.nsteady - 1.0) * q2;
             r[n] = r[n] - v * vol / P.dt_phy;
         }
     }
-    for (int n = 0; n < NPV; n++) if (n < npv) S.res[n * S.NC + t] = r[n];
+    for (int n = 0; n < NPV; n++) if (n < npv) at32(S.res + (c0 + n * NC), t) = r[n];
 }
 
 // ------------------------------------------------------------ LU-SGS sweeps
@@ -1854,11 +1918,16 @@ int launch_rhs(cav3d_ctx *c)
     hipEventRecord(c->fork, c->st);
     hipStreamWaitEvent(c->side[0], c->fork, 0);
     hipStreamWaitEvent(c->side[1], c->fork, 0);
+    unsigned nf[3] = {}, nc = 0;         // workgroups, each inside one block
+    for (const BlkD &B : c->blk) {
+        for (int d = 0; d < 3; d++) nf[d] += nblk(B.nf[d], BLK_WG);
+        nc += nblk(B.nc, BLK_WG);
+    }
 #define CAV3D_FACES(SEN, R)                                                                             \
     do {                                                                                                \
-        hipLaunchKernelGGL((k_face<0, SEN, R>), dim3(nblk(S.NF[0], 256)), dim3(256), 0, sd[0], S);      \
-        hipLaunchKernelGGL((k_face<1, SEN, R>), dim3(nblk(S.NF[1], 256)), dim3(256), 0, sd[1], S);      \
-        hipLaunchKernelGGL((k_face<2, SEN, R>), dim3(nblk(S.NF[2], 256)), dim3(256), 0, sd[2], S);      \
+        hipLaunchKernelGGL((k_face<0, SEN, R>), dim3(nf[0]), dim3(BLK_WG), 0, sd[0], S);      \
+        hipLaunchKernelGGL((k_face<1, SEN, R>), dim3(nf[1]), dim3(BLK_WG), 0, sd[1], S);      \
+        hipLaunchKernelGGL((k_face<2, SEN, R>), dim3(nf[2]), dim3(BLK_WG), 0, sd[2], S);      \
     } while (0)
     if (sensor && mixed) CAV3D_FACES(true, float);
     else if (sensor) CAV3D_FACES(true, double);
@@ -1867,21 +1936,21 @@ int launch_rhs(cav3d_ctx *c)
 #undef CAV3D_FACES
     if (c->prm.iturb >= -2) {
         if (c->prm.precision == CAV3D_MIXED) {
-            hipLaunchKernelGGL((k_vface<0, float>), dim3(nblk(S.NF[0], 256)), dim3(256), 0, sd[0], S);
-            hipLaunchKernelGGL((k_vface<1, float>), dim3(nblk(S.NF[1], 256)), dim3(256), 0, sd[1], S);
-            hipLaunchKernelGGL((k_vface<2, float>), dim3(nblk(S.NF[2], 256)), dim3(256), 0, sd[2], S);
+            hipLaunchKernelGGL((k_vface<0, float>), dim3(nf[0]), dim3(BLK_WG), 0, sd[0], S);
+            hipLaunchKernelGGL((k_vface<1, float>), dim3(nf[1]), dim3(BLK_WG), 0, sd[1], S);
+            hipLaunchKernelGGL((k_vface<2, float>), dim3(nf[2]), dim3(BLK_WG), 0, sd[2], S);
         } else {
-            hipLaunchKernelGGL((k_vface<0, double>), dim3(nblk(S.NF[0], 256)), dim3(256), 0, sd[0], S);
-            hipLaunchKernelGGL((k_vface<1, double>), dim3(nblk(S.NF[1], 256)), dim3(256), 0, sd[1], S);
-            hipLaunchKernelGGL((k_vface<2, double>), dim3(nblk(S.NF[2], 256)), dim3(256), 0, sd[2], S);
+            hipLaunchKernelGGL((k_vface<0, double>), dim3(nf[0]), dim3(BLK_WG), 0, sd[0], S);
+            hipLaunchKernelGGL((k_vface<1, double>), dim3(nf[1]), dim3(BLK_WG), 0, sd[1], S);
+            hipLaunchKernelGGL((k_vface<2, double>), dim3(nf[2]), dim3(BLK_WG), 0, sd[2], S);
         }
     }
     hipEventRecord(c->join[0], c->side[0]);
     hipEventRecord(c->join[1], c->side[1]);
     hipStreamWaitEvent(c->st, c->join[0], 0);
     hipStreamWaitEvent(c->st, c->join[1], 0);
-    if (S.P.ncav >= 2 || S.P.ides > 0) hipLaunchKernelGGL(k_combine<true>, dim3(nblk(S.NC, 256)), dim3(256), 0, c->st, S);
-    else hipLaunchKernelGGL(k_combine<false>, dim3(nblk(S.NC, 256)), dim3(256), 0, c->st, S);
+    if (S.P.ncav >= 2 || S.P.ides > 0) hipLaunchKernelGGL(k_combine<true>, dim3(nc), dim3(BLK_WG), 0, c->st, S);
+    else hipLaunchKernelGGL(k_combine<false>, dim3(nc), dim3(BLK_WG), 0, c->st, S);
     return 0;
 }
 
