@@ -159,9 +159,8 @@ __device__ __forceinline__ void cell_of(const BlkD &B, long r, int &i, int &j, i
 // block of 2^29 cells would take more than the device's memory.)
 constexpr int BLK_WG = 256;
 // the workgroup's block, and the lane's item t of that block's n[b] ones
-template <class N> __device__ __forceinline__ int wg_block(const DS &S, N n, unsigned &t)
+template <class N> __device__ __forceinline__ int wg_block(const DS &S, unsigned w, N n, unsigned &t)
 {
-    unsigned w = blockIdx.x;
     int b = 0;
     for (int q = 0; q + 1 < S.nb; q++) {
         const unsigned m = (unsigned)((n(S.b[q]) + BLK_WG - 1) / BLK_WG);
@@ -249,17 +248,11 @@ __global__ __launch_bounds__(256) void k_eos_points(Par P, int n, const double *
 }
 
 // ------------------------------------------------------------ time step
-__global__ __launch_bounds__(256) void k_reset_scal(DS S)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        unsigned long long big = 0x7ff0000000000000ull;   // +inf
-        reinterpret_cast<unsigned long long *>(S.scal)[0] = big;
-    }
-}
+constexpr unsigned long long DT_NONE = 0x7ff0000000000000ull;   // +inf: scal[0] between two time steps
 
-__global__ __launch_bounds__(256) void k_timestep(DS S)
+__device__ __forceinline__ void timestep_cells(const DS &S, unsigned wg)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    long t = (long)wg * blockDim.x + threadIdx.x;
     double dt = 1.0e300;
     if (t < S.NC) {
         const BlkD &B = S.b[find_blk(S, t, 0)];
@@ -286,15 +279,19 @@ __global__ __launch_bounds__(256) void k_timestep(DS S)
     }
 }
 
-__global__ __launch_bounds__(256) void k_time_acc(DS S)
+__global__ __launch_bounds__(256) void k_timestep(DS S) { timestep_cells(S, blockIdx.x); }
+
+// the smallest step into the accumulated time, and its place ready for the next time step
+__device__ __forceinline__ void time_acc(const DS &S)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double m = __longlong_as_double((long long)reinterpret_cast<unsigned long long *>(S.scal)[0]);
-        if (S.P.local == -1) m = S.P.cfl;
-        S.scal[1] += m;
-        S.scal[2] = m;
-    }
+    unsigned long long *const bits = reinterpret_cast<unsigned long long *>(S.scal);
+    double m = __longlong_as_double((long long)bits[0]);
+    if (S.P.local == -1) m = S.P.cfl;
+    S.scal[1] += m;
+    S.scal[2] = m;
+    bits[0] = DT_NONE;
 }
+__global__ __launch_bounds__(64) void k_time_acc(DS S) { if (threadIdx.x == 0 && blockIdx.x == 0) time_acc(S); }
 
 __global__ __launch_bounds__(256) void k_dt_fill(DS S)
 {
@@ -487,9 +484,9 @@ __device__ void apply_bc_cell(const DS &S, const Seg &s, int i, int j, int k)
     }
 }
 
-__global__ __launch_bounds__(256) void k_bc(DS S, int which)
+__device__ __forceinline__ void bc_cells(const DS &S, int which, unsigned wg)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    long t = (long)wg * blockDim.x + threadIdx.x;
     if (t >= S.NBC[which]) return;
     const Seg *sg = S.seg[which];
     int lo = 0, hi = S.nbcseg[which] - 1;
@@ -504,6 +501,12 @@ __global__ __launch_bounds__(256) void k_bc(DS S, int which)
     int j = s.is[1] + (int)((r / ni) % nj);
     int k = s.is[2] + (int)(r / ((long)ni * nj));
     apply_bc_cell(S, s, i, j, k);
+}
+// acc: the launch also takes the time step's minimum (it follows k_begin)
+__global__ __launch_bounds__(256) void k_bc(DS S, int which, int acc)
+{
+    if (acc && blockIdx.x == 0 && threadIdx.x == 0) time_acc(S);
+    bc_cells(S, which, blockIdx.x);
 }
 
 // interface copy: the sending block's cells to the donor block's ghost cells
@@ -581,10 +584,10 @@ __device__ __forceinline__ long stencil_off(const BlkD &B, int ll)
 // pressure keeps the low-Mach pressure differences; the metastable-vapour
 // switch compares against the FP64 saturation pressure).
 template <int D, bool SENSOR, class R>
-__global__ __launch_bounds__(BLK_WG) void k_face(DS S)
+__device__ __forceinline__ void face_flux(const DS &S, unsigned wg)
 {
     unsigned t;
-    const BlkD &B = S.b[wg_block(S, [](const BlkD &b) { return b.nf[D]; }, t)];
+    const BlkD &B = S.b[wg_block(S, wg, [](const BlkD &b) { return b.nf[D]; }, t)];
     if (t >= (unsigned)B.nf[D]) return;
     int i, j, k;
     face_at32<D>(B, t, i, j, k);
@@ -623,10 +626,10 @@ __global__ __launch_bounds__(BLK_WG) void k_face(DS S)
 // Viscous flux of every face of direction D (src/vsflux_module.f90:182-398),
 // with the metric averaging of src/rhs_module.f90:340-357.  R as k_face.
 template <int D, class R>
-__global__ __launch_bounds__(BLK_WG) void k_vface(DS S)
+__device__ __forceinline__ void visc_face(const DS &S, unsigned wg)
 {
     unsigned t;
-    const BlkD &B = S.b[wg_block(S, [](const BlkD &b) { return b.nf[D]; }, t)];
+    const BlkD &B = S.b[wg_block(S, wg, [](const BlkD &b) { return b.nf[D]; }, t)];
     if (t >= (unsigned)B.nf[D]) return;
     int i, j, k;
     face_at32<D>(B, t, i, j, k);
@@ -692,6 +695,32 @@ __global__ __launch_bounds__(BLK_WG) void k_vface(DS S)
     for (int n = 0; n < NPV; n++) if (n < npv) at32(out + (npv + n) * NF, t) = double(fv[n]);
 }
 
+// All fluxes in one launch: the inviscid faces of the three directions, then
+// the viscous ones (they write other halves of the face arrays), each
+// direction's workgroups filling the tail of the one before.  RV: the viscous
+// faces' arithmetic.  Six launches on three streams did the same, but an event
+// between streams costs some 10 us, and an iteration had three forks and
+// joins: it took 210 us at 16x8x8 cells and 162 in single launches on one
+// stream, 64x32x32 448 and 404, 128x64x64 1695 and 1671; from a million cells
+// on the two were equal (the viscous faces run at two wavefronts per SIMD
+// here, three in a launch of their own).
+struct FluxWgs { unsigned n[3]; };       // workgroups of each direction
+template <bool SENSOR, class R, class RV>
+__global__ __launch_bounds__(BLK_WG) void k_flux(DS S, FluxWgs g)
+{
+    unsigned w = blockIdx.x;
+    if (w < g.n[0]) { face_flux<0, SENSOR, R>(S, w); return; }
+    w -= g.n[0];
+    if (w < g.n[1]) { face_flux<1, SENSOR, R>(S, w); return; }
+    w -= g.n[1];
+    if (w < g.n[2]) { face_flux<2, SENSOR, R>(S, w); return; }
+    w -= g.n[2];
+    if (w < g.n[0]) { visc_face<0, RV>(S, w); return; }
+    w -= g.n[0];
+    if (w < g.n[1]) { visc_face<1, RV>(S, w); return; }
+    visc_face<2, RV>(S, w - g.n[1]);
+}
+
 __device__ __forceinline__ long fidx(const BlkD &B, int D, int i, int j, int k)
 {
     if (D == 0) return B.f0[0] + (i - 1) + (long)B.I * ((j - 2) + (long)(B.J - 1) * (k - 2));
@@ -707,7 +736,7 @@ template <bool MODELS>
 __global__ __launch_bounds__(BLK_WG) void k_combine(DS S)
 {
     unsigned t;
-    const BlkD &B = S.b[wg_block(S, [](const BlkD &b) { return b.nc; }, t)];
+    const BlkD &B = S.b[wg_block(S, blockIdx.x, [](const BlkD &b) { return b.nc; }, t)];
     if (t >= (unsigned)B.nc) return;
     const Par &P = S.P;
     const int npv = S.npv;
@@ -1402,11 +1431,23 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
 }
 
 // both exchange arrays to "not yet written", both tile tickets to zero
-__global__ __launch_bounds__(256) void k_sweep_reset(double *a, double *b, long n, int *ticket)
+__device__ __forceinline__ void sweep_reset(const DS &S, long n, int *ticket, unsigned wg)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    long t = (long)wg * blockDim.x + threadIdx.x;
     if (t < 2) ticket[t] = 0;
-    if (t < n) a[t] = b[t] = __longlong_as_double((long long)DQ_UNSET);
+    if (t < n) S.xqf[t] = S.xqb[t] = __longlong_as_double((long long)DQ_UNSET);
+}
+__global__ __launch_bounds__(256) void k_sweep_reset(DS S, long n, int *ticket) { sweep_reset(S, n, ticket, blockIdx.x); }
+
+// The start of an iteration in one launch: the face boundaries, the time step
+// and the sweeps' resets, none of which reads what another writes.
+__global__ __launch_bounds__(256) void k_begin(DS S, unsigned nbc, unsigned nts, long nq, int *ticket)
+{
+    unsigned w = blockIdx.x;
+    if (w < nbc) { bc_cells(S, 0, w); return; }
+    w -= nbc;
+    if (w < nts) { timestep_cells(S, w); return; }
+    sweep_reset(S, nq, ticket, w - nts);
 }
 
 // ------------------------------------------------------------ update + norms
@@ -1482,7 +1523,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 // fixed-order final reduction of the per-workgroup partials (deterministic)
-__global__ __launch_bounds__(256) void k_norm_final(DS S, int nwg)
+__device__ __forceinline__ void norm_final(const DS &S, int nwg)
 {
     __shared__ double part[256][NPV];
     __shared__ double pm[256];
@@ -1520,9 +1561,9 @@ __global__ __launch_bounds__(256) void k_norm_final(DS S, int nwg)
     }
 }
 
-__global__ __launch_bounds__(256) void k_eddy(DS S)
+__device__ __forceinline__ void eddy_cells(const DS &S, unsigned wg)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    long t = (long)wg * blockDim.x + threadIdx.x;
     if (t >= S.NC) return;
     const BlkD &B = S.b[find_blk(S, t, 0)];
     int i, j, k;
@@ -1538,6 +1579,15 @@ __global__ __launch_bounds__(256) void k_eddy(DS S)
     cell_faces(S, B, i, j, k, f6);
     long w = widx(B, i, j, k);
     S.mut[g] = sst_eddy(x7, f6, S.vol[w], S.ydn[w], d);
+}
+__global__ __launch_bounds__(256) void k_eddy(DS S) { eddy_cells(S, blockIdx.x); }
+
+// The end of an iteration: the norms' final reduction in the first workgroup,
+// the eddy viscosity in the others
+__global__ __launch_bounds__(256) void k_finish(DS S, int nwg)
+{
+    if (blockIdx.x == 0) norm_final(S, nwg);
+    else eddy_cells(S, blockIdx.x - 1);
 }
 
 // dual time: qq(2) = qq(1), qq(1) = Q(pv, dv)
@@ -1625,7 +1675,7 @@ struct cav3d_ctx {
     std::vector<Con> cons;
     std::vector<std::vector<int>> bcdesc;   // per block: nbc*7 raw
     hipStream_t st = nullptr;
-    // the residual's j and k directions run on two more streams, forked from
+    // the adjoint's j and k directions run on two more streams, forked from
     // and joined back to st by events (default priority, like st)
     hipStream_t side[2] = {};
     hipEvent_t fork = nullptr, join[2] = {};
@@ -1894,13 +1944,15 @@ int build_bcs(cav3d_ctx *c)
     return 0;
 }
 
-int launch_setbc(cav3d_ctx *c)
+// begun: after k_begin, which has done the faces and left the time step's minimum
+int launch_setbc(cav3d_ctx *c, bool begun = false)
 {
     DS &S = c->S;
-    if (S.NBC[0]) hipLaunchKernelGGL(k_bc, dim3(nblk(S.NBC[0], 128)), dim3(128), 0, c->st, S, 0);
+    if (S.NBC[0] && !begun) hipLaunchKernelGGL(k_bc, dim3(nblk(S.NBC[0], 128)), dim3(128), 0, c->st, S, 0, 0);
     if (S.NHALO) hipLaunchKernelGGL(k_halo, dim3(nblk(S.NHALO, 128)), dim3(128), 0, c->st, S);
-    if (S.NBC[1]) hipLaunchKernelGGL(k_bc, dim3(nblk(S.NBC[1], 128)), dim3(128), 0, c->st, S, 1);
-    if (S.NBC[2]) hipLaunchKernelGGL(k_bc, dim3(nblk(S.NBC[2], 128)), dim3(128), 0, c->st, S, 2);
+    // (every block has its edges and corners)
+    hipLaunchKernelGGL(k_bc, dim3(nblk(S.NBC[1], 128)), dim3(128), 0, c->st, S, 1, begun ? 1 : 0);
+    hipLaunchKernelGGL(k_bc, dim3(nblk(S.NBC[2], 128)), dim3(128), 0, c->st, S, 2, 0);
     return 0;
 }
 
@@ -1911,53 +1963,28 @@ int launch_rhs(cav3d_ctx *c)
     // AUSMPW+ stays FP64 in the mixed mode: its pressure weight
     // (p + p_ref + rho c^2)/(rho c^2) - 1 is ~1e-5 in water and cancels in FP32
     const bool mixed = c->prm.precision == CAV3D_MIXED && S.P.nscheme != 3;
-    // the three directions are independent (each writes its own face
-    // fluxes): i on st, j and k on the two side streams, joined before the
-    // combine, so that one direction's tail overlaps the others
-    hipStream_t sd[3] = {c->st, c->side[0], c->side[1]};
-    hipEventRecord(c->fork, c->st);
-    hipStreamWaitEvent(c->side[0], c->fork, 0);
-    hipStreamWaitEvent(c->side[1], c->fork, 0);
-    unsigned nf[3] = {}, nc = 0;         // workgroups, each inside one block
+    FluxWgs g = {};                      // workgroups, each inside one block
+    unsigned nc = 0;
     for (const BlkD &B : c->blk) {
-        for (int d = 0; d < 3; d++) nf[d] += nblk(B.nf[d], BLK_WG);
+        for (int d = 0; d < 3; d++) g.n[d] += nblk(B.nf[d], BLK_WG);
         nc += nblk(B.nc, BLK_WG);
     }
-#define CAV3D_FACES(SEN, R)                                                                             \
-    do {                                                                                                \
-        hipLaunchKernelGGL((k_face<0, SEN, R>), dim3(nf[0]), dim3(BLK_WG), 0, sd[0], S);      \
-        hipLaunchKernelGGL((k_face<1, SEN, R>), dim3(nf[1]), dim3(BLK_WG), 0, sd[1], S);      \
-        hipLaunchKernelGGL((k_face<2, SEN, R>), dim3(nf[2]), dim3(BLK_WG), 0, sd[2], S);      \
-    } while (0)
-    if (sensor && mixed) CAV3D_FACES(true, float);
-    else if (sensor) CAV3D_FACES(true, double);
-    else if (mixed) CAV3D_FACES(false, float);
-    else CAV3D_FACES(false, double);
-#undef CAV3D_FACES
-    if (c->prm.iturb >= -2) {
-        if (c->prm.precision == CAV3D_MIXED) {
-            hipLaunchKernelGGL((k_vface<0, float>), dim3(nf[0]), dim3(BLK_WG), 0, sd[0], S);
-            hipLaunchKernelGGL((k_vface<1, float>), dim3(nf[1]), dim3(BLK_WG), 0, sd[1], S);
-            hipLaunchKernelGGL((k_vface<2, float>), dim3(nf[2]), dim3(BLK_WG), 0, sd[2], S);
-        } else {
-            hipLaunchKernelGGL((k_vface<0, double>), dim3(nf[0]), dim3(BLK_WG), 0, sd[0], S);
-            hipLaunchKernelGGL((k_vface<1, double>), dim3(nf[1]), dim3(BLK_WG), 0, sd[1], S);
-            hipLaunchKernelGGL((k_vface<2, double>), dim3(nf[2]), dim3(BLK_WG), 0, sd[2], S);
-        }
-    }
-    hipEventRecord(c->join[0], c->side[0]);
-    hipEventRecord(c->join[1], c->side[1]);
-    hipStreamWaitEvent(c->st, c->join[0], 0);
-    hipStreamWaitEvent(c->st, c->join[1], 0);
+    const bool visc = c->prm.iturb >= -2;
+    const dim3 grid((g.n[0] + g.n[1] + g.n[2]) * (visc ? 2 : 1)), block(BLK_WG);
+    if (sensor && mixed) hipLaunchKernelGGL((k_flux<true, float, float>), grid, block, 0, c->st, S, g);
+    else if (sensor && c->prm.precision == CAV3D_MIXED) hipLaunchKernelGGL((k_flux<true, double, float>), grid, block, 0, c->st, S, g);
+    else if (sensor) hipLaunchKernelGGL((k_flux<true, double, double>), grid, block, 0, c->st, S, g);
+    else if (mixed) hipLaunchKernelGGL((k_flux<false, float, float>), grid, block, 0, c->st, S, g);
+    else hipLaunchKernelGGL((k_flux<false, double, double>), grid, block, 0, c->st, S, g);
     if (S.P.ncav >= 2 || S.P.ides > 0) hipLaunchKernelGGL(k_combine<true>, dim3(nc), dim3(BLK_WG), 0, c->st, S);
     else hipLaunchKernelGGL(k_combine<false>, dim3(nc), dim3(BLK_WG), 0, c->st, S);
     return 0;
 }
 
-int launch_timestep(cav3d_ctx *c, hipStream_t st)
+int launch_timestep(cav3d_ctx *c)
 {
     DS &S = c->S;
-    hipLaunchKernelGGL(k_reset_scal, dim3(1), dim3(64), 0, st, S);
+    const hipStream_t st = c->st;
     hipLaunchKernelGGL(k_timestep, dim3(nblk(S.NC, 256)), dim3(256), 0, st, S);
     if (c->prm.local == 0) hipLaunchKernelGGL(k_dt_fill, dim3(nblk(S.NC, 256)), dim3(256), 0, st, S);
     hipLaunchKernelGGL(k_time_acc, dim3(1), dim3(64), 0, st, S);
@@ -1965,11 +1992,21 @@ int launch_timestep(cav3d_ctx *c, hipStream_t st)
 }
 
 // the sweeps' exchange arrays back to "not yet written"
-int launch_sweep_fills(cav3d_ctx *c, hipStream_t st)
+int launch_sweep_fills(cav3d_ctx *c)
 {
     DS &S = c->S;
     const long nq = (long)NPV * S.NW;
-    hipLaunchKernelGGL(k_sweep_reset, dim3(nblk(nq, 256)), dim3(256), 0, st, S.xqf, S.xqb, nq, c->ticket);
+    hipLaunchKernelGGL(k_sweep_reset, dim3(nblk(nq, 256)), dim3(256), 0, c->st, S, nq, c->ticket);
+    return 0;
+}
+
+// the face boundaries, the time step and the sweep resets
+int launch_begin(cav3d_ctx *c)
+{
+    DS &S = c->S;
+    const long nq = (long)NPV * S.NW;
+    const unsigned nbc = nblk(S.NBC[0], 256), nts = nblk(S.NC, 256);
+    hipLaunchKernelGGL(k_begin, dim3(nbc + nts + nblk(nq, 256)), dim3(256), 0, c->st, S, nbc, nts, nq, c->ticket);
     return 0;
 }
 
@@ -1990,14 +2027,8 @@ int launch_update(cav3d_ctx *c)
 {
     DS &S = c->S;
     hipLaunchKernelGGL(k_update, dim3(c->nwg_update), dim3(256), 0, c->st, S);
-    // the final norm reduction reads only the update's partials: it runs on
-    // a side stream beside the eddy viscosity, and reaches st again at the
-    // next residual's join (before the next update rewrites the partials);
-    // cav3d_residual waits for it
-    hipEventRecord(c->fork, c->st);
-    hipStreamWaitEvent(c->side[0], c->fork, 0);
-    hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(256), 0, c->side[0], S, c->nwg_update);
-    if (c->prm.iturb == 0) hipLaunchKernelGGL(k_eddy, dim3(nblk(S.NC, 128)), dim3(128), 0, c->st, S);
+    // the final norm reduction beside the eddy viscosity, which reads nothing of it
+    hipLaunchKernelGGL(k_finish, dim3(1 + (c->prm.iturb == 0 ? nblk(S.NC, 256) : 0)), dim3(256), 0, c->st, S, c->nwg_update);
     return 0;
 }
 
@@ -2158,6 +2189,9 @@ int cav3d_create(const cav3d_params *prm, int nblocks, const cav3d_block *blocks
         (rc = dalloc(c, &S.img, (long)RC_N * S.NW)) ||
         (rc = dalloc(c, &S.xqf, (long)NPV * S.NW)) || (rc = dalloc(c, &S.xqb, (long)NPV * S.NW)) ||
         (rc = dalloc(c, &S.scal, 32))) { cav3d_destroy(c); return rc; }
+    if (hipMemcpyAsync(S.scal, &DT_NONE, sizeof(DT_NONE), hipMemcpyHostToDevice, c->st) != hipSuccess) {
+        cav3d_destroy(c); return fail("device set-up failed", -3);
+    }
     for (int d = 0; d < 3; d++)
         if ((rc = dalloc(c, &S.ff[d], 2 * npv * S.NF[d]))) { cav3d_destroy(c); return rc; }
     if (prm->iturb == 0) {
@@ -2358,7 +2392,7 @@ int cav3d_setbc(cav3d_ctx *c)
 int cav3d_timestep(cav3d_ctx *c, int b, double *dt)
 {
     if (!c || b < 0 || b >= c->nb) return fail("bad argument to cav3d_timestep", -1);
-    launch_timestep(c, c->st);
+    launch_timestep(c);
     const BlkD &B = c->blk[b];
     if (dt) HIPCHK(hipMemcpyAsync(dt, c->S.dt + B.c0, B.nc * sizeof(double), hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
@@ -2398,17 +2432,16 @@ int cav3d_timeinteg(cav3d_ctx *c, int nt_phy, int nt, double timeprev, double *t
     (void)nt;
     if (!c) return fail("null context", -1);
     if (c->profile) hipEventRecord(c->ev[0], c->st);
-    // the time step and the sweeps' exchange-array fills read nothing the
-    // boundary fill writes (interior cells and metrics only): they run on the
-    // side streams meanwhile, joined again before the combine (launch_rhs),
-    // which precedes every reader of dt and of the exchange arrays
-    hipEventRecord(c->fork, c->st);
-    hipStreamWaitEvent(c->side[0], c->fork, 0);
-    hipStreamWaitEvent(c->side[1], c->fork, 0);
-    launch_sweep_fills(c, c->side[0]);
-    launch_timestep(c, c->side[1]);
+    // (a time step that all cells share takes another pass over dt)
+    const bool begun = c->prm.local != 0;
+    if (begun) {
+        launch_begin(c);
+    } else {
+        launch_sweep_fills(c);
+        launch_timestep(c);
+    }
     if (c->profile) hipEventRecord(c->ev[1], c->st);
-    launch_setbc(c);
+    launch_setbc(c, begun);
     if (c->profile) hipEventRecord(c->ev[2], c->st);
     launch_rhs(c);
     if (c->profile) hipEventRecord(c->ev[3], c->st);
@@ -2444,7 +2477,6 @@ int cav3d_residual(cav3d_ctx *c, double *l2, int *ijk, double *resmax)
 {
     if (!c) return fail("null context", -1);
     double h[32];
-    HIPCHK(hipStreamSynchronize(c->side[0]));     // the norms' final reduction
     HIPCHK(hipMemcpyAsync(h, c->S.scal, sizeof(h), hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
     int rc = sweep_status(c);

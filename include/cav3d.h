@@ -266,7 +266,8 @@ int cav3d_eos_host(int n, const double *p, const double *t, const double *y1, co
 
 /* Device time, in milliseconds, of the last cav3d_timeinteg's kernels by phase
  * (HIP events on the context's stream, recorded while enabled):
- * out[0] timestep, [1] boundary, [2] rhs, [3] lusgs, [4] update+eddy, [5] total,
+ * out[0] time step with the face boundaries (one launch), [1] interfaces, edges
+ * and corners, [2] rhs, [3] lusgs, [4] update+eddy, [5] total,
  * [6] forward sweep kernel, [7] backward sweep kernel; [8] the kernels of the
  * last cav3d_rhs_vjp, [9] those of the last cav3d_calrhs.  out holds 10 doubles. */
 int cav3d_profile(cav3d_ctx *ctx, int enable, double *out);
