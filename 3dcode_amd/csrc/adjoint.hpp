@@ -90,9 +90,9 @@ __device__ __forceinline__ bool face_exists(const BlkD &B, int D, int i, int j, 
 // right states (k_adj_stencil takes them to the stencil points), the cells'
 // property bars (first order) and the u_ref derivative.
 template <int D, bool SENSOR>
-__global__ __launch_bounds__(128) void k_face_vjp(DS S, AD A)
+__device__ __forceinline__ void face_vjp(const DS &S, const AD &A, unsigned wg)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    long t = (long)wg * blockDim.x + threadIdx.x;
     if (t >= S.NF[D]) return;
     int i, j, k;
     const BlkD &B = face_of<D>(S, t, i, j, k);
@@ -143,9 +143,9 @@ __global__ __launch_bounds__(128) void k_face_vjp(DS S, AD A)
 // the stencil, k_adj_stencil applies them), of the two cells' mu, kappa and,
 // under SST, rho, h_T and eddy viscosity.
 template <int D>
-__global__ __launch_bounds__(128) void k_vface_vjp(DS S, AD A)
+__device__ __forceinline__ void vface_vjp(const DS &S, const AD &A, unsigned wg)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    long t = (long)wg * blockDim.x + threadIdx.x;
     if (t >= S.NF[D]) return;
     int i, j, k;
     const BlkD &B = face_of<D>(S, t, i, j, k);
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(128) void k_vface_vjp(DS S, AD A)
     double dl[ND], dr[ND];
     for (int m = 0; m < ND; m++) { dl[m] = S.dc[m * S.NG + g9]; dr[m] = S.dc[m * S.NG + gq]; }
     const double ml = S.mut ? S.mut[g9] : 0.0, mr = S.mut ? S.mut[gq] : 0.0;
-    // metrics (as k_vface)
+    // metrics (as visc_face)
     double n3[3], e4[4][3], t4[4][3];
     face_vec(S, B, D, i, j, k, n3);
     const int E = (D + 1) % 3, T = (D + 2) % 3;
@@ -218,6 +218,24 @@ __global__ __launch_bounds__(128) void k_vface_vjp(DS S, AD A)
         vp[4 * NF + t] = o.ht[1];
         if (A.dmut) { A.mtb[D][t] = o.mut[0]; A.mtb[D][NF + t] = o.mut[1]; }
     }
+}
+
+// Every face's bars in one launch, the directions' inviscid parts and then
+// their viscous ones, as k_flux (all of them run one wavefront per SIMD).
+template <bool SENSOR>
+__global__ __launch_bounds__(128) void k_faces_vjp(DS S, AD A, FluxWgs g)
+{
+    unsigned w = blockIdx.x;
+    if (w < g.n[0]) { face_vjp<0, SENSOR>(S, A, w); return; }
+    w -= g.n[0];
+    if (w < g.n[1]) { face_vjp<1, SENSOR>(S, A, w); return; }
+    w -= g.n[1];
+    if (w < g.n[2]) { face_vjp<2, SENSOR>(S, A, w); return; }
+    w -= g.n[2];
+    if (w < g.n[0]) { vface_vjp<0>(S, A, w); return; }
+    w -= g.n[0];
+    if (w < g.n[1]) { vface_vjp<1>(S, A, w); return; }
+    vface_vjp<2>(S, A, w - g.n[1]);
 }
 
 // The stencil pass: one wavefront owns a tile of ghosted cells, one variable
@@ -664,32 +682,17 @@ int launch_vjp(cav3d_ctx *c, int dmut = 0)
     for (int d = 0; d < 3; d++) { A.tiles[d] = c->a_tiles[d]; A.ntiles[d] = c->a_ntiles[d]; A.pbd[d] = c->a_pbd + (long)d * S.npv * S.NG; }
     const bool sensor = S.P.nscheme == 2 || S.P.nscheme == 3;
     const int npv = S.npv;
-    // the faces' kernels are independent of each other: i on st, j and k on
-    // the side streams, joined before the stencil pass and the cell sources
-    // (which read every direction's eddy-viscosity bars); those two run
-    // beside each other and are joined before the cells' pass
-    hipStream_t sd[3] = {c->st, c->side[0], c->side[1]};
+    FluxWgs g;
+    for (int d = 0; d < 3; d++) g.n[d] = nblk(S.NF[d], 128);
+    const dim3 fg((g.n[0] + g.n[1] + g.n[2]) * (S.P.iturb >= -2 ? 2 : 1));
+    if (sensor) hipLaunchKernelGGL(k_faces_vjp<true>, fg, dim3(128), 0, c->st, S, A, g);
+    else hipLaunchKernelGGL(k_faces_vjp<false>, fg, dim3(128), 0, c->st, S, A, g);
+    // the stencil pass and the cell sources run beside each other and are
+    // joined before the cells' pass
     hipEventRecord(c->fork, c->st);
-    hipStreamWaitEvent(c->side[0], c->fork, 0);
-    hipStreamWaitEvent(c->side[1], c->fork, 0);
-#define CAV3D_VJP_DIR(D)                                                                                             \
-    do {                                                                                                             \
-        if (sensor) hipLaunchKernelGGL((k_face_vjp<D, true>), dim3(nblk(S.NF[D], 128)), dim3(128), 0, sd[D], S, A);  \
-        else hipLaunchKernelGGL((k_face_vjp<D, false>), dim3(nblk(S.NF[D], 128)), dim3(128), 0, sd[D], S, A);        \
-        if (S.P.iturb >= -2) hipLaunchKernelGGL((k_vface_vjp<D>), dim3(nblk(S.NF[D], 128)), dim3(128), 0, sd[D], S, A); \
-    } while (0)
-    CAV3D_VJP_DIR(1);
-    CAV3D_VJP_DIR(2);
-    CAV3D_VJP_DIR(0);
-#undef CAV3D_VJP_DIR
-    hipEventRecord(c->join[0], c->side[0]);
-    hipEventRecord(c->join[1], c->side[1]);
-    hipStreamWaitEvent(c->st, c->join[0], 0);
-    hipStreamWaitEvent(c->st, c->join[1], 0);
-    hipEventRecord(c->fork, c->st);
-    hipStreamWaitEvent(c->side[0], c->fork, 0);
-    if (S.P.ides > 0 || S.P.ncav >= 2) hipLaunchKernelGGL(k_cell_vjp<true>, dim3(nblk(S.NC, 128)), dim3(128), 0, c->side[0], S, A);
-    else hipLaunchKernelGGL(k_cell_vjp<false>, dim3(nblk(S.NC, 128)), dim3(128), 0, c->side[0], S, A);
+    hipStreamWaitEvent(c->side, c->fork, 0);
+    if (S.P.ides > 0 || S.P.ncav >= 2) hipLaunchKernelGGL(k_cell_vjp<true>, dim3(nblk(S.NC, 128)), dim3(128), 0, c->side, S, A);
+    else hipLaunchKernelGGL(k_cell_vjp<false>, dim3(nblk(S.NC, 128)), dim3(128), 0, c->side, S, A);
     const dim3 tg((unsigned)(npv * (c->a_ntiles[0] + c->a_ntiles[1] + c->a_ntiles[2])));
     auto stencil = [&](auto small) {
         constexpr bool SMALL = decltype(small)::value;
@@ -699,8 +702,8 @@ int launch_vjp(cav3d_ctx *c, int dmut = 0)
     };
     if (c->a_small) stencil(std::true_type());
     else stencil(std::false_type());
-    hipEventRecord(c->join[0], c->side[0]);
-    hipStreamWaitEvent(c->st, c->join[0], 0);
+    hipEventRecord(c->join, c->side);
+    hipStreamWaitEvent(c->st, c->join, 0);
     hipLaunchKernelGGL(k_adj_cells, dim3(nblk(S.NG, 128)), dim3(128), 0, c->st, S, A);
     return 0;
 }

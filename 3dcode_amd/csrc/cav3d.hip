@@ -11,7 +11,7 @@
 // One step (t_lusgs%timeinteg, src/update_module.f90:455-733):
 //   k_timestep            local dt + global min          (timestep_module)
 //   k_bc / k_halo         faces, interfaces, edges, corners (bc_module setbc)
-//   k_face<D>             reconstruction + EOS + inviscid/viscous face flux
+//   k_flux                reconstruction + EOS + inviscid/viscous face flux of the three directions
 //   k_combine             flux differences in the reference's i,j,k order
 //                         + Merkle / SST / BDF sources   (rhs_module calrhs)
 //   k_lhs_prep            sweep-independent terms of D^-1 and of the Jacobians
@@ -1675,10 +1675,10 @@ struct cav3d_ctx {
     std::vector<Con> cons;
     std::vector<std::vector<int>> bcdesc;   // per block: nbc*7 raw
     hipStream_t st = nullptr;
-    // the adjoint's j and k directions run on two more streams, forked from
-    // and joined back to st by events (default priority, like st)
-    hipStream_t side[2] = {};
-    hipEvent_t fork = nullptr, join[2] = {};
+    // the adjoint's cell sources run on another stream, forked from and
+    // joined back to st by events (default priority, like st)
+    hipStream_t side = nullptr;
+    hipEvent_t fork = nullptr, join = nullptr;
     int dev = 0;              // device current at creation (the context's device)
     double *stage = nullptr;
     size_t stage_n = 0;
@@ -2095,13 +2095,12 @@ int cav3d_create(const cav3d_params *prm, int nblocks, const cav3d_block *blocks
     P.emutref = prm->emutref;
     P.bdf_b = prm->nsteady == 1 ? 1.0 : (prm->nsteady == 2 ? 1.5 * 0.5 : 0.0);
     if (hipStreamCreate(&c->st) != hipSuccess) { delete c; return fail("hipStreamCreate failed", -3); }
-    for (int q = 0; q < 2; q++)
-        if (hipStreamCreateWithFlags(&c->side[q], hipStreamNonBlocking) != hipSuccess ||
-            hipEventCreateWithFlags(&c->join[q], hipEventDisableTiming) != hipSuccess) {
-            cav3d_destroy(c);
-            return fail("stream set-up failed", -3);
-        }
-    if (hipEventCreateWithFlags(&c->fork, hipEventDisableTiming) != hipSuccess) { cav3d_destroy(c); return fail("stream set-up failed", -3); }
+    if (hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreateWithFlags(&c->join, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&c->fork, hipEventDisableTiming) != hipSuccess) {
+        cav3d_destroy(c);
+        return fail("stream set-up failed", -3);
+    }
     DS &S = c->S;
     memset(&S, 0, sizeof(S));
     S.nb = nblocks;
@@ -2268,10 +2267,8 @@ void cav3d_destroy(cav3d_ctx *c)
     if (c->xbuf) hipFree(c->xbuf);
     if (c->a_obj) hipFree(c->a_obj);
     for (int q = 0; q < 14; q++) if (c->ev[q]) hipEventDestroy(c->ev[q]);
-    for (int q = 0; q < 2; q++) {
-        if (c->side[q]) { hipStreamSynchronize(c->side[q]); hipStreamDestroy(c->side[q]); }
-        if (c->join[q]) hipEventDestroy(c->join[q]);
-    }
+    if (c->side) { hipStreamSynchronize(c->side); hipStreamDestroy(c->side); }
+    if (c->join) hipEventDestroy(c->join);
     if (c->fork) hipEventDestroy(c->fork);
     if (c->st) hipStreamDestroy(c->st);
     delete c;
