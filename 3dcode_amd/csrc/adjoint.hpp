@@ -221,7 +221,7 @@ __device__ __forceinline__ void vface_vjp(const DS &S, const AD &A, unsigned wg)
 }
 
 // Every face's bars in one launch, the directions' inviscid parts and then
-// their viscous ones, as k_flux (all of them run one wavefront per SIMD).
+// their viscous ones, as k_face (all of them run one wavefront per SIMD).
 template <bool SENSOR>
 __global__ __launch_bounds__(128) void k_faces_vjp(DS S, AD A, FluxWgs g)
 {

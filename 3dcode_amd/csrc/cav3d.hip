@@ -9,15 +9,15 @@
 // reference calls the EOS.
 //
 // One step (t_lusgs%timeinteg, src/update_module.f90:455-733):
-//   k_timestep            local dt + global min          (timestep_module)
-//   k_bc / k_halo         faces, interfaces, edges, corners (bc_module setbc)
-//   k_flux                reconstruction + EOS + inviscid/viscous face flux of the three directions
+//   k_begin               face boundaries; local dt + global min (timestep_module)
+//   k_halo / k_bc         interfaces, edges, corners     (bc_module setbc)
+//   k_face                reconstruction + EOS + inviscid/viscous face flux of the three directions
 //   k_combine             flux differences in the reference's i,j,k order
 //                         + Merkle / SST / BDF sources   (rhs_module calrhs)
 //   k_lhs_prep            sweep-independent terms of D^-1 and of the Jacobians
 //   k_sweep_tile<fwd>     the L (U) sweep: tiles of i-pencils, hyperplane order,
 //                         LDS hand-over inside a tile, coherent polls across tiles
-//   k_update, k_eddy      pv += dq, clip, EOS, norms; SST eddy viscosity
+//   k_update, k_finish    pv += dq, clip, EOS, norms; SST eddy viscosity
 #include "phys.hpp"
 #include "../../include/cav3d.h"
 
@@ -697,17 +697,18 @@ __device__ __forceinline__ void visc_face(const DS &S, unsigned wg)
 
 // All fluxes in one launch: the inviscid faces of the three directions, then
 // the viscous ones (they write other halves of the face arrays), each
-// direction's workgroups filling the tail of the one before.  RV: the viscous
-// faces' arithmetic.  Six launches on three streams did the same, but an event
+// direction's workgroups filling the tail of the one before.  V32: the viscous
+// faces in FP32 where R is not (AUSMPW+ in the mixed mode).  Six launches on three streams did the same, but an event
 // between streams costs some 10 us, and an iteration had three forks and
 // joins: it took 210 us at 16x8x8 cells and 162 in single launches on one
 // stream, 64x32x32 448 and 404, 128x64x64 1695 and 1671; from a million cells
 // on the two were equal (the viscous faces run at two wavefronts per SIMD
 // here, three in a launch of their own).
 struct FluxWgs { unsigned n[3]; };       // workgroups of each direction
-template <bool SENSOR, class R, class RV>
-__global__ __launch_bounds__(BLK_WG) void k_flux(DS S, FluxWgs g)
+template <int V32, bool SENSOR, class R>
+__global__ __launch_bounds__(BLK_WG) void k_face(DS S, FluxWgs g)
 {
+    using RV = std::conditional_t<V32 != 0, float, R>;
     unsigned w = blockIdx.x;
     if (w < g.n[0]) { face_flux<0, SENSOR, R>(S, w); return; }
     w -= g.n[0];
@@ -1971,11 +1972,11 @@ int launch_rhs(cav3d_ctx *c)
     }
     const bool visc = c->prm.iturb >= -2;
     const dim3 grid((g.n[0] + g.n[1] + g.n[2]) * (visc ? 2 : 1)), block(BLK_WG);
-    if (sensor && mixed) hipLaunchKernelGGL((k_flux<true, float, float>), grid, block, 0, c->st, S, g);
-    else if (sensor && c->prm.precision == CAV3D_MIXED) hipLaunchKernelGGL((k_flux<true, double, float>), grid, block, 0, c->st, S, g);
-    else if (sensor) hipLaunchKernelGGL((k_flux<true, double, double>), grid, block, 0, c->st, S, g);
-    else if (mixed) hipLaunchKernelGGL((k_flux<false, float, float>), grid, block, 0, c->st, S, g);
-    else hipLaunchKernelGGL((k_flux<false, double, double>), grid, block, 0, c->st, S, g);
+    if (sensor && mixed) hipLaunchKernelGGL((k_face<0, true, float>), grid, block, 0, c->st, S, g);
+    else if (sensor && c->prm.precision == CAV3D_MIXED) hipLaunchKernelGGL((k_face<1, true, double>), grid, block, 0, c->st, S, g);
+    else if (sensor) hipLaunchKernelGGL((k_face<0, true, double>), grid, block, 0, c->st, S, g);
+    else if (mixed) hipLaunchKernelGGL((k_face<0, false, float>), grid, block, 0, c->st, S, g);
+    else hipLaunchKernelGGL((k_face<0, false, double>), grid, block, 0, c->st, S, g);
     if (S.P.ncav >= 2 || S.P.ides > 0) hipLaunchKernelGGL(k_combine<true>, dim3(nc), dim3(BLK_WG), 0, c->st, S);
     else hipLaunchKernelGGL(k_combine<false>, dim3(nc), dim3(BLK_WG), 0, c->st, S);
     return 0;
