@@ -19,16 +19,15 @@
 //                         LDS hand-over inside a tile, coherent polls across tiles
 //   k_update, k_finish    pv += dq, clip, EOS, norms; SST eddy viscosity
 #include "phys.hpp"
+#include "copyout.hpp"
 #include "../../include/cav3d.h"
 
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <array>
-#include <atomic>
 #include <cstdio>
 #include <cstring>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -1666,6 +1665,26 @@ inline unsigned nblk(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 }  // namespace
 
 // ============================================================ host context
+// the runtime calls of copyout.hpp
+struct HipCopy {
+    using Error = hipError_t;
+    using Event = hipEvent_t;
+    using Stream = hipStream_t;
+    using Thread = std::thread;
+    static constexpr Error OK = hipSuccess;
+    static Error alloc(char **p, size_t n) { return hipHostMalloc((void **)p, n, hipHostMallocDefault); }
+    static void release(char *p) { (void)hipHostFree(p); }
+    static Error event_create(Event *e) { return hipEventCreateWithFlags(e, hipEventDisableTiming); }
+    static void event_destroy(Event e) { (void)hipEventDestroy(e); }
+    static Error event_record(Event e, Stream st) { return hipEventRecord(e, st); }
+    static Error event_wait(Event e) { return hipEventSynchronize(e); }
+    static Error to_host(void *dst, const void *src, size_t n, Stream st) { return hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st); }
+    static Error stream_wait(Stream st) { return hipStreamSynchronize(st); }
+    static int device() { int d = 0; (void)hipGetDevice(&d); return d; }
+    static void set_device(int d) { (void)hipSetDevice(d); }
+    static void clear_error() { (void)hipGetLastError(); }
+};
+
 struct cav3d_ctx {
     cav3d_params prm;
     Par P;
@@ -1683,8 +1702,7 @@ struct cav3d_ctx {
     int dev = 0;              // device current at creation (the context's device)
     double *stage = nullptr;
     size_t stage_n = 0;
-    char *pin = nullptr;      // pinned staging of large results (copy_out), OUT_BUFS chunks
-    hipEvent_t pin_ev[8] = {};
+    CopyRing<HipCopy> ring;   // results to the caller (copy_out)
     int nwg_update = 0;
     int sweep_blocks = 0;     // grid of the sweep kernels: as many workgroups as fit the device at once
     int *tiles = nullptr;     // tile table of the sweeps (device): block, j0, k0, diagonal
@@ -1733,67 +1751,10 @@ int ensure_stage(cav3d_ctx *c, size_t n)
     return 0;
 }
 
-// Large device results to the caller's memory.  The copy of pageable memory
-// inside the runtime is a serial chain of a transfer to its staging buffer
-// and one thread's memcpy from it (20 and 70 us per chunk), the memcpy paying
-// the page faults of a fresh array as well.  Here OUT_THREADS threads each own
-// OUT_BUFS / OUT_THREADS pinned chunks of the context: a thread copies one out
-// while its next is being filled.  128x64x64: the state (47 MB) 2.75 -> 1.59
-// ms, the residual and its Jacobians (75 MB into fresh arrays, with the 0.9 ms
-// of the kernels) 8.6 -> 4.3 ms.
-// Below OUT_MIN the plain copy is the faster one (the threads cost some 50 us).
-constexpr int OUT_BUFS = 8, OUT_THREADS = 4;
-constexpr size_t OUT_CHUNK = 1u << 20, OUT_MIN = 4 * OUT_CHUNK;
 int copy_out(cav3d_ctx *c, void *dst, const void *src, size_t bytes)
 {
-    if (bytes >= OUT_MIN && !c->pin) {
-        bool ok = hipHostMalloc((void **)&c->pin, OUT_BUFS * OUT_CHUNK, hipHostMallocDefault) == hipSuccess;
-        for (int q = 0; ok && q < OUT_BUFS; q++) ok = hipEventCreateWithFlags(&c->pin_ev[q], hipEventDisableTiming) == hipSuccess;
-        if (!ok) {
-            (void)hipGetLastError();
-            if (c->pin) (void)hipHostFree(c->pin);
-            c->pin = nullptr;
-        }
-    }
-    if (bytes < OUT_MIN || !c->pin) {
-        HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->st));
-        HIPCHK(hipStreamSynchronize(c->st));
-        return 0;
-    }
-    const long n = (long)((bytes + OUT_CHUNK - 1) / OUT_CHUNK);
-    std::atomic<int> err{0};
-    auto size = [&](long q) { return std::min(OUT_CHUNK, bytes - (size_t)q * OUT_CHUNK); };
-    auto fill = [&](long q) {        // chunk q into its buffer
-        const int b = (int)(q % OUT_BUFS);
-        hipError_t e = hipMemcpyAsync(c->pin + b * OUT_CHUNK, (const char *)src + q * OUT_CHUNK, size(q), hipMemcpyDeviceToHost, c->st);
-        if (e == hipSuccess) e = hipEventRecord(c->pin_ev[b], c->st);
-        if (e != hipSuccess) err = (int)e;
-    };
-    for (long q = 0; q < std::min<long>(n, OUT_BUFS); q++) fill(q);
-    auto work = [&](int t) {         // chunks t, t + OUT_THREADS, ...
-        hipSetDevice(c->dev);
-        for (long q = t; q < n && !err; q += OUT_THREADS) {
-            const int b = (int)(q % OUT_BUFS);
-            const hipError_t e = hipEventSynchronize(c->pin_ev[b]);
-            if (e != hipSuccess) { err = (int)e; break; }
-            memcpy((char *)dst + q * OUT_CHUNK, c->pin + b * OUT_CHUNK, size(q));
-            if (q + OUT_BUFS < n) fill(q + OUT_BUFS);
-        }
-    };
-    std::thread th[OUT_THREADS - 1];
-    int started = 0;
-    try {
-        for (; started < OUT_THREADS - 1; started++) th[started] = std::thread(work, started + 1);
-    } catch (const std::system_error &) {
-    }
-    work(0);
-    for (int t = started + 1; t < OUT_THREADS; t++) work(t);      // the threads that could not be started
-    for (int t = 0; t < started; t++) th[t].join();
-    if (err) {
-        (void)hipStreamSynchronize(c->st);
-        return fail(std::string("copy to the host: ") + hipGetErrorString((hipError_t)err.load()), -3);
-    }
-    return 0;
+    const hipError_t e = c->ring.copy(c->st, c->dev, dst, src, bytes);
+    return e == hipSuccess ? 0 : fail(std::string("copy to the host: ") + hipGetErrorString(e), -3);
 }
 
 int wall_fn(int iturb) { return iturb == 0 ? FN_WALLVISKW : (iturb == -2 ? FN_WALLVIS : FN_WALLINV); }
@@ -2263,8 +2224,7 @@ void cav3d_destroy(cav3d_ctx *c)
     if (c->st) hipStreamSynchronize(c->st);
     for (void *p : c->allocs) hipFree(p);
     if (c->stage) hipFree(c->stage);
-    if (c->pin) hipHostFree(c->pin);
-    for (hipEvent_t e : c->pin_ev) if (e) hipEventDestroy(e);
+    c->ring.close();
     if (c->xbuf) hipFree(c->xbuf);
     if (c->a_obj) hipFree(c->a_obj);
     for (int q = 0; q < 14; q++) if (c->ev[q]) hipEventDestroy(c->ev[q]);

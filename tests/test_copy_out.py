@@ -1,0 +1,36 @@
+"""The copy of device results to the caller's memory (copyout.hpp) over
+runtime calls on the host (tests/native/copycheck.cpp): every size's bytes,
+and what a caller with several devices or a system out of memory, events or
+threads is left with."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+MB = 1 << 20
+SIZES = [1, 4 * MB - 1, 4 * MB, 8 * MB, 8 * MB + 1, 13 * MB + 4567]   # the plain copy, its edge, the ring with and without refills
+
+
+@pytest.fixture(scope="module")
+def copy(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("copy") / "libcopycheck.so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-pthread", os.path.join(HERE, "native", "copycheck.cpp"),
+                    "-o", so], check=True)
+    L = C.CDLL(so)
+    L.cc_copy.argtypes = [C.c_long] + [C.c_int] * 6 + [C.POINTER(C.c_int)]
+
+    def run(n, dev=0, caller=0, bad_event=-1, bad_thread=-1, bad_kind=0, again=1):
+        out = (C.c_int * 6)()
+        L.cc_copy(n, dev, caller, bad_event, bad_thread, bad_kind, again, out)
+        return dict(zip(("error", "copied", "device", "events", "pinned", "waits"), out))
+    return run
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_callers_device_stays(copy, n):
+    """A context on device 0 called from a thread whose device is 1."""
+    r = copy(n, dev=0, caller=1)
+    assert (r["error"], r["copied"], r["device"]) == (0, 1, 1)
+    assert r["events"] == 0 and r["pinned"] == 0
