@@ -36,8 +36,7 @@ template <class A> struct CopyRing {
         for (int q = 0; ok && q < BUFS; q++) ok = A::event_create(&ev[q]) == A::OK;
         if (!ok) {
             A::clear_error();
-            if (pin) A::release(pin);
-            pin = nullptr;
+            close();
         }
         if (cur != dev) A::set_device(cur);
         return ok;
@@ -46,7 +45,11 @@ template <class A> struct CopyRing {
     void close()
     {
         if (pin) A::release(pin);
-        for (auto &e : ev) if (e) A::event_destroy(e);
+        pin = nullptr;
+        for (auto &e : ev) {
+            if (e) A::event_destroy(e);
+            e = {};
+        }
     }
 
     // src (device dev, ordered behind what is on st) into dst, complete on return

@@ -34,3 +34,17 @@ def test_callers_device_stays(copy, n):
     r = copy(n, dev=0, caller=1)
     assert (r["error"], r["copied"], r["device"]) == (0, 1, 1)
     assert r["events"] == 0 and r["pinned"] == 0
+
+
+@pytest.mark.parametrize("bad", [0, 3, 7])
+def test_no_events_left_when_one_cannot_be_made(copy, bad):
+    """The plain copy takes over, and neither buffers nor events stay."""
+    r = copy(13 * MB + 4567, bad_event=bad, again=0)
+    assert (r["error"], r["copied"]) == (0, 1)
+    assert (r["events"], r["pinned"]) == (0, 0)
+
+
+def test_ring_opened_after_a_failed_attempt(copy):
+    r = copy(13 * MB + 4567, bad_event=3, again=2)
+    assert (r["error"], r["copied"]) == (0, 1)
+    assert (r["events"], r["pinned"]) == (0, 0)
