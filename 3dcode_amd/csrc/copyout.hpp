@@ -15,7 +15,6 @@
 #include <atomic>
 #include <cstddef>
 #include <cstring>
-#include <system_error>
 
 namespace cav {
 
@@ -87,7 +86,7 @@ template <class A> struct CopyRing {
         int started = 0;
         try {
             for (; started < THREADS - 1; started++) th[started] = typename A::Thread(other, started + 1);
-        } catch (const std::system_error &) {
+        } catch (...) {                  // (no thread: std::system_error; no memory for its state: std::bad_alloc)
         }
         work(0);
         for (int t = started + 1; t < THREADS; t++) work(t);      // the threads that could not be started

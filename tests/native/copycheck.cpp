@@ -3,6 +3,7 @@
 #include "../../3dcode_amd/csrc/copyout.hpp"
 #include <mutex>
 #include <new>
+#include <system_error>
 #include <thread>
 #include <vector>
 

@@ -48,3 +48,12 @@ def test_ring_opened_after_a_failed_attempt(copy):
     r = copy(13 * MB + 4567, bad_event=3, again=2)
     assert (r["error"], r["copied"]) == (0, 1)
     assert (r["events"], r["pinned"]) == (0, 0)
+
+
+@pytest.mark.parametrize("kind", ["no thread", "no memory"])
+@pytest.mark.parametrize("started", [0, 1, 2])
+def test_threads_that_cannot_be_started(copy, kind, started):
+    """The calling thread does their share; nothing leaves the C entry."""
+    r = copy(13 * MB + 4567, bad_thread=started, bad_kind=["no thread", "no memory"].index(kind) + 1, again=0)
+    assert (r["error"], r["copied"]) == (0, 1)
+    assert (r["events"], r["pinned"]) == (0, 0)
