@@ -1680,6 +1680,15 @@ struct HipCopy {
     static Error event_wait(Event e) { return hipEventSynchronize(e); }
     static Error to_host(void *dst, const void *src, size_t n, Stream st) { return hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st); }
     static Error stream_wait(Stream st) { return hipStreamSynchronize(st); }
+    // memory the runtime knows nothing of (a failed launch before is left for its own check to report)
+    static bool pageable(const void *p)
+    {
+        if (hipPeekAtLastError() != hipSuccess) return true;
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+        (void)hipGetLastError();
+        return true;
+    }
     static int device() { int d = 0; (void)hipGetDevice(&d); return d; }
     static void set_device(int d) { (void)hipSetDevice(d); }
     static void clear_error() { (void)hipGetLastError(); }

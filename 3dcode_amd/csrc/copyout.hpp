@@ -9,7 +9,10 @@
 // thread copies one out while its next is being filled.  128x64x64: the state
 // (47 MB) 2.75 -> 1.59 ms, the residual and its Jacobians (75 MB into fresh
 // arrays, with the 0.9 ms of the kernels) 8.6 -> 4.3 ms.
-// Below MIN the plain copy is the faster one (the threads cost some 50 us).
+// Below MIN the plain copy is the faster one (the threads cost some 50 us), and
+// so it is into memory the runtime knows: a transfer into pinned memory goes
+// straight there (the same state 0.92 ms, 1.59 through the chunks), and device
+// memory is not a thread's to write.
 #pragma once
 #include <algorithm>
 #include <atomic>
@@ -54,8 +57,7 @@ template <class A> struct CopyRing {
     // src (device dev, ordered behind what is on st) into dst, complete on return
     Error copy(typename A::Stream st, int dev, void *dst, const void *src, size_t bytes)
     {
-        if (bytes >= MIN && !pin) open(dev);
-        if (bytes < MIN || !pin) {
+        if (bytes < MIN || !A::pageable(dst) || (!pin && !open(dev))) {
             const Error e = A::to_host(dst, src, bytes, st);
             return e == A::OK ? A::stream_wait(st) : e;
         }

@@ -11,7 +11,8 @@ namespace {
 
 std::mutex lock;
 thread_local int current = 0;                 // the thread's device
-int events, pinned, waits, fail_event, fail_thread, thread_error;
+int events, pinned, waits, copies, fail_event, fail_thread, thread_error;
+const char *known = nullptr;                  // memory the runtime knows
 
 struct Host {
     using Error = int;
@@ -42,7 +43,8 @@ struct Host {
     static void event_destroy(Event e) { events--; delete e; }
     static Error event_record(Event e, Stream st) { return e->dev == st ? OK : 400; }
     static Error event_wait(Event) { return OK; }
-    static Error to_host(void *d, const void *s, size_t n, Stream) { memcpy(d, s, n); return OK; }
+    static bool pageable(const void *p) { return p != known; }
+    static Error to_host(void *d, const void *s, size_t n, Stream) { copies++; memcpy(d, s, n); return OK; }
     static Error stream_wait(Stream) { waits++; return OK; }
     static int device() { return current; }
     static void set_device(int d) { current = d; }
@@ -54,15 +56,17 @@ struct Host {
 extern "C" {
 
 // one copy of the given size; out = {error, copied, the caller's device afterwards,
-// events and pinned buffers alive after close, stream waits}
-void cc_copy(long bytes, int dev, int caller, int bad_event, int bad_thread, int bad_kind, int again, int *out)
+// events and pinned buffers alive after close, stream waits, transfers}; registered:
+// into memory the runtime knows
+void cc_copy(long bytes, int dev, int caller, int bad_event, int bad_thread, int bad_kind, int again, int registered, int *out)
 {
-    events = pinned = waits = 0;
+    events = pinned = waits = copies = 0;
     fail_event = bad_event;
     fail_thread = bad_thread;
     thread_error = bad_kind;
     std::vector<unsigned char> a(bytes), b(bytes, 0);
     for (long q = 0; q < bytes; q++) a[q] = (unsigned char)(q * 131 + (q >> 12));
+    known = registered ? (const char *)b.data() : nullptr;
     const int before = current;
     current = caller;
     cav::CopyRing<Host> r;
@@ -75,7 +79,7 @@ void cc_copy(long bytes, int dev, int caller, int bad_event, int bad_thread, int
     }
     out[2] = current;
     r.close();
-    out[3] = events; out[4] = pinned; out[5] = waits;
+    out[3] = events; out[4] = pinned; out[5] = waits; out[6] = copies;
     current = before;
 }
 
