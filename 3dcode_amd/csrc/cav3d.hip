@@ -1760,9 +1760,9 @@ int ensure_stage(cav3d_ctx *c, size_t n)
     return 0;
 }
 
-int copy_out(cav3d_ctx *c, void *dst, const void *src, size_t bytes)
+int copy_out(cav3d_ctx *c, void *dst, const void *src, size_t bytes, bool wait = true)
 {
-    const hipError_t e = c->ring.copy(c->st, c->dev, dst, src, bytes);
+    const hipError_t e = c->ring.copy(c->st, c->dev, dst, src, bytes, wait);
     return e == hipSuccess ? 0 : fail(std::string("copy to the host: ") + hipGetErrorString(e), -3);
 }
 
@@ -2483,7 +2483,7 @@ int cav3d_eos(cav3d_ctx *c, int n, const double *p, const double *t, const doubl
     HIPCHK(hipMemcpyAsync(d + 3L * n, y2, n * 8, hipMemcpyHostToDevice, c->st));
     hipLaunchKernelGGL(k_eos_points, dim3(nblk(n, 128)), dim3(128), 0, c->st, c->P, n, (const double *)d, (const double *)(d + n),
                        (const double *)(d + 2L * n), (const double *)(d + 3L * n), d + 4L * n, d + 22L * n);
-    if ((rc = copy_out(c, dv, d + 4L * n, 18L * n * 8)) || (rc = copy_out(c, tv, d + 22L * n, 2L * n * 8))) return rc;
+    if ((rc = copy_out(c, dv, d + 4L * n, 18L * n * 8, false)) || (rc = copy_out(c, tv, d + 22L * n, 2L * n * 8))) return rc;
     return check_launch("cav3d_eos");
 }
 

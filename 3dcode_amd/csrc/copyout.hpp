@@ -54,12 +54,13 @@ template <class A> struct CopyRing {
         }
     }
 
-    // src (device dev, ordered behind what is on st) into dst, complete on return
-    Error copy(typename A::Stream st, int dev, void *dst, const void *src, size_t bytes)
+    // src (device dev, ordered behind what is on st) into dst, complete on
+    // return unless wait is false: then a later copy's wait may be the one that completes it
+    Error copy(typename A::Stream st, int dev, void *dst, const void *src, size_t bytes, bool wait = true)
     {
         if (bytes < MIN || !A::pageable(dst) || (!pin && !open(dev))) {
             const Error e = A::to_host(dst, src, bytes, st);
-            return e == A::OK ? A::stream_wait(st) : e;
+            return e == A::OK && wait ? A::stream_wait(st) : e;
         }
         const long n = (long)((bytes + CHUNK - 1) / CHUNK);
         std::atomic<Error> err{A::OK};

@@ -57,7 +57,7 @@ extern "C" {
 
 // one copy of the given size; out = {error, copied, the caller's device afterwards,
 // events and pinned buffers alive after close, stream waits, transfers}; registered:
-// into memory the runtime knows
+// into memory the runtime knows; again: further copies, or -1 for one more in two parts
 void cc_copy(long bytes, int dev, int caller, int bad_event, int bad_thread, int bad_kind, int again, int registered, int *out)
 {
     events = pinned = waits = copies = 0;
@@ -78,6 +78,13 @@ void cc_copy(long bytes, int dev, int caller, int bad_event, int bad_thread, int
         out[1] = out[1] && a == b;
     }
     out[2] = current;
+    if (again < 0) {                          // two results of one call, the first not waited for by itself
+        std::fill(b.begin(), b.end(), 0);
+        waits = 0;
+        const long n1 = bytes / 2;
+        out[0] = r.copy(dev, dev, b.data(), a.data(), (size_t)n1, false) || r.copy(dev, dev, b.data() + n1, a.data() + n1, (size_t)(bytes - n1));
+        out[1] = out[1] && a == b;
+    }
     r.close();
     out[3] = events; out[4] = pinned; out[5] = waits; out[6] = copies;
     current = before;

@@ -66,6 +66,13 @@ def test_memory_the_runtime_knows_is_copied_to_at_once(copy, n):
     assert (r["error"], r["copied"], r["copies"], r["waits"]) == (0, 1, 1, 1)
 
 
+@pytest.mark.parametrize("n", [2, 3200, 4 * MB])
+def test_two_small_results_wait_once(copy, n):
+    """The results of one call, each below the chunked copy's smallest size."""
+    r = copy(n, again=-1)
+    assert (r["error"], r["copied"], r["waits"]) == (0, 1, 1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("where", ["pinned", "device"])
 @pytest.mark.parametrize("cells", [(8, 6, 6), (40, 40, 40)])
