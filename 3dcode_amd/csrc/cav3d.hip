@@ -20,6 +20,7 @@
 //   k_update, k_finish    pv += dq, clip, EOS, norms; SST eddy viscosity
 #include "phys.hpp"
 #include "copyout.hpp"
+#include "sweep_rows.hpp"
 #include "../../include/cav3d.h"
 
 #include <hip/hip_runtime.h>
@@ -818,25 +819,6 @@ __global__ __launch_bounds__(BLK_WG) void k_combine(DS S)
 }
 
 // ------------------------------------------------------------ LU-SGS sweeps
-// What a sweep step reads of a cell lies side by side in memory, in a record
-// of 92 doubles (736 bytes, 46 pieces of 16), ranges and order of the dcv
-// array of the reference (1:I+1 and so on; the outer layer stays zero and is
-// what a pencil's absent neighbours read):
-//   RC_FP, RC_FM  the +i,+j,+k (-i,-j,-k) faces x (+-n3[3], +-u, lam, vis) / 2:
-//                 the forward (backward) sweep's split Jacobians with their
-//                 sign and factor (exact: a power of two)
-//   RC_Q          the Jacobian's cell terms, in both sweeps
-//   RC_GX         the diagonal-inverse terms
-//   RC_RES        the residual; the forward sweep puts its dcv there
-// Field by field, the sweeps gathered 128 numbers a cell (the shared ones
-// once for each of the three pencils that read them) in 32-byte pieces of
-// 128-byte lines: 1.46 GB a forward sweep at 128x64x64, sixteen 64-lane
-// transfers of 32 lines each a step, whose issue was the length of a step.
-// Now it is 86 numbers a cell in whole lines and eleven transfers.
-enum { RC_FP = 0, RC_FM = 18, RC_Q = 36, RC_GX = 54, RC_RES = RC_GX + NGX, RC_N = RC_RES + NPV };
-enum { Q_RP = 0, Q_RT, Q_RY1, Q_RY2, Q_RHO, Q_BETA, Q_HP, Q_HT, Q_HY1, Q_HY2, Q_U, Q_V, Q_W, Q_Y1, Q_Y2, Q_K, Q_O, Q_H };
-static_assert(RC_GX - RC_Q == Q_H + 1 && RC_N == 92, "record layout");
-
 // Per-cell terms of the LU-SGS operator that do not depend on the sweep:
 // the diagonal-inverse coefficients and the Jacobian's cell and face terms
 // (src/lhs_module.f90:346-457, src/jacobian_module.f90:182-403), written as
@@ -865,22 +847,7 @@ __global__ __launch_bounds__(128) void k_lhs_prep(DS S)
     if (P.ncav) for (int m = 0; m < 4; m++) ic[m] = S.icav[m * S.NC + tc];
     if (P.iturb == 0) for (int m = 0; m < 4; m++) it[m] = S.itt[m * S.NC + tc];
     double r[RC_N];
-    for (int q = 0; q < 6; q++) {
-        const JacFace f = jac_face(P, cc, f6[q]);
-        double *o = r + ((q & 1) ? RC_FP : RC_FM) + 6 * (q >> 1);
-        const double h = (q & 1) ? 0.5 : -0.5;
-        o[0] = h * f6[q][0]; o[1] = h * f6[q][1]; o[2] = h * f6[q][2];
-        o[3] = h * f.u; o[4] = 0.5 * f.lam; o[5] = 0.5 * f.vis;
-    }
-    const JacCell jc = jac_cell(P, cc);
-    double *const c = r + RC_Q;
-    c[Q_RP] = cc.d[D_RP]; c[Q_RT] = cc.d[D_RT]; c[Q_RY1] = cc.d[D_RY1]; c[Q_RY2] = cc.d[D_RY2];
-    c[Q_RHO] = cc.d[D_RHO]; c[Q_BETA] = jc.beta;
-    c[Q_HP] = cc.d[D_HP]; c[Q_HT] = cc.d[D_HT]; c[Q_HY1] = cc.d[D_HY1]; c[Q_HY2] = cc.d[D_HY2];
-    c[Q_U] = cc.pv[1]; c[Q_V] = cc.pv[2]; c[Q_W] = cc.pv[3]; c[Q_Y1] = cc.pv[5]; c[Q_Y2] = cc.pv[6];
-    c[Q_K] = S.npv > 7 ? cc.pv[7] : 0.0; c[Q_O] = S.npv > 7 ? cc.pv[8] : 0.0;
-    c[Q_H] = jc.h;
-    getx_prep(P, S.npv, cc, f6, S.dt[tc], ic, it, r + RC_GX);
+    cell_record(P, S.npv, cc, f6, S.dt[tc], ic, it, r);
     for (int n = 0; n < NPV; n++) r[RC_RES + n] = n < S.npv ? S.res[n * S.NC + tc] : 0.0;
 #pragma unroll
     for (int c0 = 0; c0 < RC_N; c0 += CH) {
@@ -951,159 +918,16 @@ constexpr int TJ = 4, TK = 4;
 // that uses it).  A ring of SLABS hyperplanes: a step reads its own slab and
 // the next one while the ones after are on their way.  The steps are unrolled
 // over the ring, so that the places are constants of the LDS reads.
-enum {
-    SP_F = 0, SP_Q = 18, SP_GX = 36, SP_RES = SP_GX + NGX, SP_N = SP_RES + NPV,
-    SE_F = 0, SE_Q = 6, SE_N = 24,
-    SLAB_E = TJ * TK * SP_N, SLAB_USED = SLAB_E + (TJ + TK) * SE_N,
-    SLAB_LOADS = (SLAB_USED + 127) / 128, SLAB_N = 128 * SLAB_LOADS
-};
+enum { SLAB_E = TJ * TK * SP_N, SLAB_USED = SLAB_E + (TJ + TK) * SE_N, SLAB_LOADS = (SLAB_USED + 127) / 128, SLAB_N = 128 * SLAB_LOADS };
 constexpr int SLABS = 5;
-static_assert(SP_N == RC_N - 18 && SP_RES - SP_GX == RC_RES - RC_GX && SP_GX - SP_Q == RC_GX - RC_Q, "stage layout");
 
-// lane q of the lane's 16-lane row, by one 64-bit DPP move (no LDS traffic)
-template <int Q>
-__device__ __forceinline__ double row_lane(double v)
-{
-    return __longlong_as_double(__builtin_amdgcn_mov_dpp(__double_as_longlong(v), 0x150 + Q, 0xF, 0xF, false));
-}
-// Row form of a pencil's step.  A pencil's 16 lanes hold the rows of its
-// cell's system; everything else a step reads (the state, properties, face
-// and diagonal-inverse terms: some 90 numbers a cell) is the same for all
-// lanes.  The lanes read them from the stage one item each (lane l its own
-// items, RowMap) and pass them around with DPP row broadcasts.  Reading every
-// item into every lane took 140 LDS reads a step, whose return path (each
-// read brings 64 lanes x 8 bytes at 128 bytes a clock for the four pencil
-// wavefronts of the CU) bound the step.  Now it is 39, and the terms that are
-// one expression per column are formed once, a column per lane, not in every
-// lane.  What a lane needs another operand for than its neighbours it reads
-// from another place rather than selecting among broadcasts.
-struct RowMap {
-    int v1, a, lb, v2, p, g[7], co[3];     // stage items of this lane, within its pencil's part of a slab
-    bool face, aface;               // v1 (and lb), a: items of F (of the i face; the j and k faces' lie 6 and 12 further)
-    double one[7];                  // 1 in the lane of the column
-    double en, kw, men, mom;        // 1 in lane 4, 1 in the lanes of k and omega, -1 in lane 4, 1 in lanes 1..3
-    bool m13, cpl, n0, n4, n5, n7, n8;
+// lane Q of the lane's 16-lane row, by one 64-bit DPP move (no LDS traffic)
+struct Dpp {
+    template <int Q> __device__ __forceinline__ static double lane(double v)
+    {
+        return __longlong_as_double(__builtin_amdgcn_mov_dpp(__double_as_longlong(v), 0x150 + Q, 0xF, 0xF, false));
+    }
 };
-__device__ __forceinline__ RowMap row_map(int lane, int npv)
-{
-    RowMap m;
-    m.m13 = lane >= 1 && lane <= 3;
-    // lanes 0..6: the column's factor of r1 (rho_p, n3, rho_T, rho_y1, rho_y2); lane 13: rho
-    m.face = m.m13;
-    m.v1 = m.m13 ? SP_F + lane - 1 : SP_Q + (lane == 0 ? Q_RP : lane == 4 ? Q_RT : lane == 5 ? Q_RY1 : lane == 6 ? Q_RY2 : Q_RHO);
-    // u, followed by lam and vis; in lanes 1..3 rho
-    m.aface = !m.m13;
-    m.a = m.m13 ? SP_Q + Q_RHO : SP_F + 3;
-    // the factor of lam: in lane 0 beta, else that of u and vis
-    m.lb = lane == 0 ? SP_Q + Q_BETA : m.v1;
-    // lanes 0..6: the column's factor in the energy row (h_p, u, v, w, h_T, h_y1, h_y2)
-    m.v2 = SP_Q + (lane == 0 ? Q_HP : lane <= 3 ? Q_U + lane - 1 : lane == 4 ? Q_HT : lane == 5 ? Q_HY1 : Q_HY2);
-    // the row's own factor: pv(n), in the energy row the total enthalpy
-    // (lane 0 and the lanes without a row read one that they do not use)
-    m.p = SP_Q + (m.m13 ? Q_U + lane - 1 : lane == 4 ? Q_H : lane >= 5 && lane <= 8 ? Q_Y1 + lane - 5 : Q_U);
-    // the row's entries of D^-1 (getx_apply): k1..k4, e1, e2, f1
-    m.n0 = lane == 0; m.n4 = lane == 4; m.n5 = lane == 5; m.n7 = lane == 7; m.n8 = lane == 8;
-    m.cpl = m.n0 || m.n4 || m.n5;
-    const bool row7 = lane >= 7;
-    m.g[0] = SP_GX + (m.n0 ? GX_C4C1 : m.n4 ? GX_C4IB1S1 : m.n7 ? GX_RBT4 : m.n8 ? GX_RBT1 : GX_C4SSIB1);
-    m.g[1] = SP_GX + (m.n0 ? GX_C2 : m.n4 ? GX_C1 : m.n7 ? GX_T2 : m.n8 ? GX_T3 : GX_SS);
-    m.g[2] = SP_GX + (m.n0 ? GX_C3 : m.n4 ? GX_C3IB1 : GX_C1);
-    m.g[3] = SP_GX + (m.n0 ? GX_RB1 : GX_C2IB1);
-    m.g[4] = SP_GX + (m.n0 ? GX_CROSS1 : GX_S1P5);
-    m.g[5] = SP_GX + (m.n0 ? GX_CP5 : GX_SSY1);
-    m.g[6] = SP_GX + (m.cpl ? GX_MM : row7 ? GX_IT : GX_IB1);
-    // lanes 0, 1, 2: the three sums res0 a + b uuu + c res6 that rows 0, 4, 5 share
-    m.co[0] = SP_GX + (lane == 0 ? GX_AAA1 : lane == 1 ? GX_AAA2 : GX_SSHM);
-    m.co[1] = lane == 0 ? SP_Q + Q_RY1 : lane == 1 ? SP_Q + Q_RT : SP_GX + GX_RRR;
-    m.co[2] = SP_GX + (lane == 0 ? GX_CROSS : lane == 1 ? GX_CROSS2 : GX_SSY2);
-    for (int l = 0; l < 7; l++) m.one[l] = lane == l ? 1.0 : 0.0;
-    m.en = m.one[4]; m.men = -m.one[4];
-    m.mom = m.m13 ? 1.0 : 0.0;
-    m.kw = row7 && lane < npv ? 1.0 : 0.0;
-    return m;
-}
-
-// A lane's Jacobian items of a cell and face (RowMap): v1, u (rho in lanes
-// 1..3), lam, vis, the factor of lam, v2, p
-struct RowJac {
-    double v1, a, b, c, lb, v2, p;
-};
-
-// Row coefficients of one neighbour's split Jacobian, c[l] = +-0.5 a(n,l)
-// (jac_row's products and sums in its order; jac_row_coef has the same row by
-// row): r1[l] and the energy row's factor of column l sit in lane l.  The
-// factor 0.5 and the sign are in u, lam, vis and n3 already, which they pass
-// through exactly.  A term that only some rows have is added as
-// fma(term, 1 or 0, sum), which rounds as the sum.
-__device__ __forceinline__ void row_coef(const RowMap &m, const RowJac &j, double *c)
-{
-    const double t0 = j.a * j.v1, t = t0 + j.b * j.lb + j.c * j.v1, r = m.m13 ? t0 : t;
-    // (lane 13 holds rho, u, lam and vis; the broadcasts stay out of the
-    // selects: they need every lane active)
-    const double ru = row_lane<13>(j.v1 * (j.a + j.b + j.c));
-    const double P = m.n0 ? 1.0 : j.p, Q = ru * m.en;
-    c[0] = P * row_lane<0>(r) + Q * row_lane<0>(j.v2);
-    c[1] = P * row_lane<1>(r) + Q * row_lane<1>(j.v2);
-    c[2] = P * row_lane<2>(r) + Q * row_lane<2>(j.v2);
-    c[3] = P * row_lane<3>(r) + Q * row_lane<3>(j.v2);
-    c[4] = P * row_lane<4>(r) + Q * row_lane<4>(j.v2);
-    c[5] = P * row_lane<5>(r) + Q * row_lane<5>(j.v2);
-    c[6] = P * row_lane<6>(r) + Q * row_lane<6>(j.v2);
-    // the pressure column: n3 in the momentum rows, -lam, then -vis in the energy row
-    c[0] = fma(j.v1, m.mom, c[0]);
-    c[0] = fma(j.b, m.men, c[0]);
-    c[0] = fma(j.c, m.men, c[0]);
-#pragma unroll
-    for (int l = 1; l < 7; l++) if (l != 4) c[l] = fma(ru, m.one[l], c[l]);
-    c[7] = ru * m.kw;
-}
-
-// y += c x, the neighbour's row n in lane n (jac_row_apply)
-__device__ __forceinline__ void row_apply(const double *c, double x, double &y)
-{
-    y = y + c[0] * row_lane<0>(x);
-    y = y + c[1] * row_lane<1>(x);
-    y = y + c[2] * row_lane<2>(x);
-    y = y + c[3] * row_lane<3>(x);
-    y = y + c[4] * row_lane<4>(x);
-    y = y + c[5] * row_lane<5>(x);
-    y = y + c[6] * row_lane<6>(x);
-    y = y + c[7] * x;
-}
-
-// What a step reads of its own cell, read during the step before: the rows'
-// residual, the Jacobian items, the rows' D^-1 entries
-struct RowCell {
-    RowJac j;
-    double res, g[7], a, co[3];
-};
-
-// Row n of D^-1 y in lane n (y: the row's right-hand side).  Rows 0, 4 and 5
-// are sums of four products, rows 7 and 8 of two, the rest one difference:
-// every row forms ((k1 x1 + k2 x2) + k3 x3) + k4 ((x4 + e1 z1) + e2 z2) with
-// its own entries and operands and takes the partial sum it needs.
-// Subtractions are sums with the entry's sign flipped, so the operations and
-// their order are getx_apply's.
-__device__ __forceinline__ double row_dinv(const RowMap &m, const RowCell &c, double y)
-{
-    auto neg = [](double x, bool f) { return __longlong_as_double(__double_as_longlong(x) ^ (long long)((unsigned long long)f << 63)); };
-    const double y0 = row_lane<0>(y), y5 = row_lane<5>(y), y6 = row_lane<6>(y);
-    const double s1 = y - y0 * c.j.p;
-    const double r6 = row_lane<6>(s1), rk = row_lane<7>(s1), ro = row_lane<8>(s1);
-    const double uuu = row_lane<1>(y) * row_lane<1>(c.j.v2) + row_lane<2>(y) * row_lane<2>(c.j.v2)
-                     + row_lane<3>(y) * row_lane<3>(c.j.v2) - row_lane<4>(y);
-    const double co = y0 * c.co[0] + c.co[1] * uuu + c.co[2] * y6;
-    const double co1 = row_lane<0>(co), co2 = row_lane<1>(co), co3 = row_lane<2>(co);
-    const bool row7 = m.n7 || m.n8;
-    const double x1 = row7 ? s1 : r6;
-    const double x2 = m.n5 ? s1 : m.n7 ? ro : m.n8 ? rk : co1;
-    const double x3 = m.n4 ? co3 : co2, x4 = m.n0 ? co2 : co3;
-    const double z1 = m.n0 ? y5 : y0, z2 = m.n0 ? y0 : y5;
-    const double s2 = neg(c.g[0], !m.n4) * x1 + neg(c.g[1], m.n0) * x2;
-    const double w = x4 + neg(c.g[4], !m.n0) * z1 + neg(c.g[5], m.n0) * z2;
-    const double s4 = s2 + neg(c.g[2], !m.n0) * x3 + (m.n4 ? -1.0 : c.g[3]) * (m.n5 ? x4 : w);
-    return (m.cpl ? s4 : row7 ? s2 : s1) * c.g[6] * c.a;
-}
 
 // Workgroup barrier for LDS hand-over: this wavefront's LDS accesses are
 // complete (lgkmcnt), nothing else is waited for, so global loads and the
@@ -1188,13 +1012,13 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             int at[SLAB_LOADS];                  // its cell is at - 1 past the pencil's first zero record in sweep order
 #pragma unroll
             for (int t = 0; t < SLAB_LOADS; t++) {
-                const int u = 64 * t + l, F = FWD ? RC_FP : RC_FM;
+                const int u = 64 * t + l;
                 int jj, kk, jn, kn, q, early;
                 if (u < TJ * TK * SP_N / 2) {
                     const int g = u / (SP_N / 2), c = u % (SP_N / 2);
                     jj = jn = j0 + g % TJ;
                     kk = kn = k0 + g / TJ;
-                    q = 2 * c < SP_Q ? F + 2 * c : RC_Q + 2 * c - SP_Q;
+                    q = stage_item(FWD, 2 * c);
                     early = 0;
                 } else {
                     const int v = u - TJ * TK * SP_N / 2, e = min(v / (SE_N / 2), TJ + TK - 1), c = v % (SE_N / 2);
@@ -1203,7 +1027,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
                     kk = k0 + (!a ? e : FWD ? 0 : TK - 1);
                     jn = a ? jj : jj - sg;
                     kn = a ? kk - sg : kk;
-                    q = 2 * c < SE_Q ? F + 6 * (a ? 2 : 1) + 2 * c : RC_Q + 2 * c - SE_Q;
+                    q = edge_item(FWD, a ? 2 : 1, 2 * c);
                     early = 1;
                 }
                 // cells are numbered 0..I in sweep order, the zero records at
@@ -1331,31 +1155,11 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
         // Places of the stage items: this pencil's, and its j and k
         // neighbours' (a pencil of the tile, or an edge neighbour), each in a
         // slab; of the upstream dq in the hand-over object
-        struct JacAt { const double *v1, *a, *lb, *v2, *p; };
-        auto jac_at = [&](int pencil, bool e, int f) {
-            const int q = e ? SE_Q - SP_Q : 0;
-            const double *st = stage + pencil;
-            return JacAt{st + rows.v1 + (rows.face ? f : q), st + rows.a + (rows.aface ? f : q), st + rows.lb + (rows.face ? f : q),
-                         st + rows.v2 + q, st + rows.p + q};
-        };
-        auto jac = [&](const JacAt &w, int slab) {
-            return RowJac{w.v1[slab], w.a[slab], w.a[slab + 1], w.a[slab + 2], w.lb[slab], w.v2[slab], w.p[slab]};
-        };
         const int mp = grp * SP_N;
-        const JacAt ai = jac_at(mp, false, 0), aj = jac_at(ej ? SLAB_E + gk * SE_N : (grp - sg) * SP_N, ej, ej ? 0 : 6),
-                    ak = jac_at(ek ? SLAB_E + (TK + gj) * SE_N : (grp - sg * TJ) * SP_N, ek, ek ? 0 : 12);
-        auto cell = [&](int slab) {
-            const double *st = stage + mp;
-            RowCell c;
-            c.j = jac(ai, slab);
-            c.res = st[slab + SP_RES + ln];
-#pragma unroll
-            for (int q = 0; q < 7; q++) c.g[q] = st[slab + rows.g[q]];
-            c.a = st[slab + SP_GX + GX_A];
-#pragma unroll
-            for (int q = 0; q < 3; q++) c.co[q] = st[slab + rows.co[q]];
-            return c;
-        };
+        const JacAt ai = jac_at(rows, stage + mp, false, 0),
+                    aj = jac_at(rows, stage + (ej ? SLAB_E + gk * SE_N : (grp - sg) * SP_N), ej, 1),
+                    ak = jac_at(rows, stage + (ek ? SLAB_E + (TK + gj) * SE_N : (grp - sg * TJ) * SP_N), ek, 2);
+        auto cell = [&](int slab) { return row_cell(rows, ai, stage + mp, slab, ln); };
         // (indices into the hand-over object, not pointers chosen among
         // several, so the compiler sees these reads cannot touch the stage)
         const int oi = grp * NPV + ln, oj = (lj ? (grp - sg) * NPV : nj ? HX + gk * NPV : HZ) + ln,
@@ -1370,8 +1174,8 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < 8; q++) ci[q] = 0.0;
-        row_coef(rows, jac(aj, (SLABS - 1) * SLAB_N), cj);
-        row_coef(rows, jac(ak, (SLABS - 1) * SLAB_N), ck);
+        row_coef<Dpp>(rows, row_jac(aj, (SLABS - 1) * SLAB_N), cj);
+        row_coef<Dpp>(rows, row_jac(ak, (SLABS - 1) * SLAB_N), ck);
         own = cell(0);
         __syncthreads();
         int i = i0, left = (sb - sa) * sg;                           // this step's cell, the steps after it
@@ -1384,11 +1188,11 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             const double xi = hand[oi + before * HN], xj = hand[oj + before * HN], xk = hand[ok + before * HN];
             // dcv = res + the three upstream products, in the reference's i, j, k order
             double y = own.res;
-            row_apply(ci, xi, y);
-            row_apply(cj, xj, y);
-            row_apply(ck, xk, y);
+            row_apply<Dpp>(ci, xi, y);
+            row_apply<Dpp>(cj, xj, y);
+            row_apply<Dpp>(ck, xk, y);
             // dq = D^-1 dcv
-            const double xn = row_dinv(rows, own, y);
+            const double xn = row_dinv<Dpp>(rows, own, y);
             if (lane < NPV) {
                 hand[oi + c * HN] = act ? xn : 0.0;
                 // the dq that other tiles wait for goes out at once.  Forward,
@@ -1406,10 +1210,10 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             // coefficients of the next step (independent of dq): this cell's
             // row through its face to the next cell, and the j / k neighbours
             // of the next cell; and the next cell's own terms
-            const RowJac nbj = jac(aj, c * SLAB_N), nbk = jac(ak, c * SLAB_N);
-            row_coef(rows, own.j, ci);
-            row_coef(rows, nbj, cj);
-            row_coef(rows, nbk, ck);
+            const RowJac nbj = row_jac(aj, c * SLAB_N), nbk = row_jac(ak, c * SLAB_N);
+            row_coef<Dpp>(rows, own.j, ci);
+            row_coef<Dpp>(rows, nbj, cj);
+            row_coef<Dpp>(rows, nbk, ck);
             own = cell(after * SLAB_N);
             // formed before the barrier (while the poll wavefront may still be
             // waiting), not after it on the next step's path

@@ -1161,8 +1161,9 @@ HD void jac_row(int npv, const JacNb &q, int sign, int n, const double *x, doubl
     }
 }
 
-// Row n of the same product as coefficients, formed without branching on n
-// (the rows of a cell sit on neighbouring lanes): y = y + c[l] x[l] over
+// Row n of the same product as coefficients, formed by one lane alone without
+// branching on n (the host tests hold it and the sweeps' row_coef, which
+// shares the work among a pencil's lanes, against jac_row): y = y + c[l] x[l] over
 // l = 0..6 in order, then y = y + c[7] x[n], repeats jac_row's roundings.
 // Every a(n,l) is built from jac_row's products in jac_row's order; the
 // terms a row does not have enter as exact zeros (P r1 + 0 hy, a + 0), the
@@ -1342,7 +1343,8 @@ HD double bsel(bool c, double a, double b)
 
 // getx_apply for any row without branching on n: every row's value is
 // formed with getx_apply's operations in getx_apply's order, then row n's is
-// selected (the rows of a cell sit on neighbouring lanes).
+// selected (by one lane alone; the sweeps' row_dinv shares the work, and the
+// host tests hold both against getx_apply).
 template <class F>
 HD double getx_apply_sel(F G, const double *pv, double d_ry1, double d_rt, const double *res, int n, double resn, double pvn)
 {
