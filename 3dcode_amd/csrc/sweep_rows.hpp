@@ -136,7 +136,12 @@ HD RowJac row_jac(const JacAt &w, int slab)
 // row): r1[l] and the energy row's factor of column l sit in lane l.  The
 // factor 0.5 and the sign are in u, lam, vis and n3 already, which they pass
 // through exactly.  A term that only some rows have is added as
-// fma(term, 1 or 0, sum), which rounds as the sum.
+// fma(term, 1 or 0, sum), which rounds as the sum where the term is finite.
+// A term that is not makes NaN of the rows that do not have it; those are
+// not finite without it either (u, lam or vis are in every row's columns), so
+// a run that overflows loses the same rows and only shows NaN where
+// jac_row_coef shows infinity.  (Selecting the term takes three instructions
+// for each fma.)
 template <class X> HD void row_coef(const RowMap &m, const RowJac &j, double *c)
 {
     const double t0 = j.a * j.v1, t = t0 + j.b * j.lb + j.c * j.v1, r = m.m13 ? t0 : t;

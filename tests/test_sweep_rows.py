@@ -67,3 +67,24 @@ def test_rows_of_lanes_bit_exact(L, pkg, npv, fwd, edge):
         assert np.array_equal(yr[:npv], yp[:npv])
         assert np.array_equal(xr[:npv], xp[:npv])
         assert np.abs(xr[:npv]).max() > 0.0
+
+
+@pytest.mark.parametrize("npv", [7, 9])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 1e200])
+def test_a_non_finite_operand_reaches_the_same_rows(L, pkg, npv, value):
+    """A number of a cell or its neighbours that is not finite (or whose
+    products overflow) leaves the rows finite that it leaves finite in the
+    form without lanes; which of infinity and NaN the others hold may differ
+    only where the energy row, and so the cell's temperature, is one of them."""
+    case, iv, dv = problem(pkg, npv)
+    for fwd in (0, 1):
+        for item in range(42):
+            for cell in range(4):
+                rng = np.random.default_rng([npv, fwd, item, cell])
+                c = cells(pkg, rng, npv, case.params["pref"])
+                c[cell, item] = value
+                yr, xr, _, _, ys, xs = step(L, iv, dv, fwd, cell & 1, c, rng)
+                assert np.array_equal(np.isfinite(yr[:npv]), np.isfinite(ys[:npv])), (item, cell)
+                assert np.array_equal(np.isfinite(xr[:npv]), np.isfinite(xs[:npv])), (item, cell)
+                if not np.array_equal(np.isnan(xr[:npv]), np.isnan(xs[:npv])):
+                    assert not np.isfinite(xr[4]), (item, cell)      # the cell's temperature is lost in either
