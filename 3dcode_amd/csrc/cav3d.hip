@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <array>
+#include <climits>
 #include <cstdio>
 #include <cstring>
 #include <string>
@@ -70,11 +71,11 @@ struct DS {           // device state, passed by value
     long NG, NC, NW, NF[3], NCX, NEX, NTX, NBC[3], NHALO;
     double *pv, *dc, *mut, *vol, *ydn, *cx, *ex, *tx;
     double *res, *dt, *icav, *itt, *ocut, *rcav, *qq;
-    double *img;      // the sweeps' cell records [NW][RC_N]
+    double *img;      // the sweeps' cell records, in pencils with a record of zeros before and after each [NF[0] + 1][RC_N]
     double *xqf, *xqb; // dq of the sweeps [NW][NPV], a cell's values adjacent: forward
                        // the cross-tile values only, backward every cell's
     long NPLANE;      // sum over blocks of (J-1)(K-1)
-    double *ff[3];    // face fluxes [2*npv][NF]
+    double *ff[3];    // face fluxes [2*npv][NF] (in img's memory)
     double *red;      // norm partials
     double *scal;     // [0] dt min bits, [1] accumulated time, [2..] norms
     Seg *seg[3];
@@ -825,11 +826,27 @@ __global__ __launch_bounds__(BLK_WG) void k_combine(DS S)
 // the cells' records.  Bound by HBM (736 bytes a cell written, some 450
 // read), so a wavefront turns its 64 records around in LDS, 24 numbers a cell
 // at a time, and twelve adjacent lanes write 192 bytes of one record.
-__global__ __launch_bounds__(128) void k_lhs_prep(DS S)
+// The workgroups from wz on write the records of zeros between the pencils,
+// which the face fluxes have been written over.
+constexpr int ZERO_ROWS = 64;       // pencils of such a workgroup
+__global__ __launch_bounds__(128) void k_lhs_prep(DS S, unsigned wz)
 {
     constexpr int CH = 24;
     __shared__ double turn[2][64][CH + 1];
     __shared__ double *to[2][64];
+    if (blockIdx.x >= wz) {
+        const long r0 = (long)(blockIdx.x - wz) * ZERO_ROWS;
+        for (int q = threadIdx.x; q < ZERO_ROWS * (RC_N / 2); q += 128) {
+            const long r = r0 + q / (RC_N / 2);
+            if (r > S.NPLANE) return;
+            int b = 0;
+            for (int m = 1; m < S.nb; m++) if (r >= S.b[m].p0) b = m;
+            const BlkD &B = S.b[b];
+            const long slot = B.f0[0] + (r - B.p0) * B.I;      // (the last pencil's end is the slot behind it)
+            *(double2 *)(S.img + slot * RC_N + 2 * (q % (RC_N / 2))) = make_double2(0.0, 0.0);
+        }
+        return;
+    }
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const bool on = t < S.NC;
@@ -838,7 +855,7 @@ __global__ __launch_bounds__(128) void k_lhs_prep(DS S)
     const Par &P = S.P;
     int i, j, k;
     cell_of(B, tc - B.c0, i, j, k);
-    to[wv][lane] = on ? S.img + widx(B, i, j, k) * RC_N : nullptr;
+    to[wv][lane] = on ? S.img + fidx(B, 0, i, j, k) * RC_N : nullptr;
     CellJ cc;
     load_cell(S, B, i, j, k, cc);
     double f6[6][3];
@@ -1004,8 +1021,8 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
             // issued, the last SLABS - 3 may still be on their way.
             // Lane and transfer (16 bytes) to piece of a record: the 37 pieces
             // of a pencil, F then Q, GX and RES; the 12 of an edge neighbour.
-            // A pencil outside the block, and a cell before or past a
-            // pencil's ends, is a record of the zero outer layer.
+            // Before and past a pencil's ends, and everywhere in a pencil
+            // outside the block, it is a record of zeros.
             int l = threadIdx.x - 320;
             asm volatile("" : "+v"(l));          // (worked out per tile: kept across tiles, its pieces end up in scratch memory)
             const double *src[SLAB_LOADS];       // the piece of the coming slab
@@ -1033,8 +1050,10 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
                 // cells are numbered 0..I in sweep order, the zero records at
                 // the pencil's ends included; slab -1 holds cell at - 1 of it
                 at[t] = FWD ? sa - sg - jj - kk - 1 + early : B.I + 1 - (sa - sg - jj - kk) + early;
-                const int c0 = min(max(at[t], 0), B.I);
-                src[t] = S.img + widx(B, FWD ? 1 + c0 : B.I + 1 - c0, min(jn, B.J + 1), min(kn, B.K + 1)) * RC_N + q;
+                const bool in = ((unsigned)(jn - 2) < (unsigned)(B.J - 1)) & ((unsigned)(kn - 2) < (unsigned)(B.K - 1));
+                at[t] = in ? at[t] : INT_MIN / 2;        // (stays at the end of the block's first pencil)
+                const int c0 = min(max(at[t], 0), B.I), row = in ? jn - 2 + (B.J - 1) * (kn - 2) : 0;
+                src[t] = S.img + (B.f0[0] + (long)B.I * row + (FWD ? c0 : B.I - c0)) * RC_N + q;
             }
             const unsigned BI = B.I;
             auto issue = [&](int slot) {
@@ -1167,7 +1186,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_sweep_tile(DS S, const int *t
         // where this pencil's results go, from the cell of the first hyperplane on
         const int i0 = sa - j - k;
         double *xe = xq + (widx(B, i0, min(j, B.J), min(k, B.K)) * NPV + lane);
-        double *yo = S.img + (widx(B, i0, min(j, B.J), min(k, B.K)) * RC_N + RC_RES + lane);
+        double *yo = S.img + (fidx(B, 0, i0, min(j, B.J), min(k, B.K)) * RC_N + RC_RES + lane);
         if (lane < NPV) hand[(SLABS - 1) * HN + oi] = 0.0;           // the first step's upstream reads zeros
         double ci[8], cj[8], ck[8];                                  // coefficients of the coming step
         RowCell own;                                                 // its cell
@@ -1788,7 +1807,8 @@ int launch_begin(cav3d_ctx *c)
 int launch_sweeps(cav3d_ctx *c)
 {
     DS &S = c->S;
-    hipLaunchKernelGGL(k_lhs_prep, dim3(nblk(S.NC, 128)), dim3(128), 0, c->st, S);
+    const unsigned wz = nblk(S.NC, 128);
+    hipLaunchKernelGGL(k_lhs_prep, dim3(wz + nblk(S.NPLANE + 1, ZERO_ROWS)), dim3(128), 0, c->st, S, wz);
     const dim3 grid(c->sweep_blocks), block(SWEEP_THREADS);
     if (c->profile) hipEventRecord(c->ev[6], c->st);
     hipLaunchKernelGGL(k_sweep_tile<true>, grid, block, 0, c->st, S, (const int *)c->tiles, c->ntiles, c->sweep_err, c->ticket);
@@ -1960,14 +1980,19 @@ int cav3d_create(const cav3d_params *prm, int nblocks, const cav3d_block *blocks
     if ((rc = dalloc(c, &S.pv, npv * S.NG)) || (rc = dalloc(c, &S.dc, (long)ND * S.NG)) ||
         (rc = dalloc(c, &S.vol, S.NW)) || (rc = dalloc(c, &c->xc, 3 * S.NW)) || (rc = dalloc(c, &S.cx, 3 * S.NCX)) || (rc = dalloc(c, &S.ex, 3 * S.NEX)) ||
         (rc = dalloc(c, &S.tx, 3 * S.NTX)) || (rc = dalloc(c, &S.res, npv * S.NC)) || (rc = dalloc(c, &S.dt, S.NC)) ||
-        (rc = dalloc(c, &S.img, (long)RC_N * S.NW)) ||
+        (rc = dalloc(c, &S.img, RC_N * (S.NF[0] + 1))) ||
         (rc = dalloc(c, &S.xqf, (long)NPV * S.NW)) || (rc = dalloc(c, &S.xqb, (long)NPV * S.NW)) ||
         (rc = dalloc(c, &S.scal, 32))) { cav3d_destroy(c); return rc; }
     if (hipMemcpyAsync(S.scal, &DT_NONE, sizeof(DT_NONE), hipMemcpyHostToDevice, c->st) != hipSuccess) {
         cav3d_destroy(c); return fail("device set-up failed", -3);
     }
-    for (int d = 0; d < 3; d++)
-        if ((rc = dalloc(c, &S.ff[d], 2 * npv * S.NF[d]))) { cav3d_destroy(c); return rc; }
+    // the face fluxes live from the faces to the combine, the records from
+    // k_lhs_prep behind it to the backward sweep: they share their memory (18
+    // numbers a face, of which there are at most 4 to a cell where a block
+    // has 3 cells a direction, against RC_N a cell)
+    static_assert(2 * NPV * 4 <= RC_N, "the fluxes fit the records' memory");
+    S.ff[0] = S.img;
+    for (int d = 1; d < 3; d++) S.ff[d] = S.ff[d - 1] + 2 * npv * S.NF[d - 1];
     if (prm->iturb == 0) {
         if ((rc = dalloc(c, &S.mut, S.NG)) || (rc = dalloc(c, &S.ydn, S.NW)) || (rc = dalloc(c, &S.itt, 4 * S.NC)) ||
             (rc = dalloc(c, &S.ocut, S.NC))) { cav3d_destroy(c); return rc; }

@@ -8,9 +8,9 @@
 namespace cav {
 
 // What a sweep step reads of a cell lies side by side in memory, in a record
-// of 92 doubles (736 bytes, 46 pieces of 16), ranges and order of the dcv
-// array of the reference (1:I+1 and so on; the outer layer stays zero and is
-// what a pencil's absent neighbours read):
+// of 92 doubles (736 bytes, 46 pieces of 16).  A pencil's records follow one
+// another, with a record of zeros before and after each pencil (one between
+// two) for the neighbours that it does not have:
 //   RC_FP, RC_FM  the +i,+j,+k (-i,-j,-k) faces x (+-n3[3], +-u, lam, vis) / 2:
 //                 the forward (backward) sweep's split Jacobians with their
 //                 sign and factor (exact: a power of two)
