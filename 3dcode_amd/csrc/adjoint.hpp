@@ -27,8 +27,9 @@
 // d/d(p_ref) is the sum of pv_bar over the pressure component: the residual
 // reads gauge pressure only as p + p_ref or in differences (the pressure
 // floor included), so shifting p_ref shifts it as shifting every gauge
-// pressure does.  d/d(u_ref) is carried on one extra lane of the flux-core
-// passes (the low-Mach preconditioning is the only reader).
+// pressure does.  d/d(u_ref) comes out of the flux cores' reverse passes (the
+// low-Mach preconditioning is its only reader there) and of the mass-transfer
+// sources'.
 //
 // Included once, from cav3d.hip, after the context definition.
 
@@ -260,14 +261,6 @@ __global__ __launch_bounds__(128) void k_faces_vjp(DS S, AD A, FluxWgs g)
 // with the limiter's bars in registers, 1.58 with a tile a direction.
 constexpr int ADJ_TILE[2][3][3] = {{{32, 8, 8}, {16, 16, 8}, {16, 8, 16}}, {{16, 8, 8}, {16, 8, 8}, {16, 8, 8}}};
 constexpr int ADJ_CELLS[2] = {2048, 1024};
-// Element q of the array at base, the same for every lane: the base stays in
-// scalar registers and a lane holds one 32-bit offset for all the stencil's
-// points.  (A field of one block is below 4 GB: 2^29 cells of a context's
-// arrays would take more than the device's memory.)
-template <class T> __device__ __forceinline__ T lane_at(const T *base, unsigned q)
-{
-    return *(const T *)((const char *)base + (size_t)(q * (unsigned)sizeof(T)));
-}
 template <int D, int NM, bool SMALL>
 __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, int item, double *acc)
 {
@@ -310,8 +303,8 @@ __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, int it
         const int f[3] = {lo[0] + q - q1 * cnt[0], lo[1] + q1 - q2 * cnt[1], lo[2] + q2};
         // the face's place in its block (fidx)
         const unsigned t = (unsigned)(f[0] - (D == 0 ? 1 : 2) + fn[0] * (f[1] - (D == 1 ? 1 : 2) + fn[1] * (f[2] - (D == 2 ? 1 : 2))));
-        double wl = lane_at(A.w[D] + (long)n * NF + B.f0[D], t), wr = lane_at(A.w[D] + (long)(npv + n) * NF + B.f0[D], t);
-        const int cell = lane_at(A.cell[D] + B.f0[D], t);
+        double wl = at32(A.w[D] + (long)n * NF + B.f0[D], t), wr = at32(A.w[D] + (long)(npv + n) * NF + B.f0[D], t);
+        const int cell = at32(A.cell[D] + B.f0[D], t);
         // the face's left cell in tile coordinates; which offsets along each axis land in the tile
         const int l[3] = {f[0] - c0[0], f[1] - c0[1], f[2] - c0[2]};
         const int w3[3] = {c1[0] - c0[0], c1[1] - c0[1], c1[2] - c0[2]};
@@ -342,10 +335,10 @@ __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, int it
         // whether or not the reconstruction's bars are zero): one memory latency a round
         double v0 = 0.0, v1 = 0.0, v2 = 0.0, vc = 0.0;
         if (vq >= 0) {
-            v0 = lane_at(A.vb[D] + (long)(3 * vq) * NF + B.f0[D], t);
-            v1 = 0.0625 * lane_at(A.vb[D] + (long)(3 * vq + 1) * NF + B.f0[D], t);
-            v2 = 0.0625 * lane_at(A.vb[D] + (long)(3 * vq + 2) * NF + B.f0[D], t);
-            if (cq >= 0) vc = 0.5 * lane_at(A.vb[D] + (long)(3 * nv + cq) * NF + B.f0[D], t);
+            v0 = at32(A.vb[D] + (long)(3 * vq) * NF + B.f0[D], t);
+            v1 = 0.0625 * at32(A.vb[D] + (long)(3 * vq + 1) * NF + B.f0[D], t);
+            v2 = 0.0625 * at32(A.vb[D] + (long)(3 * vq + 2) * NF + B.f0[D], t);
+            if (cq >= 0) vc = 0.5 * at32(A.vb[D] + (long)(3 * nv + cq) * NF + B.f0[D], t);
         }
         if constexpr (NM > 0) {
             const double *f0 = S.pv + (long)n * S.NG + B.g0;
@@ -353,7 +346,7 @@ __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, int it
             double x[NSLOT];
 #pragma unroll
             for (int ll = 1; ll <= NSLOT; ll++)
-                if (NM == 2 || ll == 9 || ll == 10 || ll == 23 || ll == 32 || ll >= 37) x[ll - 1] = lane_at(f0 + stencil_off<D>(B, ll), gl);
+                if (NM == 2 || ll == 9 || ll == 10 || ll == 23 || ll == 32 || ll >= 37) x[ll - 1] = at32(f0 + stencil_off<D>(B, ll), gl);
             if (on && (wl != 0.0 || wr != 0.0)) o = muscl_back<NM == 2>(S.P.nlim, [&](int ll) -> double { return x[ll - 1]; }, wl, wr);
         }
         b9 += o.x9;
@@ -364,7 +357,7 @@ __device__ __forceinline__ void adj_stencil_dir(const DS &S, const AD &A, int it
         auto ex = [&](int ll) -> double { return exl(ll) + exr(ll); };
         if (vq >= 0 || sen) {
             // the 18 points of the viscous differences (and of the pressure sensor)
-            auto sn = [&](int ll) -> double { return (sen ? lane_at(sen + (long)(ll - 1) * NF + B.f0[D], t) : 0.0) + ex(ll); };
+            auto sn = [&](int ll) -> double { return (sen ? at32(sen + (long)(ll - 1) * NF + B.f0[D], t) : 0.0) + ex(ll); };
             add(1, -v1 - v2 + sn(1));
             add(2, -v1 - v2 + sn(2));
             add(3, o.x3 - 2.0 * v2 + sn(3));
@@ -616,8 +609,8 @@ __global__ __launch_bounds__(256) void k_dotdiff_fixed(const double *w, const do
 // The stencil pass takes the small tiles below this many large ones (times the
 // variables): two rounds of the wavefronts that fit the chip (two a SIMD).
 // 64x32x32 cells, 7 variables, TVD: 1575 large tiles take 161 us, the small
-// ones 114; 53x41x27, 9 variables, MLP: 1296, 399 and 358; 128x64x64, 9
-// variables, MLP: 10935, 1577 and 1719.
+// ones 113; 53x41x27, 9 variables, MLP: 1728, 396 and 358; 128x64x64, 9
+// variables, MLP: 10935, 1577 and 1712.
 constexpr long ADJ_FEW = 4096;
 
 int adj_alloc(cav3d_ctx *c)

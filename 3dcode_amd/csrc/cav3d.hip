@@ -50,7 +50,7 @@ int fail(const std::string &m, int code = -1) { g_err = m; return code; }
 
 struct BlkD {
     int I, J, K, nx, ny;
-    long g0, c0, w0, f0[3], cx0, ex0, tx0, p0;   // p0: first (j,k) slot of the block's sweep plane
+    long g0, c0, w0, f0[3], cx0, ex0, tx0, p0;   // p0: the block's first pencil
     long ng, nc, nw, nf[3], ncx, nex, ntx;
 };
 
@@ -74,7 +74,7 @@ struct DS {           // device state, passed by value
     double *img;      // the sweeps' cell records, in pencils with a record of zeros before and after each [NF[0] + 1][RC_N]
     double *xqf, *xqb; // dq of the sweeps [NW][NPV], a cell's values adjacent: forward
                        // the cross-tile values only, backward every cell's
-    long NPLANE;      // sum over blocks of (J-1)(K-1)
+    long NPLANE;      // pencils: sum over blocks of (J-1)(K-1)
     double *ff[3];    // face fluxes [2*npv][NF] (in img's memory)
     double *red;      // norm partials
     double *scal;     // [0] dt min bits, [1] accumulated time, [2..] norms
@@ -179,7 +179,7 @@ template <class T> __device__ __forceinline__ const T &at32(const T *base, unsig
 {
     return *(const T *)((const char *)base + (size_t)(q * (unsigned)sizeof(T)));
 }
-// 32-bit places within block B's arrays: ghosted, dcv ranges, face vectors of axis AX
+// 32-bit places within block B's arrays: ghosted, cells with one layer around, face vectors of axis AX
 __device__ __forceinline__ unsigned gidx32(const BlkD &B, int i, int j, int k)
 {
     return (unsigned)(i + 1) + (unsigned)B.nx * ((unsigned)(j + 1) + (unsigned)B.ny * (unsigned)(k + 1));
@@ -702,7 +702,7 @@ __device__ __forceinline__ void visc_face(const DS &S, unsigned wg)
 // faces in FP32 where R is not (AUSMPW+ in the mixed mode).  Six launches on three streams did the same, but an event
 // between streams costs some 10 us, and an iteration had three forks and
 // joins: it took 210 us at 16x8x8 cells and 162 in single launches on one
-// stream, 64x32x32 448 and 404, 128x64x64 1695 and 1671; from a million cells
+// stream, 64x32x32 448 and 409, 128x64x64 1695 and 1671; from a million cells
 // on the two were equal (the viscous faces run at two wavefronts per SIMD
 // here, three in a launch of their own).
 struct FluxWgs { unsigned n[3]; };       // workgroups of each direction
@@ -909,7 +909,7 @@ __device__ __forceinline__ void st_dev(double *p, double v)
 // Tiled sweep: a workgroup owns a tile of TJ x TK pencils of one block and
 // walks its hyperplanes s = i + j + k in sweep order with one barrier per
 // hyperplane.  A pencil's neighbour inside the tile hands over its dq through
-// LDS (double-buffered by the parity of s); a neighbour in another tile
+// LDS (by the place of s in the ring); a neighbour in another tile
 // through a device-coherent exchange array that holds a cell's values side by
 // side (one write of 72 bytes, not nine 8-byte writes to nine lines), waited
 // for with a bounded poll.
@@ -1263,7 +1263,14 @@ __device__ __forceinline__ void sweep_reset(const DS &S, long n, int *ticket, un
 __global__ __launch_bounds__(256) void k_sweep_reset(DS S, long n, int *ticket) { sweep_reset(S, n, ticket, blockIdx.x); }
 
 // The start of an iteration in one launch: the face boundaries, the time step
-// and the sweeps' resets, none of which reads what another writes.
+// and the sweeps' resets, none of which reads what another writes.  All its
+// workgroups take the boundary part's registers (one wavefront a SIMD; the
+// time step alone runs at five, the resets at eight), so it gains where
+// launches count and loses where the cells do: with the three in launches of
+// their own, 16x8x8 cells take 2.7 + 5.4 + 8.7 us and two launches more, here
+// 13.8; 128x64x64 14 + 34 + 11, here 75; 192x96x64 28 + 69 + 11, here 164.  The
+// launches ran beside each other on three streams before, whose joins cost
+// what this loses: an iteration of 192x96x64 cells took 3498 us so, 3499 here.
 __global__ __launch_bounds__(256) void k_begin(DS S, unsigned nbc, unsigned nts, long nq, int *ticket)
 {
     unsigned w = blockIdx.x;

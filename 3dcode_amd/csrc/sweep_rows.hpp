@@ -62,7 +62,7 @@ HD int edge_item(bool fwd, int ax, int q) { return q + (q < SE_Q ? (fwd ? RC_FP 
 // items, RowMap) and pass them around with DPP row broadcasts.  Reading every
 // item into every lane took 140 LDS reads a step, whose return path (each
 // read brings 64 lanes x 8 bytes at 128 bytes a clock for the four pencil
-// wavefronts of the CU) bound the step.  Now it is 39, and the terms that are
+// wavefronts of the CU) bound the step.  Now it is 36, and the terms that are
 // one expression per column are formed once, a column per lane, not in every
 // lane.  What a lane needs another operand for than its neighbours it reads
 // from another place rather than selecting among broadcasts.
